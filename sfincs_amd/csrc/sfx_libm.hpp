@@ -109,45 +109,38 @@ SFX_HD inline double pow_estimate(float x, int which) {
   return (double)x * (double)x * y * corr;
 }
 
-// The device's estimate of the same powers: the cube root's polynomial and Newton steps as
-// fused multiply-adds, and ln x for the float exponents' offsets from the hardware log2 of
-// the mantissa (v_log_f32, absolute error near 2^-23 on [1, 2), which the offsets of at most
-// 8e-8 turn into 2^-47 relative), about half the double operations of pow_estimate. Its
-// rounding decisions need it within 2^-40 of the exact power: a device test checks it
-// against pow_estimate (itself verified within 2^-44 of pow for every table input) for
-// every float of [2^-40, 2^14) and each exponent.
+// The device's estimate of the same powers. The hardware's f32 log2 and exp2 give
+// z0 = x^(-1/3) to about 2^-19.7 (the log2 of x, at most 128 in magnitude, is rounded to f32), and
+// one third-order step z = z0 (1 + r/3 + 2 r^2/9), r = 1 - x z0^3, leaves 14 r^3/81 < 2^-56: z0^2
+// is exact in f64, so the cube root takes six f64 operations and no range reduction. The float
+// exponents' offsets from 1/3, 5/3 and 7/3 (at most 8e-8) multiply by 1 + t + t^2/2, t = d ln x,
+// from the same log2: in f32 for 1/3 (t < 2.8e-7 over the table range, so 2^-45 of the result), in
+// f64 for the others. The rounding decisions need it within 2^-40 of the exact power: a device
+// test checks it against pow_estimate (itself verified within 2^-44 of pow for every table input)
+// for every float of [2^-40, 2^14) and each exponent. The power is the largest single piece of a
+// wet point's arithmetic (67 of about 450 vector instructions with the polynomial and two Newton
+// steps of pow_estimate, 33 here).
 __device__ inline double pow_estimate_dev(float x, int which) {
   if (which == 3) return (double)x * sqrt((double)x);
-  const uint32_t b = f2u(x);
-  if (b < 0x00800000u) return pow_estimate(x, which);
-  const int e = (int)(b >> 23) - 127;
-  const float mf = u2f((b & 0x7fffffu) | 0x3f800000u);
-  const double m = (double)mf;
-  const int q = e >= 0 ? e / 3 : -((2 - e) / 3);
-  const int r = e - 3 * q;
-  const double a = m * (double)(1 << r);
-  const double cr = r == 0 ? 1.0 : (r == 1 ? 0.79370052598409979 : 0.62996052494743658);
-  double z = fma(fma(fma(fma(0.0285876759712902, m, -0.22121268212268402), m, 0.6954153443691581), m,
-                     -1.1728037038550854), m, 1.6699753569259383);
-  z = z * cr;
-  const double third = 1.0 / 3.0;
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const double w = a * z * z;
-    z = fma(z * third, fma(-w, z, 1.0), z);
+  if (f2u(x) < 0x00800000u) return pow_estimate(x, which);
+  const float xf = x < 3.4028234663852886e38f ? x : 3.4028234663852886e38f;
+  const float L = (float)__builtin_amdgcn_frexp_expf(xf) + __builtin_amdgcn_logf(__builtin_amdgcn_frexp_mantf(xf));
+  const double xd = (double)xf, z0 = (double)__builtin_amdgcn_exp2f(L * (-1.0f / 3.0f));
+  const double r = fma(-(xd * (z0 * z0)), z0, 1.0);
+  const double z = fma(z0 * r, fma(r, 2.0 / 9.0, 1.0 / 3.0), z0);
+  const double y = xd * z * z;
+  if (which == 0) {
+    const float t = L * (float)(((double)(1.0f / 3.0f) - 1.0 / 3.0) * 0.69314718055994530942);
+    return fma(y, (double)__builtin_fmaf(0.5f * t, t, t), y);
   }
-  union { uint64_t u; double d; } p2;
-  p2.u = (uint64_t)(q + 1023) << 52;
-  const double y = a * z * z * p2.d;
-  const double lnx = ((double)e + (double)__builtin_amdgcn_logf(mf)) * 0.69314718055994530942;
-  const double d13 = (double)(1.0f / 3.0f) - 1.0 / 3.0;
+  const double lnx = ((double)__builtin_amdgcn_frexp_expf(xf) + (double)__builtin_amdgcn_logf(__builtin_amdgcn_frexp_mantf(xf))) *
+                     0.69314718055994530942;
   const double d53 = (double)(5.0f / 3.0f) - 5.0 / 3.0;
   const double d73 = (double)(7.0f / 3.0f) - 7.0 / 3.0;
-  const double t = (which == 0 ? d13 : (which == 1 ? d53 : d73)) * lnx;
+  const double t = (which == 1 ? d53 : d73) * lnx;
   const double corr = fma(t, fma(0.5, t, 1.0), 1.0);
-  if (which == 0) return y * corr;
-  if (which == 1) return (double)x * y * y * corr;
-  return (double)x * (double)x * y * corr;
+  if (which == 1) return xd * y * y * corr;
+  return xd * xd * y * corr;
 }
 
 // True when the double value r lies within 2^-32 (relative) of a midpoint between two
@@ -184,6 +177,7 @@ SFX_HD inline bool near_midpoint_fp(double r) {
 template <typename P>
 SFX_HD inline float pow_lookup(P t, uint32_t key, float fallback, uint32_t mask = POW_HASH_SIZE - 1) {
   uint32_t h = hash_bits(key) & mask;
+#pragma unroll 1   // almost every lookup ends at its first slot (load factor 0.28)
   for (int probe = 0; probe < 64; ++probe) {
     const uint64_t e = t[h];
     const uint32_t k = (uint32_t)e;

@@ -62,7 +62,7 @@ def cont_bytes(reads_per_cell, n_cells, stores_per_step):
         sum(n * b for n, b in zip(stores_per_step[:5], CONT_WRITE))
 
 
-def byte_model(sizes, counts_per_step, stores_per_step, point_kernel):
+def byte_model(sizes, counts_per_step, stores_per_step, point_kernel, step_kernel=False):
     sg = bool(sizes["subgrid"])
     np_ = sizes["np"]
     c0, c1, c2, c3, c4, c5 = counts_per_step
@@ -73,6 +73,8 @@ def byte_model(sizes, counts_per_step, stores_per_step, point_kernel):
     mom = (np_ - c5 / 2) * MOM_CELL[sg] + copied * MOM_UV["copied"] + c1 * dry + c2 * MOM_UV["wet"][sg] + \
         c3 * MOM_UV["partial"] + c4 * MOM_UV["held"] + c5 * MOM_UV["tile_skipped"]
     cont = cont_bytes(CONT_READ[sg], np_, stores_per_step)
+    if step_kernel:   # one launch: the levels and faces that continuity needs are already there
+        cont -= (np_ - c5 / 2) * MOM_CELL[sg] + 8 * np_
     return mom, cont, dict(copied=copied, dry=c1, dry_zeros_held=c4, quiescent_tile=c5, wet=c2, partial=c3)
 
 
@@ -193,6 +195,7 @@ def whole_period(model, tuning, t_end, twin=True):
 # four face indices 16, iref 1, zs 8, zsmax 4, four faces 16; writes zs 8 and zsmax 4 when
 # they change (counted).
 IDX_MOM_CELL = 12
+STEP_KERNEL = -8      # tuning["momentum_kernel"] of the kernel that takes a whole step in one launch
 IDX_MOM_UV = {"copied": 17, "dry": 24, "held": 14, "wet": 69, "partial": 69}
 IDX_CONT_READ = 46
 
@@ -475,7 +478,8 @@ def main():
     batch = _lib.Batch()
     batch.add(inst, 1.0e9)
     batch.advance(8)
-    mom_b, cont_b, branches = byte_model(sizes, counts, stores, tuning["momentum_kernel"] < 0)
+    one = tuning["momentum_kernel"] == STEP_KERNEL
+    mom_b, cont_b, branches = byte_model(sizes, counts, stores, tuning["momentum_kernel"] < 0, one)
     print(f"# per launch ms forcing/momentum/continuity = {ms}; branches {branches}", file=sys.stderr, flush=True)
 
     # timed region: exactly K steps (graph-captured), barrier + synchronize on both sides
@@ -499,11 +503,12 @@ def main():
         del src, dst
 
     value = sizes["np"] * args.steps / secs
-    mom_gbs = mom_b / (ms[1] * 1e-3) / 1e9
-    cont_gbs = cont_b / (ms[2] * 1e-3) / 1e9
+    launch_b = mom_b + cont_b if one else mom_b       # of the dominant kernel: the whole step, or momentum
+    mom_gbs = launch_b / (ms[1] * 1e-3) / 1e9
+    cont_gbs = None if one else cont_b / (ms[2] * 1e-3) / 1e9
     step_gbs = (mom_b + cont_b) / (secs / args.steps) / 1e9
     mk = tuning["momentum_kernel"]
-    kernel = (f"k_mom_point<float, true, {-mk}>" if mk < 0 else
+    kernel = ("k_step<true>" if one else f"k_mom_point<float, true, {-mk}>" if mk < 0 else
               "k_mom_cell<float, true>" if mk == 0 else "k_mom_strip<float, true>")
     traffic = traffic_of(kernel)
     out = {
@@ -526,10 +531,10 @@ def main():
         "roofline": {"bound": "hbm", "achieved": mom_gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": mom_gbs / PEAK_HBM_GBS, "traffic": traffic,
                      "kernel": kernel,
-                     "bytes_per_launch": mom_b, "launch_ms": ms[1]},
-        "continuity": {"achieved_GBs": cont_gbs, "frac": cont_gbs / PEAK_HBM_GBS, "bytes_per_launch": cont_b,
-                       "launch_ms": ms[2]},
-        "forcing_launch_ms": ms[0],
+                     "bytes_per_launch": launch_b, "launch_ms": ms[1]},
+        "continuity": None if one else {"achieved_GBs": cont_gbs, "frac": cont_gbs / PEAK_HBM_GBS,
+                                        "bytes_per_launch": cont_b, "launch_ms": ms[2]},
+        "forcing_launch_ms": None if one else ms[0],
         "step_GBs": step_gbs,
         "branches_per_step": branches,
         "continuity_stores_per_step": dict(zip(("zs", "z_volume", "zs0", "zsderv", "zsmax", "steady_skipped"), stores)),

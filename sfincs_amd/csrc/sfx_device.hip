@@ -71,7 +71,18 @@ struct Scalars {
   float twindupd, meteo_t0, meteo_t1, mtw, momtw, msm;
   int32_t mwin, mspin;
   int32_t ahead;                 // the next step's fold, scalars and series are staged (StepImage)
-  int32_t pad_;
+  // step kernel (k_step): the side of the level arrays (zs, vol, zsderv, kfuv, uvmean) that holds
+  // the state, whether the last sweep's keys are still to be turned into min_dt, and their set
+  int32_t side, pend, kset;
+};
+
+// The step kernel's scalars and CFL keys. A launch reads s[f] and writes s[f ^ 1] (f alternates
+// from launch to launch), so that no block can see the scalars of the step it belongs to half
+// written; of the three key sets it reads one, raises the next and clears the third.
+constexpr int NKEY = 64, KEY_STRIDE = 32;
+struct ScalarBlock {
+  Scalars s[2];
+  alignas(128) uint32_t key[3][NKEY * KEY_STRIDE];
 };
 
 // Step scalars and forcing series of one scenario as a forcing block works on them: the
@@ -94,10 +105,21 @@ struct DevInst {
   int32_t tn_sh, mtn_sh;         // log2 of tn and mtn (tiles hold 256 cells, so both are powers of two)
   int32_t sk, nstrip;            // dense momentum kernel: strip march with sk rows per wave (sk > 0), per-cell (0), per-point with -sk points per thread (-1, -2, -4)
   int32_t mtn, mtm, mntn;        // dense momentum, per-cell kernel: tile shape and tiles along n
+  uint32_t mmagic;               // tile / mntn = tile * mmagic >> 32 (0: divide; see div_magic)
   int32_t xchunk, xchunk_c;      // momentum / continuity work-list runs per XCD (0: one contiguous band per XCD)
   int32_t count;                 // per-branch counting on
   int32_t nmt;                   // momentum tiles of the current tile shape
   int32_t mrow_sh;               // per-point kernel: log2 of the cell rows of a tile (mtm * P)
+  // step kernel (k_step): rows and number of its tiles, n-columns (nmax * row blocks), division by
+  // nmax; per tile: how often it did nothing in a row, the marks that wake it (two sets), what it
+  // holds (FT_*), its boundary flux points (index << 1 | owner) and balance faces, as CSR lists
+  int32_t frows, fnt, fcols;
+  uint32_t fmagic;
+  uint8_t* fquiet; uint8_t* fwake; const uint8_t* fflag;
+  const int32_t* fb_ptr; const int32_t* fb_ent; const int32_t* ff_ptr; const int32_t* ff_ent;
+  // its level arrays: [0] are zs, vol, zsderv, kfuv, uvmean below
+  double* zs_s[2]; double* vol_s[2]; float* zsd_s[2]; int8_t* kf_s[2]; float* um_s[2];
+  ScalarBlock* sb;
   // Quiescent per-point tiles: mq[tile] holds one byte per wave, 1 when all the wave's points
   // were dry with their zeros held at the tile's last run; md[tile] is raised when a cell
   // level the tile reads may have changed since (continuity, forcing; host writes reset
@@ -107,11 +129,12 @@ struct DevInst {
   Scalars* sc;
   StepImage* snext;              // the next step computed ahead (valid while sc->ahead)
   float* qtsrc_nx;               // its discharges
-  // CFL reduction: each wave of a momentum tile lowers blkmin[tile] to the minimum of its
-  // points' time steps (an atomic min on the tile's own word, so no two tiles share an
+  // CFL reduction: each wave of a momentum tile raises blkkey[tile] to the largest key
+  // (step_key) of its points (an atomic max on the tile's own word, so no two tiles share an
   // address and no wave waits for the others of its block); the fold at the start of the
-  // next step reduces the tiles and sets every word back to dtmax.
-  float* blkmin;
+  // next step reduces the tiles, turns the largest key into the time step (key_step) and
+  // sets every word back to 0.
+  uint32_t* blkkey;
   uint32_t* blkcnt;              // per tile, NCNT words: uv-points copied (kcuv not 1/6), dry, wet/full, partial, dry with zeros held, skipped
   uint32_t* cntstore;            // per continuity tile, NSTORE words: cells that stored zs, V, zs0, zsderv, zsmax; steady cells skipped
   // cells
@@ -274,46 +297,76 @@ size_t cont_tiles(const DevInst& I) {
   return I.dense ? cell_tiles(I, I.tn, I.tm) : (size_t)((I.np + BLOCK - 1) / BLOCK);
 }
 
-__device__ __forceinline__ float wave_min(float v) {
-  for (int o = WAVE / 2; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, WAVE));
-  return v;
-}
-
-// Minimum over the 64 lanes of a wave of positive floats, as their bit patterns (which
-// order like the values), valid in lane 63 only; all lanes must be active. DPP row shifts
-// reduce each row of 16 lanes into its last lane; row_bcast:15 then folds row 0 into
-// row 1 and row 2 into row 3, row_bcast:31 lane 31 into rows 2-3. Lanes without a source
-// keep their own value (bound_ctrl off, old = v), which the minimum ignores.
+// Maximum over the 64 lanes of a wave, valid in lane 63 only; all lanes must be active. DPP
+// row shifts reduce each row of 16 lanes into its last lane; row_bcast:15 then folds row 0
+// into row 1 and row 2 into row 3, row_bcast:31 lane 31 into rows 2-3. Lanes without a source
+// keep their own value (bound_ctrl off, old = v), which the maximum ignores.
 template <int CTRL, int ROWS>
-__device__ __forceinline__ uint32_t dpp_min(uint32_t v) {
+__device__ __forceinline__ uint32_t dpp_max(uint32_t v) {
   const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROWS, 0xf, false);
-  return o < v ? o : v;
+  return o > v ? o : v;
 }
-__device__ __forceinline__ uint32_t wave_min_last(uint32_t v) {
-  v = dpp_min<0x111, 0xf>(v);   // row_shr:1
-  v = dpp_min<0x112, 0xf>(v);   // row_shr:2
-  v = dpp_min<0x114, 0xf>(v);   // row_shr:4
-  v = dpp_min<0x118, 0xf>(v);   // row_shr:8
-  v = dpp_min<0x142, 0xa>(v);   // row_bcast:15
-  v = dpp_min<0x143, 0xc>(v);   // row_bcast:31
+__device__ __forceinline__ uint32_t wave_max_last(uint32_t v) {
+  v = dpp_max<0x111, 0xf>(v);   // row_shr:1
+  v = dpp_max<0x112, 0xf>(v);   // row_shr:2
+  v = dpp_max<0x114, 0xf>(v);   // row_shr:4
+  v = dpp_max<0x118, 0xf>(v);   // row_shr:8
+  v = dpp_max<0x142, 0xa>(v);   // row_bcast:15
+  v = dpp_max<0x143, 0xc>(v);   // row_bcast:31
   return v;
 }
 
-// Block-wide minimum over NT threads; the result is valid in every thread.
+// Block-wide maximum over NT threads; the result is valid in every thread.
 template <int NT = BLOCK>
-__device__ __forceinline__ float block_min(float v) {
-  __shared__ float red[NT / WAVE];
-  v = wave_min(v);
+__device__ __forceinline__ uint32_t block_max(uint32_t v) {
+  __shared__ uint32_t red[NT / WAVE];
+  v = wave_max_last(v);
   const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
-  if (lane == 0) red[w] = v;
+  if (lane == WAVE - 1) red[w] = v;
   __syncthreads();
-  float m = red[0];
-  for (int i = 1; i < NT / WAVE; ++i) m = fminf(m, red[i]);
+  uint32_t m = red[0];
+  for (int i = 1; i < NT / WAVE; ++i) m = red[i] > m ? red[i] : m;
   return m;
 }
 
-// Completes a momentum sweep (run by one whole block): min_dt = min(dtmax, per-tile
-// minima) as in sfincs_momentum.f90:121,542-545, and the q/uv double buffer flips.
+// The CFL reduction's word for the largest denominator `den` of a thread's wet points (their
+// step is 1 / den; 0: none), ordered so that the largest word means the smallest step, and the
+// step that the largest word of a sweep stands for, at most dtmax. FP32: the bits of den,
+// since a correctly rounded quotient falls as its divisor grows, so the division runs once a
+// sweep instead of once a thread. FP64 twin: the step itself is rounded to f32 before it is
+// compared, so its bits, reversed. A step that is zero or NaN does not take part.
+template <typename R>
+__device__ __forceinline__ uint32_t step_key(R den, float dtmax);
+template <>
+__device__ __forceinline__ uint32_t step_key<float>(float den, float dtmax) {
+  (void)dtmax;
+  const uint32_t b = __float_as_uint(den);   // den >= 0
+  return b < 0x7f800000u ? b : 0u;
+}
+template <>
+__device__ __forceinline__ uint32_t step_key<double>(double den, float dtmax) {
+  const float dt = den > 0.0 ? fminf(dtmax, (float)(1.0 / den)) : dtmax;
+  return dt > 0.f && dt < dtmax ? 0x7fffffffu - __float_as_uint(dt) : 0u;
+}
+__device__ __forceinline__ float key_step(uint32_t key, int fp64, float dtmax) {
+  if (key == 0u) return dtmax;
+  return fp64 ? __uint_as_float(0x7fffffffu - key) : fminf(dtmax, 1.0f / __uint_as_float(key));
+}
+
+// t / d for the tile numbers of a list, with magic = div_magic(d, tiles): a multiplication in
+// the scalar unit instead of a division on the vector unit in every block.
+__device__ __forceinline__ int tile_div(int t, int d, uint32_t magic) {
+  return magic ? (int)__umulhi((uint32_t)t, magic) : t / d;
+}
+// ceil(2^32 / d): floor(t * magic / 2^32) = t / d while t * d < 2^32 (the excess of magic over
+// 2^32 / d is below 1); otherwise 0.
+inline uint32_t div_magic(int d, size_t tiles) {
+  if (d < 2 || tiles * (size_t)d >= ((size_t)1 << 32)) return 0u;
+  return (uint32_t)((((uint64_t)1 << 32) + (uint64_t)d - 1) / (uint64_t)d);
+}
+
+// Completes a momentum sweep (run by one whole block): min_dt = min(dtmax, the points'
+// steps) as in sfincs_momentum.f90:121,542-545, and the q/uv double buffer flips.
 // Blocks of the per-scenario kernels (forcing, fold): one block covers a scenario's
 // boundary points and tile minima.
 constexpr int FBLOCK = 1024;
@@ -324,25 +377,25 @@ __device__ void fold_sweep(const DevInst& I) {
   if (threadIdx.x == 0) sh_done = S->mom_done;
   __syncthreads();
   if (!sh_done) return;
-  float v = I.c.dtmax;
-  const auto p = G(I.blkmin);
+  uint32_t v = 0u;
+  const auto p = G(I.blkkey);
   const int n = I.nmt;
   // chunks of 32 entries per thread, each chunk in one round trip (clamped indices
-  // repeat the last entry, which leaves the minimum unchanged)
+  // repeat the last entry, which leaves the maximum unchanged)
   for (int base = 0; base < n; base += 32 * FBLOCK) {
-    float w[32];
+    uint32_t w[32];
 #pragma unroll
     for (int j = 0; j < 32; ++j) w[j] = p[min(base + (int)threadIdx.x + j * FBLOCK, n - 1)];
 #pragma unroll
-    for (int j = 0; j < 32; ++j) v = fminf(v, w[j]);
+    for (int j = 0; j < 32; ++j) v = w[j] > v ? w[j] : v;
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
       const int i = base + (int)threadIdx.x + j * FBLOCK;
-      if (i < n) p[i] = I.c.dtmax;   // ready for the next sweep
+      if (i < n) p[i] = 0u;   // ready for the next sweep
     }
   }
-  v = block_min<FBLOCK>(v);
-  if (threadIdx.x == 0) { S->cur ^= 1; S->mom_done = 0; S->min_dt = v; }
+  v = block_max<FBLOCK>(v);
+  if (threadIdx.x == 0) { S->cur ^= 1; S->mom_done = 0; S->min_dt = key_step(v, I.fp64, I.c.dtmax); }
   __syncthreads();
 }
 
@@ -454,24 +507,24 @@ __device__ __forceinline__ void copy_words(T* dst, const T* src) {
   if ((int)threadIdx.x < NW) ((uint32_t*)dst)[threadIdx.x] = ((const uint32_t*)src)[threadIdx.x];
 }
 
-// Fold of the tile minima into the image, leaving the minima in place (a step computed
+// Fold of the tile keys into the image, leaving the keys in place (a step computed
 // ahead of its turn leaves them to the launch that commits it, which resets them, and to
 // a host-side fold, which re-reads them).
 template <int NT>
 __device__ void fold_image(const DevInst& I, StepImage& F) {
   if (F.s.mom_done) {
-    float v = I.c.dtmax;
-    const auto p = G(I.blkmin);
+    uint32_t v = 0u;
+    const auto p = G(I.blkkey);
     const int n = I.nmt;
     for (int base = 0; base < n; base += 16 * NT) {
-      float w[16];
+      uint32_t w[16];
 #pragma unroll
       for (int j = 0; j < 16; ++j) w[j] = p[min(base + (int)threadIdx.x + j * NT, n - 1)];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) v = fminf(v, w[j]);
+      for (int j = 0; j < 16; ++j) v = w[j] > v ? w[j] : v;
     }
-    v = block_min<NT>(v);
-    if (threadIdx.x == 0) { F.s.cur ^= 1; F.s.mom_done = 0; F.s.min_dt = v; F.folded = 1; }
+    v = block_max<NT>(v);
+    if (threadIdx.x == 0) { F.s.cur ^= 1; F.s.mom_done = 0; F.s.min_dt = key_step(v, I.fp64, I.c.dtmax); F.folded = 1; }
   } else if (threadIdx.x == 0) {
     F.folded = 0;
   }
@@ -479,8 +532,64 @@ __device__ void fold_image(const DevInst& I, StepImage& F) {
 }
 
 __device__ void reset_tiles(const DevInst& I) {
-  const auto p = G(I.blkmin);
-  for (int i = threadIdx.x; i < I.nmt; i += blockDim.x) p[i] = I.c.dtmax;
+  const auto p = G(I.blkkey);
+  for (int i = threadIdx.x; i < I.nmt; i += blockDim.x) p[i] = 0u;
+}
+
+// The step's scalars: whether it runs, its time step from the last sweep's minimum, the new
+// time, the instability check (sfincs_lib.f90:379-392, 634-648).
+__device__ __forceinline__ int advance(const Consts& c, Scalars& sc) {
+  if (sc.error_pending) { sc.error = 1; sc.error_pending = 0; sc.t = (double)c.t1 + 1.0; }
+  const int go = (sc.t < sc.tend) && !sc.error;
+  sc.active = go;
+  if (go) {
+    sc.nt += 1;
+    sc.dt = c.alpha * sc.min_dt;
+    sc.dtchk = c.alpha * sc.min_dt;
+    sc.t = sc.t + (double)sc.dt;
+    if (sc.dtchk < c.dtmin && sc.nt > 1) sc.error_pending = 1;
+  }
+  return go;
+}
+
+// Uniform rain (m/s) at time t and the series position (sfincs_meteo.f90:1520-1545).
+__device__ __forceinline__ float rain_at(const DevInst& I, double t, int32_t& last) {
+  int itp;
+  for (itp = last; itp <= I.ntprcp; ++itp)
+    if ((double)G(I.tprcpt)[itp - 1] > t) break;
+  if (itp > I.ntprcp) itp = I.ntprcp;
+  if (itp < 2) itp = 2;   // series start at or before t0 (checked at initialisation)
+  const float twfac = (float)((t - (double)G(I.tprcpt)[itp - 2]) / (double)(G(I.tprcpt)[itp - 1] - G(I.tprcpt)[itp - 2]));
+  last = itp - 1;
+  return (G(I.tprcpv)[itp - 2] * (1.0f - twfac) + G(I.tprcpv)[itp - 1] * twfac) / (float)(1000 * 3600);
+}
+
+// Position of time t in the boundary series: the samples itb0, itb1 (1-based) and the weight of
+// the second (sfincs_boundaries.f90:700-727).
+__device__ __forceinline__ float boundary_at(const DevInst& I, double t, int32_t& last, int32_t& itb0, int32_t& itb1) {
+  const int nt = I.ntbnd;
+  float tb = 0.f;
+  itb0 = 1; itb1 = 1;
+  if ((double)G(I.t_bnd)[0] > t - (double)1.0e-3f) tb = G(I.t_bnd)[0];
+  else if ((double)G(I.t_bnd)[nt - 1] < t + (double)1.0e-3f) { itb0 = nt; itb1 = nt; tb = G(I.t_bnd)[nt - 1]; }
+  else {
+    for (int itb = last; itb <= nt; ++itb)
+      if ((double)G(I.t_bnd)[itb - 1] > t + (double)1.0e-6f) { itb0 = itb - 1; itb1 = itb; tb = (float)t; last = itb - 1; break; }
+  }
+  return (tb - G(I.t_bnd)[itb0 - 1]) / sfx::vmax<float>(G(I.t_bnd)[itb1 - 1] - G(I.t_bnd)[itb0 - 1], 1.0e-6f);
+}
+
+// Position of time t in the discharge series (0: past its end, the discharges stay) and the
+// discharge of one source there (sfincs_discharges.f90:353-369).
+__device__ __forceinline__ int sources_at(const DevInst& I, double t, int32_t& last) {
+  for (int it = max(last, 2); it <= I.ntsrc; ++it)
+    if ((double)G(I.tsrc)[it - 1] > t) { last = it - 1; return it; }
+  return 0;
+}
+__device__ __forceinline__ float source_at(const DevInst& I, double t, int it, int src) {
+  const float q0v = G(I.qsrc)[(it - 2) * I.nsrc + src], q1v = G(I.qsrc)[(it - 1) * I.nsrc + src];
+  return (float)((double)q0v + (double)(q1v - q0v) * (t - (double)G(I.tsrc)[it - 2]) /
+                                   (double)(G(I.tsrc)[it - 1] - G(I.tsrc)[it - 2]));
 }
 
 // The step scalars (sfincs_lib.f90:379-392) and the forcing series at the new time
@@ -491,20 +600,8 @@ __device__ void step_series(const DevInst& I, StepImage& F, float* qout, int mod
   if (threadIdx.x == 0) {
     Scalars& sc = F.s;
     int go = 1;
-    if (mode == 0) {
-      if (sc.error_pending) { sc.error = 1; sc.error_pending = 0; sc.t = (double)c.t1 + 1.0; }
-      go = (sc.t < sc.tend) && !sc.error;
-      sc.active = go;
-      if (go) {
-        sc.nt += 1;
-        sc.dt = c.alpha * sc.min_dt;
-        sc.dtchk = c.alpha * sc.min_dt;
-        sc.t = sc.t + (double)sc.dt;
-        if (sc.dtchk < c.dtmin && sc.nt > 1) sc.error_pending = 1;
-      }
-    } else {
-      sc.active = 1;
-    }
+    if (mode == 0) go = advance(c, sc);
+    else sc.active = 1;
     F.go = go;
   }
   __syncthreads();
@@ -560,43 +657,17 @@ __device__ void step_series(const DevInst& I, StepImage& F, float* qout, int mod
     }
   }
   if (wave == 2 && lane == 0 && (c.flags & sfx::F_PRECIP) && I.ntprcp > 0) {
-    int itp;
-    for (itp = F.s.itprcplast; itp <= I.ntprcp; ++itp)
-      if ((double)G(I.tprcpt)[itp - 1] > t) break;
-    if (itp > I.ntprcp) itp = I.ntprcp;
-    if (itp < 2) itp = 2;   // series start at or before t0 (checked at initialisation)
-    const float twfac = (float)((t - (double)G(I.tprcpt)[itp - 2]) / (double)(G(I.tprcpt)[itp - 1] - G(I.tprcpt)[itp - 2]));
-    F.s.netprcp = (G(I.tprcpv)[itp - 2] * (1.0f - twfac) + G(I.tprcpv)[itp - 1] * twfac) / (float)(1000 * 3600);
-    F.s.itprcplast = itp - 1;
+    F.s.netprcp = rain_at(I, t, F.s.itprcplast);
   }
   if (wave == 3 && lane == 0 && I.nbnd > 0) {
-    int itb0 = 1, itb1 = 1;
-    float tb = 0.f;
-    const int nt = I.ntbnd;
-    if ((double)G(I.t_bnd)[0] > t - (double)1.0e-3f) { itb0 = 1; itb1 = 1; tb = G(I.t_bnd)[0]; }
-    else if ((double)G(I.t_bnd)[nt - 1] < t + (double)1.0e-3f) { itb0 = nt; itb1 = nt; tb = G(I.t_bnd)[nt - 1]; }
-    else {
-      for (int itb = F.s.itbndlast; itb <= nt; ++itb)
-        if ((double)G(I.t_bnd)[itb - 1] > t + (double)1.0e-6f) { itb0 = itb - 1; itb1 = itb; tb = (float)t; F.s.itbndlast = itb - 1; break; }
-    }
-    F.itb0 = itb0; F.itb1 = itb1;
-    F.tbfac = (tb - G(I.t_bnd)[itb0 - 1]) / sfx::vmax<float>(G(I.t_bnd)[itb1 - 1] - G(I.t_bnd)[itb0 - 1], 1.0e-6f);
+    F.tbfac = boundary_at(I, t, F.s.itbndlast, F.itb0, F.itb1);
   }
   if (wave == 0 && I.nsrc > 0) {   // discharges: the series position once, the sources one lane each
     int itsel = 0;
-    if (lane == 0) {
-      for (int it = max(F.s.itsrclast, 2); it <= I.ntsrc; ++it)
-        if ((double)G(I.tsrc)[it - 1] > t) { itsel = it; F.s.itsrclast = it - 1; break; }
-    }
+    if (lane == 0) itsel = sources_at(I, t, F.s.itsrclast);
     itsel = __shfl(itsel, 0, WAVE);
-    if (itsel) {
-      const int it = itsel;
-      for (int src = lane; src < I.nsrc; src += WAVE) {
-        const float q0v = G(I.qsrc)[(it - 2) * I.nsrc + src], q1v = G(I.qsrc)[(it - 1) * I.nsrc + src];
-        G(qout)[src] = (float)((double)q0v + (double)(q1v - q0v) * (t - (double)G(I.tsrc)[it - 2]) /
-                                                  (double)(G(I.tsrc)[it - 1] - G(I.tsrc)[it - 2]));
-      }
-    }
+    if (itsel)
+      for (int src = lane; src < I.nsrc; src += WAVE) G(qout)[src] = source_at(I, t, itsel, src);
   }
   __syncthreads();
 }
@@ -716,7 +787,8 @@ struct BndPt {
 // update_boundary_points / update_boundary_conditions (:728-917) for the point's boundary
 // cell, and the point's other inputs (:941-1000).
 template <typename R>
-__device__ __forceinline__ void bnd_load(const DevInst& I, const BndStep<R>& B, int ib, BndPt<R>& p) {
+__device__ __forceinline__ void bnd_load(const DevInst& I, const BndStep<R>& B, int ib, BndPt<R>& p, GA<const double> zs,
+                                         GA<const double> vol, GA<const R> uvmean) {
   const Consts& c = I.c;
   p.ib = ib;
   p.nmb = G(I.k2_nmb)[ib];
@@ -725,15 +797,15 @@ __device__ __forceinline__ void bnd_load(const DevInst& I, const BndStep<R>& B, 
   p.nmi = G(I.k2_nmi)[ib];
   p.ip = G(I.k2_slot)[ib];
   p.dir = G(I.k2_dir)[ib];
-  p.zsnmi = (R)G(I.zs)[p.nmi];
-  p.uvm = G((const R*)I.uvmean)[ib];
+  p.zsnmi = (R)zs[p.nmi];
+  p.uvm = uvmean[ib];
   p.kcuv = G(I.kcuv)[p.ip];
   p.floorz = I.subgrid ? G(I.z_zmin)[p.nmb] : G(I.zb)[p.nmb];
   if (I.subgrid) {
     const float4 s4 = ldf4(G(I.uv_s4), p.ip);
     p.zmaxu = s4.x; p.havg_zmax = s4.y;
     p.zbuv_or_zmin = G(I.uv_zmin)[p.ip];
-    p.vol_nmi = G(I.vol)[p.nmi];
+    p.vol_nmi = vol[p.nmi];
     p.zb_nmi = 0.0f;
   } else {
     p.zbuv_or_zmin = G(I.k2_zbuv)[ib];
@@ -778,7 +850,7 @@ __device__ __forceinline__ void bnd_load(const DevInst& I, const BndStep<R>& B, 
   } else if (p.kb == 5) {
     // downstream river cell (:878-901): the interior level plus the slope offset, raised
     // to the bed, in f64 (the interior cell is an ordinary cell, which no boundary step writes)
-    const double zst = sfx::vmax<double>(G(I.zs)[G(I.gb_rcell)[indb]] + (double)G(I.gb_rdzs)[indb], (double)p.floorz);
+    const double zst = sfx::vmax<double>(zs[G(I.gb_rcell)[indb]] + (double)G(I.gb_rdzs)[indb], (double)p.floorz);
     p.zsb0 = (float)zst;
     p.zsb1 = p.zsb0;
   } else {
@@ -788,11 +860,11 @@ __device__ __forceinline__ void bnd_load(const DevInst& I, const BndStep<R>& B, 
 }
 
 // update_boundary_fluxes (:941-1117), bndtype 1 (weakly reflective), from the loaded inputs.
-template <typename R, typename QP, typename MP>
-__device__ __forceinline__ void bnd_finish(const DevInst& I, const BndStep<R>& B, const BndPt<R>& p, QP q, QP uv,
-                                           MP uvmean, MP zsmax) {
+// The point's discharge goes to qb, its velocity to ub, its filtered mean to um.
+template <typename R>
+__device__ __forceinline__ void bnd_flux(const DevInst& I, const BndStep<R>& B, const BndPt<R>& p, R& qb, R& ub, R& um) {
   const Consts& c = I.c;
-  const int ip = p.ip, ib = p.ib, nmb = p.nmb;
+  const int ip = p.ip;
   const R zsnmi = p.zsnmi;
   R zsnmb = p.zsb1;
   R zs0nmb = p.zsb0;
@@ -822,18 +894,18 @@ __device__ __forceinline__ void bnd_finish(const DevInst& I, const BndStep<R>& B
     zsnmb = sfx::vmax<R>(zsnmb, (R)p.floorz);
     zs0nmb = sfx::vmax<R>(zs0nmb, (R)p.floorz);
   }
-  R qb, um;   // the point's discharge and uvmean as the filter below reads them
+  R um0;   // uvmean as the filter below reads it
   const R uvm = p.uvm;
   if (hnmb < huth + R(1.0e-6f) || p.kcuv == 3) {
     qb = R(0);
-    um = R(0);
-    q[ip] = R(0); uv[ip] = R(0);
+    ub = R(0);
+    um0 = R(0);
   } else {
     const R g = c.g;
     const R ui = sfx::rsqrt_<R>(g / hnmb) * (zsnmb - zs0nmb);
     const int dir = p.dir;
-    const R ub = (R)dir * (R(2) * ui - sfx::rsqrt_<R>(g / hnmb) * (zsnmi - zs0nmb));
-    qb = ub * hnmb + uvm;
+    const R ui2 = (R)dir * (R(2) * ui - sfx::rsqrt_<R>(g / hnmb) * (zsnmi - zs0nmb));
+    qb = ui2 * hnmb + uvm;
     if (I.subgrid) {
       if (p.vol_nmi <= 0.0) qb = (dir == 1) ? sfx::vmax<R>(qb, R(0)) : sfx::vmin<R>(qb, R(0));
       if (zsnmb - (R)p.floorz < huth) qb = (dir == 1) ? sfx::vmin<R>(qb, R(0)) : sfx::vmax<R>(qb, R(0));
@@ -841,15 +913,23 @@ __device__ __forceinline__ void bnd_finish(const DevInst& I, const BndStep<R>& B
       if (zsnmi - (R)p.zb_nmi <= huth) qb = (dir == 1) ? sfx::vmax<R>(qb, R(0)) : sfx::vmin<R>(qb, R(0));
       if (zsnmb - (R)p.floorz < huth) qb = (dir == 1) ? sfx::vmin<R>(qb, R(0)) : sfx::vmax<R>(qb, R(0));
     }
-    q[ip] = qb;
-    uv[ip] = sfx::vmax<R>(sfx::vmin<R>(qb / hnmb, R(4)), R(-4));
-    um = uvm;
+    ub = sfx::vmax<R>(sfx::vmin<R>(qb / hnmb, R(4)), R(-4));
+    um0 = uvm;
   }
-  if (c.btfilter >= -1.0e-6f) uvmean[ib] = B.factime * qb + B.facrel * B.one_minus_factime * um;
-  else uvmean[ib] = R(0);
-  G(I.zs)[nmb] = (double)p.zsb1;
-  mark_cell(I, nmb);
-  if (c.flags & sfx::F_ZSMAX) zsmax[nmb] = (R)sfx::vmax<double>((double)zsmax[nmb], (double)p.zsb1);
+  if (c.btfilter >= -1.0e-6f) um = B.factime * qb + B.facrel * B.one_minus_factime * um0;
+  else um = R(0);
+}
+
+template <typename R, typename QP, typename MP>
+__device__ __forceinline__ void bnd_finish(const DevInst& I, const BndStep<R>& B, const BndPt<R>& p, QP q, QP uv,
+                                           MP uvmean, MP zsmax) {
+  R qb, ub, um;
+  bnd_flux<R>(I, B, p, qb, ub, um);
+  q[p.ip] = qb; uv[p.ip] = ub;
+  uvmean[p.ib] = um;
+  G(I.zs)[p.nmb] = (double)p.zsb1;
+  mark_cell(I, p.nmb);
+  if (I.c.flags & sfx::F_ZSMAX) zsmax[p.nmb] = (R)sfx::vmax<double>((double)zsmax[p.nmb], (double)p.zsb1);
 }
 
 // One block per scenario: the step's fold, scalars and forcing series (committed from
@@ -909,8 +989,9 @@ __global__ void __launch_bounds__(FBLOCK) k_forcing(const DevInst* __restrict__ 
   for (int k0 = threadIdx.x; k0 < I.nflux; k0 += 2 * FBLOCK) {
     const int k1 = k0 + FBLOCK;
     BndPt<R> a, b;
-    bnd_load<R>(I, B, G(I.k2_flux)[k0], a);
-    if (k1 < I.nflux) bnd_load<R>(I, B, G(I.k2_flux)[k1], b);
+    bnd_load<R>(I, B, G(I.k2_flux)[k0], a, G((const double*)I.zs), G((const double*)I.vol), G((const R*)I.uvmean));
+    if (k1 < I.nflux)
+      bnd_load<R>(I, B, G(I.k2_flux)[k1], b, G((const double*)I.zs), G((const double*)I.vol), G((const R*)I.uvmean));
     bnd_finish<R>(I, B, a, q, uv, uvmean, zsmax);
     if (k1 < I.nflux) bnd_finish<R>(I, B, b, q, uv, uvmean, zsmax);
   }
@@ -921,6 +1002,12 @@ __global__ void __launch_bounds__(FBLOCK) k_forcing(const DevInst* __restrict__ 
 }
 
 // ----------------------------------------------------------------------------- momentum
+// Counts a uv-point of class k (NCNT) when counting is on. Counted in place, so that ordinary
+// runs carry no counters in registers.
+__device__ __forceinline__ void tally(const DevInst& I, int tile, int k) {
+  if (I.count) atomicAdd((unsigned int*)&G(I.blkcnt)[NCNT * (uint32_t)tile + (uint32_t)k], 1u);
+}
+
 // Loads the wet/dry threshold of a uv-point: subgrid_uv_zmin or zbuvmx.
 template <bool SUBGRID>
 __device__ __forceinline__ float uv_floor(const DevInst& I, int slot) {
@@ -1007,7 +1094,8 @@ __device__ __forceinline__ void gather_uv(const DevInst& I, QP q0, QP u0, int s,
   in.qy_nm = q0[v_nm]; in.qy_nmu = q0[v_nmu]; in.qy_ndm = q0[v_ndm]; in.qy_ndmu = q0[v_ndmu];
   in.uu_nmd = u0[s_nmd]; in.uu_nmu = u0[s_nmu]; in.uu_ndm = u0[s_ndm]; in.uu_num = u0[s_num];
   in.v_ndm = u0[v_ndm]; in.v_ndmu = u0[v_ndmu]; in.v_nm = u0[v_nm]; in.v_nmu = u0[v_nmu];
-  in.kcuv_nmd = G(I.kcuv)[s_nmd]; in.kcuv_nmu = G(I.kcuv)[s_nmu];
+  in.kcuv_nmd = in.kcuv_nmu = 0;
+  if (I.c.flags & sfx::F_THETA) { in.kcuv_nmd = G(I.kcuv)[s_nmd]; in.kcuv_nmu = G(I.kcuv)[s_nmu]; }
   in.kfuv = G(I.kfuv)[s] & 1; in.mask_adv = G(I.mask_adv)[s];
   if (SUBGRID) {
     in.vol_nm = G(I.vol)[c_nm]; in.vol_nmu = G(I.vol)[c_nmu];
@@ -1018,7 +1106,7 @@ __device__ __forceinline__ void gather_uv(const DevInst& I, QP q0, QP u0, int s,
 }
 
 template <typename R, bool SUBGRID>
-__device__ __forceinline__ void mom_cell(const DevInst& I, int tile, int* cnt, R& mden) {
+__device__ __forceinline__ void mom_cell(const DevInst& I, int tile, R& mden) {
   const auto S = G(I.sc);
   const int cur = __builtin_amdgcn_readfirstlane(S->cur);
   const R dt = (R)S->dt;
@@ -1027,7 +1115,7 @@ __device__ __forceinline__ void mom_cell(const DevInst& I, int tile, int* cnt, R
   const auto q1 = G((R*)I.q[cur ^ 1]);
   const auto u1 = G((R*)I.uv[cur ^ 1]);
   const int nmax = I.nmax, mmax = I.mmax, np = I.np, dm = 2 * np;
-  const int tn = tile % I.mntn, tmi = tile / I.mntn;
+  const int tmi = tile_div(tile, I.mntn, I.mmagic), tn = tile - tmi * I.mntn;
   const int n = tn * I.mtn + (threadIdx.x & (I.mtn - 1));
   const int m = tmi * I.mtm + (threadIdx.x >> I.mtn_sh);
   if (n >= nmax || m >= mmax) return;
@@ -1058,16 +1146,16 @@ __device__ __forceinline__ void mom_cell(const DevInst& I, int tile, int* cnt, R
       uv_meteo<R>(I, S, c, c + nmax, iu);
       int br = 0;
       finish_uv<R, SUBGRID>(I, c, iu, fu, dt, q1, u1, mden, br);
-      cnt[br]++;
+      tally(I, tile, br);
     } else if (ku == 3) {
       q1[c] = weir_flux<R>(I, c, iu.zs_nm, iu.zs_nmu); u1[c] = R(0);
-      cnt[0]++;
+      tally(I, tile, 0);
     } else {
       q1[c] = iu.qx_nm; u1[c] = iu.uu_nm;
-      cnt[0]++;
+      tally(I, tile, 0);
     }
   } else {
-    cnt[0]++;
+    tally(I, tile, 0);
   }
   if (hv) {
     const int s = np + c;
@@ -1076,57 +1164,65 @@ __device__ __forceinline__ void mom_cell(const DevInst& I, int tile, int* cnt, R
       uv_meteo<R>(I, S, c, c + 1, iv);
       int br = 0;
       finish_uv<R, SUBGRID>(I, s, iv, fv, dt, q1, u1, mden, br);
-      cnt[br]++;
+      tally(I, tile, br);
     } else if (kv == 3) {
       q1[s] = weir_flux<R>(I, s, iv.zs_nm, iv.zs_nmu); u1[s] = R(0);
-      cnt[0]++;
+      tally(I, tile, 0);
     } else {
       q1[s] = iv.qx_nm; u1[s] = iv.uu_nm;
-      cnt[0]++;
+      tally(I, tile, 0);
     }
   } else {
-    cnt[0]++;
+    tally(I, tile, 0);
   }
 }
 
-// The stencil of dense uv-point (n, m) of plane `vplane` beyond its branch inputs: the q
-// and uv of its neighbours in both planes (missing ones read the dummy slot or the point
-// itself, as the reference's tables for a full rectangle give them), the kcuv of its two
-// neighbours along its direction, its advection mask and the cell values of its two cells.
-template <typename R, bool SUBGRID, typename QC>
-__device__ __forceinline__ void point_stencil(const DevInst& I, int n, int m, int vplane, int kf, QC q0, QC u0,
-                                              sfx::UvIn<R>& in) {
-  const int nmax = I.nmax, mmax = I.mmax, np = I.np, dm = 2 * np;
-  const bool hu = m < mmax - 1, hv = n < nmax - 1;
-  const int c = m * nmax + n;
-  const int s = vplane ? np + c : c;
-  const int c_nmu = vplane ? c + 1 : c + nmax;
-  int s_nmd, s_nmu, s_ndm, s_num, v_nm, v_ndm, v_nmu, v_ndmu;
-  if (!vplane) {
-    s_nmd = m >= 1 ? c - nmax : dm; s_nmu = m + 1 < mmax - 1 ? c + nmax : dm;
-    s_ndm = n >= 1 ? c - 1 : c; s_num = n < nmax - 1 ? c + 1 : c;
-    v_nm = hv ? np + c : dm; v_ndm = n >= 1 ? np + c - 1 : dm;
-    v_nmu = hv ? np + c + nmax : dm; v_ndmu = n >= 1 ? np + c + nmax - 1 : dm;
+// The stencil of dense uv-point (n, m) of plane VP (0: u, 1: v) beyond its branch inputs: the q
+// and uv of its neighbours in both planes, the kcuv of its two neighbours along its direction,
+// its advection mask and the cell values of its two cells. Where the reference's tables for a
+// full rectangle give the dummy point (q = uv = 0), the neighbour's slot is one that holds no
+// point (a u-slot of the last column m = mmax - 1, a v-slot of the last row n = nmax - 1): such
+// slots are created as zeros and never written, so they are read like any other. Only the row
+// below m = 0 would lie outside the plane; it is taken from the last column, which holds no
+// u-point. So five offset registers and the instructions' offset fields reach all eight
+// neighbours at the grid's edges as inside, and a missing cross neighbour is replaced by the
+// point itself after the load. Choosing the dummy for each neighbour took about 60 vector
+// instructions a point.
+// vol and zsd are the cells' volumes and wiggle detector (subgrid meshes).
+template <typename R, bool SUBGRID, int VP, typename QC>
+__device__ __forceinline__ void point_stencil(const DevInst& I, int n, int m, int kf, QC q0, QC u0, GA<const double> vol,
+                                              GA<const R> zsd, sfx::UvIn<R>& in) {
+  const uint32_t nmax = I.nmax, np = I.np, c = (uint32_t)m * nmax + (uint32_t)n;
+  const uint32_t below = c - nmax + (m == 0 ? np : 0u), above = c + nmax;   // (n, m - 1), (n, m + 1)
+  if (VP == 0) {
+    const uint32_t v = np + c, v2 = np + above;
+    in.qx_nm = q0[c]; in.uu_nm = u0[c];
+    in.qx_nmd = q0[below]; in.qx_nmu = q0[above]; in.uu_nmd = u0[below]; in.uu_nmu = u0[above];
+    in.qy_nm = q0[v]; in.qy_nmu = q0[v2]; in.qy_ndm = q0.at(v, -1); in.qy_ndmu = q0.at(v2, -1);
+    in.v_nm = u0[v]; in.v_nmu = u0[v2]; in.v_ndm = u0.at(v, -1); in.v_ndmu = u0.at(v2, -1);
+    const R d = u0[n == 0 ? c : c - 1u], u = u0.at(c, 1);
+    in.uu_ndm = d; in.uu_num = n == (int)nmax - 1 ? in.uu_nm : u;
   } else {
-    s_nmd = n >= 1 ? s - 1 : dm; s_nmu = n + 1 < nmax - 1 ? s + 1 : dm;
-    s_ndm = m >= 1 ? s - nmax : s; s_num = m < mmax - 1 ? s + nmax : s;
-    v_nm = hu ? c : dm; v_ndm = m >= 1 ? c - nmax : dm;
-    v_nmu = hu ? c + 1 : dm; v_ndmu = m >= 1 ? c + 1 - nmax : dm;
+    const uint32_t s = np + c;
+    in.qx_nm = q0[s]; in.uu_nm = u0[s];
+    in.qx_nmd = q0.at(s, -1); in.qx_nmu = q0.at(s, 1); in.uu_nmd = u0.at(s, -1); in.uu_nmu = u0.at(s, 1);
+    in.qy_nm = q0[c]; in.qy_nmu = q0.at(c, 1); in.qy_ndm = q0[below]; in.qy_ndmu = q0.at(below, 1);
+    in.v_nm = u0[c]; in.v_nmu = u0.at(c, 1); in.v_ndm = u0[below]; in.v_ndmu = u0.at(below, 1);
+    in.uu_ndm = u0[m == 0 ? s : s - nmax]; in.uu_num = u0[m == I.mmax - 1 ? s : s + nmax];
   }
-  in.qx_nm = q0[s]; in.uu_nm = u0[s];
-  in.qx_nmd = q0[s_nmd]; in.qx_nmu = q0[s_nmu];
-  in.qy_nm = q0[v_nm]; in.qy_nmu = q0[v_nmu]; in.qy_ndm = q0[v_ndm]; in.qy_ndmu = q0[v_ndmu];
-  in.uu_nmd = u0[s_nmd]; in.uu_nmu = u0[s_nmu]; in.uu_ndm = u0[s_ndm]; in.uu_num = u0[s_num];
-  in.v_ndm = u0[v_ndm]; in.v_ndmu = u0[v_ndmu]; in.v_nm = u0[v_nm]; in.v_nmu = u0[v_nmu];
-  in.kcuv_nmd = G(I.kcuv)[s_nmd]; in.kcuv_nmu = G(I.kcuv)[s_nmu];
+  const uint32_t s = VP ? np + c : c;
+  in.kcuv_nmd = in.kcuv_nmu = 0;
+  if (I.c.flags & sfx::F_THETA) {
+    in.kcuv_nmd = VP ? G(I.kcuv).at(s, -1) : G(I.kcuv)[below]; in.kcuv_nmu = VP ? G(I.kcuv).at(s, 1) : G(I.kcuv)[above];
+  }
   in.kfuv = kf & 1; in.mask_adv = G(I.mask_adv)[s];
   if (SUBGRID) {
-    in.vol_nm = G(I.vol)[c]; in.vol_nmu = G(I.vol)[c_nmu];
-    in.zsderv_nm = G((const R*)I.zsderv)[c]; in.zsderv_nmu = G((const R*)I.zsderv)[c_nmu];
+    in.vol_nm = vol[c]; in.vol_nmu = VP ? vol.at(c, 1) : vol[above];
+    in.zsderv_nm = zsd[c]; in.zsderv_nmu = VP ? zsd.at(c, 1) : zsd[above];
   } else {
-    in.zb_nm = G(I.zb)[c]; in.zb_nmu = G(I.zb)[c_nmu];
+    in.zb_nm = G(I.zb)[c]; in.zb_nmu = VP ? G(I.zb).at(c, 1) : G(I.zb)[above];
   }
-  in.idir = vplane; in.iref = 1; in.itype = 0;
+  in.idir = VP; in.iref = 1; in.itype = 0;
 }
 
 // Dense scenarios, one thread per uv-point: tile 2t covers the u-points and tile 2t+1 the
@@ -1141,11 +1237,11 @@ __device__ __forceinline__ void point_stencil(const DevInst& I, int n, int m, in
 template <typename R, bool SUBGRID, typename QC, typename QW>
 __device__ __forceinline__ bool point_finish(const DevInst& I, GA<Scalars> S, int n, int m, int vplane, int kc, int kf,
                                              double zs_nm, double zs_nmu, float fl, R dt, QC q0, QC u0, QW q1,
-                                             QW u1, int* cnt, R& mden) {
-  const int nmax = I.nmax, mmax = I.mmax, np = I.np, dm = 2 * np;
+                                             QW u1, int tile, R& mden) {
+  const int nmax = I.nmax, mmax = I.mmax, np = I.np;
   if (n >= nmax || m >= mmax) return true;
   const bool hu = m < mmax - 1, hv = n < nmax - 1;
-  if (vplane ? !hv : !hu) { cnt[0]++; return true; }
+  if (vplane ? !hv : !hu) { tally(I, tile, 0); return true; }
   const int c = m * nmax + n;
   const int s = vplane ? np + c : c;
   const int c_nmu = vplane ? c + 1 : c + nmax;
@@ -1156,28 +1252,31 @@ __device__ __forceinline__ bool point_finish(const DevInst& I, GA<Scalars> S, in
   else tb.zbuvmx = fl;
   if (kc == 3) {
     q1[s] = weir_flux<R>(I, s, zs_nm, zs_nmu); u1[s] = R(0);
-    cnt[0]++;
+    tally(I, tile, 0);
     return false;
   }
   if (!(kc == 1 || kc == 6)) {
     q1[s] = q0[s]; u1[s] = u0[s];
-    cnt[0]++;
+    tally(I, tile, 0);
     return false;
   }
   R zsu;
   if (!sfx::uv_wet<R, SUBGRID>(in, tb, I.c, zsu)) {
-    if (kf & KF_ZERO2) { cnt[4]++; return true; }   // both buffers already hold the zeros
+    if (kf & KF_ZERO2) { tally(I, tile, 4); return true; }   // both buffers already hold the zeros
     q1[s] = R(0); u1[s] = R(0);
     G(I.kfuv)[s] = (kf & KF_ZERO1) ? KF_ZERO2 : KF_ZERO1;
-    cnt[1]++;
+    tally(I, tile, 1);
     return false;
   }
   // the rest of the stencil of a wet point
   uv_meteo<R>(I, S, c, c_nmu, in);
-  point_stencil<R, SUBGRID>(I, n, m, vplane, kf, q0, u0, in);
+  const auto vol = G((const double*)I.vol);
+  const auto zsd = G((const R*)I.zsderv);
+  if (vplane) point_stencil<R, SUBGRID, 1>(I, n, m, kf, q0, u0, vol, zsd, in);
+  else point_stencil<R, SUBGRID, 0>(I, n, m, kf, q0, u0, vol, zsd, in);
   int br = 0;
   wet_uv<R, SUBGRID>(I, s, in, tb, zsu, dt, q1, u1, mden, br, kf);
-  cnt[br]++;
+  tally(I, tile, br);
   return false;
 }
 
@@ -1188,12 +1287,12 @@ __device__ __forceinline__ bool point_finish(const DevInst& I, GA<Scalars> S, in
 // scalars are read and the active test is made. Returns false if the scenario is not
 // active (nothing is written).
 template <typename R, bool SUBGRID, int P>
-__device__ __forceinline__ bool mom_point(const DevInst& I, Scalars* Sp, int tile, int* cnt, R& mden, bool& held) {
+__device__ __forceinline__ bool mom_point(const DevInst& I, Scalars* Sp, int tile, R& mden, bool& held) {
   const auto S = G(Sp);
   const int nmax = I.nmax, mmax = I.mmax, np = I.np;
   const int vplane = tile & 1;
   const int t = tile >> 1;
-  const int tn = t % I.mntn, tmi = t / I.mntn;
+  const int tmi = tile_div(t, I.mntn, I.mmagic), tn = t - tmi * I.mntn;
   const int n = tn * I.mtn + (threadIdx.x & (I.mtn - 1));
   const int m0 = tmi * I.mtm * P + (threadIdx.x >> I.mtn_sh);
   int kc[P], kf[P];
@@ -1223,23 +1322,23 @@ __device__ __forceinline__ bool mom_point(const DevInst& I, Scalars* Sp, int til
 #pragma unroll
   for (int j = 0; j < P; ++j)
     held = point_finish<R, SUBGRID>(I, S, n, m0 + j * I.mtm, vplane, kc[j], kf[j], za[j], zb[j], fl[j], dt, q0, u0, q1,
-                                    u1, cnt, mden) && held;
+                                    u1, tile, mden) && held;
   return true;
 }
 
 // Points of a skipped (quiescent) per-point tile, for the counters: class 5, or copied (0)
 // for the absent edge slots, as a run would count them.
 template <int P>
-__device__ __forceinline__ void count_tile_points(const DevInst& I, int tile, int* cnt) {
+__device__ __forceinline__ void count_tile_points(const DevInst& I, int tile) {
   const int nmax = I.nmax, mmax = I.mmax;
   const int vplane = tile & 1, t = tile >> 1;
-  const int tn = t % I.mntn, tmi = t / I.mntn;
+  const int tmi = tile_div(t, I.mntn, I.mmagic), tn = t - tmi * I.mntn;
   const int n = tn * I.mtn + (threadIdx.x & (I.mtn - 1));
   const int m0 = tmi * I.mtm * P + (threadIdx.x >> I.mtn_sh);
 #pragma unroll
   for (int j = 0; j < P; ++j) {
     const int m = m0 + j * I.mtm;
-    if (n < nmax && m < mmax) ++cnt[(vplane ? n < nmax - 1 : m < mmax - 1) ? 5 : 0];
+    if (n < nmax && m < mmax) tally(I, tile, (vplane ? n < nmax - 1 : m < mmax - 1) ? 5 : 0);
   }
 }
 
@@ -1300,7 +1399,7 @@ __device__ __forceinline__ void strip_nbrs(Row<R>& w) {
 }
 
 template <typename R, bool SUBGRID>
-__device__ __forceinline__ void mom_strip(const DevInst& I, int tile, int* cnt, R& mden) {
+__device__ __forceinline__ void mom_strip(const DevInst& I, int tile, R& mden) {
   const auto S = G(I.sc);
   const int cur = __builtin_amdgcn_readfirstlane(S->cur);
   const R dt = (R)S->dt;
@@ -1351,16 +1450,16 @@ __device__ __forceinline__ void mom_strip(const DevInst& I, int tile, int* cnt, 
           else { in.zb_nm = (float)B.zd; in.zb_nmu = (float)C.zd; }
           int br = 0;
           finish_uv<R, SUBGRID>(I, c, in, uv_floor<SUBGRID>(I, c), dt, q1, u1, mden, br);
-          cnt[br]++;
+          tally(I, tile, br);
         } else if (B.ku == 3) {
           q1[c] = weir_flux<R>(I, c, B.z, C.z); u1[c] = R(0);
-          cnt[0]++;
+          tally(I, tile, 0);
         } else {
           q1[c] = B.uq; u1[c] = B.uu;
-          cnt[0]++;
+          tally(I, tile, 0);
         }
       } else {
-        cnt[0]++;
+        tally(I, tile, 0);
       }
       // v-point between cells (n,m) and (n+1,m)
       if (n < nmax - 1) {
@@ -1383,16 +1482,16 @@ __device__ __forceinline__ void mom_strip(const DevInst& I, int tile, int* cnt, 
           else { in.zb_nm = (float)B.zd; in.zb_nmu = (float)B.r_zd; }
           int br = 0;
           finish_uv<R, SUBGRID>(I, s, in, uv_floor<SUBGRID>(I, s), dt, q1, u1, mden, br);
-          cnt[br]++;
+          tally(I, tile, br);
         } else if (B.kv == 3) {
           q1[s] = weir_flux<R>(I, s, B.z, B.r_z); u1[s] = R(0);
-          cnt[0]++;
+          tally(I, tile, 0);
         } else {
           q1[s] = B.vq; u1[s] = B.vu;
-          cnt[0]++;
+          tally(I, tile, 0);
         }
       } else {
-        cnt[0]++;
+        tally(I, tile, 0);
       }
     }
     A = B; B = C; C = D;
@@ -1403,7 +1502,7 @@ __device__ __forceinline__ void mom_strip(const DevInst& I, int tile, int* cnt, 
 // As on dense meshes, the branch inputs come first and only wet points read the
 // neighbour tables and values.
 template <typename R, bool SUBGRID>
-__device__ __forceinline__ void mom_idx(const DevInst& I, int tile, int* cnt, R& mden) {
+__device__ __forceinline__ void mom_idx(const DevInst& I, int tile, R& mden) {
   const auto S = G(I.sc);
   const int cur = __builtin_amdgcn_readfirstlane(S->cur);
   const R dt = (R)S->dt;
@@ -1424,20 +1523,20 @@ __device__ __forceinline__ void mom_idx(const DevInst& I, int tile, int* cnt, R&
   else tb.zbuvmx = G(I.zbuvmx)[ip];
   if (kc == 3) {
     q1[ip] = weir_flux<R>(I, ip, in.zs_nm, in.zs_nmu); u1[ip] = R(0);
-    cnt[0]++;
+    tally(I, tile, 0);
     return;
   }
   if (!(kc == 1 || kc == 6)) {
     q1[ip] = q0[ip]; u1[ip] = u0[ip];
-    cnt[0]++;
+    tally(I, tile, 0);
     return;
   }
   R zsu;
   if (!sfx::uv_wet<R, SUBGRID>(in, tb, I.c, zsu)) {   // zero flags as in the per-point kernel
-    if (kf & KF_ZERO2) { cnt[4]++; return; }
+    if (kf & KF_ZERO2) { tally(I, tile, 4); return; }
     q1[ip] = R(0); u1[ip] = R(0);
     G(I.kfuv)[ip] = (kf & KF_ZERO1) ? KF_ZERO2 : KF_ZERO1;
-    cnt[1]++;
+    tally(I, tile, 1);
     return;
   }
   const uint8_t f = G(I.uvf)[ip];
@@ -1452,7 +1551,8 @@ __device__ __forceinline__ void mom_idx(const DevInst& I, int tile, int* cnt, R&
     in.qy_nm = q0[f2]; in.qy_nmu = q0[h]; in.qy_ndm = q0[e]; in.qy_ndmu = q0[g];
     in.uu_nmd = u0[a]; in.uu_nmu = u0[b]; in.uu_ndm = u0[cdn]; in.uu_num = u0[d];
     in.v_ndm = u0[e]; in.v_ndmu = u0[g]; in.v_nm = u0[f2]; in.v_nmu = u0[h];
-    in.kcuv_nmd = G(I.kcuv)[a]; in.kcuv_nmu = G(I.kcuv)[b];
+    in.kcuv_nmd = in.kcuv_nmu = 0;
+    if (I.c.flags & sfx::F_THETA) { in.kcuv_nmd = G(I.kcuv)[a]; in.kcuv_nmu = G(I.kcuv)[b]; }
   } else {
     in.qx_nmd = in.qx_nmu = in.qy_nm = in.qy_nmu = in.qy_ndm = in.qy_ndmu = R(0);
     in.uu_nmd = in.uu_nmu = in.uu_ndm = in.uu_num = in.v_ndm = in.v_ndmu = in.v_nm = in.v_nmu = R(0);
@@ -1468,38 +1568,19 @@ __device__ __forceinline__ void mom_idx(const DevInst& I, int tile, int* cnt, R&
   }
   int br = 0;
   wet_uv<R, SUBGRID>(I, ip, in, tb, zsu, dt, q1, u1, mden, br, kf);
-  cnt[br]++;
+  tally(I, tile, br);
 }
 
-// Wave epilogue of a momentum tile, without a block barrier: the wave's minimum time step
-// lowers blkmin[tile] (NaN or non-positive values do not take part; the reduction starts
-// at dtmax), the wave's per-branch counts are added to the tile's blkcnt slots, and the
-// sweep-done flag is raised. Positive floats order like their bit patterns, so the
-// minimum is an unsigned atomic min. Waves with no value below dtmax (every dry wave)
-// skip the reduction.
+// Wave epilogue of a momentum tile, without a block barrier: the wave's largest key raises
+// blkkey[tile] (waves without a wet point skip that), and the sweep-done flag is raised.
 template <typename R>
-__device__ __forceinline__ void mom_epilogue(const DevInst& I, int tile, R mden, const int* cnt) {
-  // the thread's step: min(dtmax, 1 / den) over its wet points (dtmax when it has none)
-  float mdt = I.c.dtmax;
-  if (mden > R(0)) mdt = fminf(mdt, (float)(R(1) / mden));
-  const float v = mdt == mdt && mdt > 0.f ? mdt : I.c.dtmax;
-  if (__ballot(v < I.c.dtmax)) {
-    const uint32_t m = wave_min_last(__float_as_uint(v));
-    if (threadIdx.x % WAVE == WAVE - 1) atomicMin((unsigned int*)&G(I.blkmin)[tile], m);
+__device__ __forceinline__ void mom_epilogue(const DevInst& I, int tile, R mden) {
+  const uint32_t key = step_key<R>(mden, I.c.dtmax);
+  if (__ballot(key != 0u)) {
+    const uint32_t m = wave_max_last(key);
+    if (threadIdx.x % WAVE == WAVE - 1) atomicMax((unsigned int*)&G(I.blkkey)[tile], m);
   }
-  int cw[NCNT] = {0, 0, 0, 0, 0, 0};
-  if (I.count)
-    for (int k = 0; k < NCNT; ++k) {
-      int v = cnt[k];
-      for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-      cw[k] = v;
-    }
-  if (threadIdx.x % WAVE == 0) {
-    if (tile == 0 && threadIdx.x == 0) { G(I.sc)->mom_done = 1; G(I.sc)->ahead = 0; }   // a new sweep: no staged step
-    if (I.count)
-      for (int k = 0; k < NCNT; ++k)
-        if (cw[k]) atomicAdd((unsigned int*)&G(I.blkcnt)[NCNT * (uint32_t)tile + k], (unsigned int)cw[k]);
-  }
+  if (tile == 0 && threadIdx.x == 0) { G(I.sc)->mom_done = 1; G(I.sc)->ahead = 0; }   // a new sweep: no staged step
 }
 
 // The (scenario, tile) of this block; false for the padding of a list. The scenario is an
@@ -1531,9 +1612,8 @@ __global__ void __launch_bounds__(BLOCK) k_mom_cell(const DevInst* __restrict__ 
   Scalars* Sp = L.direct ? L.sc : I.sc;
   if (!G(Sp)->active) return;
   R mden = R(0);
-  int cnt[NCNT] = {0, 0, 0, 0, 0, 0};
-  mom_cell<R, SUBGRID>(I, tile, cnt, mden);
-  mom_epilogue<R>(I, tile, mden, cnt);
+  mom_cell<R, SUBGRID>(I, tile, mden);
+  mom_epilogue<R>(I, tile, mden);
 }
 
 template <typename R, bool SUBGRID, int P>
@@ -1543,19 +1623,18 @@ __global__ void __launch_bounds__(BLOCK) k_mom_point(const DevInst* __restrict__
   const DevInst& I = insts[inst];
   Scalars* Sp = L.direct ? L.sc : I.sc;
   R mden = R(0);
-  int cnt[NCNT] = {0, 0, 0, 0, 0, 0};
   if (G(I.mq)[tile] == 0x01010101u && G(I.md)[tile] == 0) {   // quiescent: nothing would change
     if (!G(Sp)->active) return;
-    if (I.count) count_tile_points<P>(I, tile, cnt);
-    mom_epilogue<R>(I, tile, mden, cnt);
+    if (I.count) count_tile_points<P>(I, tile);
+    mom_epilogue<R>(I, tile, mden);
     return;
   }
   bool held;
-  if (!mom_point<R, SUBGRID, P>(I, Sp, tile, cnt, mden, held)) return;   // scenario not active
+  if (!mom_point<R, SUBGRID, P>(I, Sp, tile, mden, held)) return;   // scenario not active
   if (threadIdx.x == 0) G(I.md)[tile] = 0;
   const bool wave_held = __ballot(!held) == 0;
   if (threadIdx.x % WAVE == 0) G((uint8_t*)I.mq)[4 * (uint32_t)tile + threadIdx.x / WAVE] = wave_held ? 1 : 0;
-  mom_epilogue<R>(I, tile, mden, cnt);
+  mom_epilogue<R>(I, tile, mden);
 }
 
 template <typename R, bool SUBGRID>
@@ -1566,9 +1645,8 @@ __global__ void __launch_bounds__(BLOCK) k_mom_strip(const DevInst* __restrict__
   Scalars* Sp = L.direct ? L.sc : I.sc;
   if (!G(Sp)->active) return;
   R mden = R(0);
-  int cnt[NCNT] = {0, 0, 0, 0, 0, 0};
-  mom_strip<R, SUBGRID>(I, tile, cnt, mden);
-  mom_epilogue<R>(I, tile, mden, cnt);
+  mom_strip<R, SUBGRID>(I, tile, mden);
+  mom_epilogue<R>(I, tile, mden);
 }
 
 template <typename R, bool SUBGRID>
@@ -1579,9 +1657,8 @@ __global__ void __launch_bounds__(BLOCK) k_mom_idx(const DevInst* __restrict__ i
   Scalars* Sp = L.direct ? L.sc : I.sc;
   if (!G(Sp)->active) return;
   R mden = R(0);
-  int cnt[NCNT] = {0, 0, 0, 0, 0, 0};
-  mom_idx<R, SUBGRID>(I, tile, cnt, mden);
-  mom_epilogue<R>(I, tile, mden, cnt);
+  mom_idx<R, SUBGRID>(I, tile, mden);
+  mom_epilogue<R>(I, tile, mden);
 }
 
 // Combined uv-points at refinement transitions (sfincs_momentum.f90:757-779).
@@ -1902,16 +1979,377 @@ __global__ void __launch_bounds__(BLOCK) k_continuity(const DevInst* __restrict_
   if (RX && (I.c.flags & (sfx::F_INFIL | sfx::F_MPRCP | sfx::F_CNA))) add_infiltrated(I, tile, inf);   // every lane of the block is here
 }
 
+// ------------------------------------------------------------------------------- step kernel
+// One launch per time step: the step's scalars, its boundary, momentum and continuity, on dense
+// FP32 meshes with the default physics (the rule is step_rule). As separate launches, a small
+// mesh spends its step in three kernels of 4 to 6 us, each a chain of dependent reads after the
+// caches were emptied at the launch boundary, and a large one reads its levels and discharges twice.
+//
+// What makes one launch enough:
+//  * A block owns 63 neighbouring columns of cells by I.frows rows and computes the discharge of
+//    every face of its cells: its own faces (right and above each cell) and again those of the
+//    row before and the column to the left, which the neighbouring blocks own. The repeated faces
+//    (one row in frows, one lane in 64) give the same bits; only the owner stores them. The four
+//    faces of a cell then meet in LDS and the cell is updated without another pass over memory.
+//  * Everything that one block updates and another reads is held on two sides: a step reads one
+//    side of the levels, volumes, wiggle detector, kfuv and boundary means and writes the other,
+//    as q and uv always were.
+//  * The time step needs the largest CFL key of the whole last sweep: blocks raise one of 64
+//    words, and every block of the next launch reduces them itself (one load) and derives the
+//    step's scalars itself; the block of tile 0 also stores them for the next launch.
+//  * A block within reach of the water-level boundary computes the boundary points it reads from
+//    the interior levels and stores them in the buffer it reads from; blocks that share a point
+//    store the same bits. Nobody else reads those places in this launch.
+//
+// Columns are counted along n through the row blocks (column j = row block * nmax + n), so that
+// 63 of 64 lanes own cells whatever nmax is. The blocks that do nothing (all points dry before
+// and after, no cell changed) twice in a row hold the same values on both sides and are skipped
+// until a neighbouring block does something, rain falls or the host writes state; blocks with
+// boundary, source or inactive cells always run.
+constexpr int STEP_COLS = WAVE - 1;
+constexpr uint8_t FT_RUN = 1, FT_BND = 2, FT_BAL = 4;          // fflag: never skipped; has boundary points; has balance faces
+
+// kfuv on the step kernel's sides: 1 wet; 0, 2, 4 dry -- 2 when the kernel has stored q = uv = 0
+// for the point in its last step, 4 when it did so in its last two (both q buffers hold zeros, so
+// nothing is stored while it stays dry). Readers of kfuv take bit 0.
+constexpr int8_t SF_ZERO1 = 2, SF_ZERO2 = 4;
+
+// What decides a face's branch, read ahead of its turn: kcuv, kfuv, the levels of its two cells and
+// its wet/dry threshold. n, m: its cell; ok: the face exists and is wanted.
+struct FaceIn {
+  double za, zb;
+  float floor;
+  int kc, kf, m;
+  bool ok;
+};
+// Faces of a tile: items 0 .. fr are the u faces of its rows -1 .. fr-1, items fr+1 .. 2 fr the v
+// faces of its rows (one wave each).
+template <bool SG>
+__device__ __forceinline__ FaceIn step_load(const DevInst& I, int item, int n, int m0, bool jok, int lane, GA<const double> zs,
+                                            GA<const int8_t> kf0) {
+  FaceIn f;
+  const int fr = I.frows;
+  const bool v = item > fr;
+  f.m = m0 + (v ? item - fr - 1 : item - 1);
+  f.ok = jok && item < 2 * fr + 1 && (v ? f.m < I.mmax && n < I.nmax - 1 : lane > 0 && f.m >= 0 && f.m < I.mmax - 1);
+  f.za = f.zb = 0.0; f.floor = 0.f; f.kc = f.kf = 0;
+  if (f.ok) {
+    const uint32_t c = (uint32_t)f.m * (uint32_t)I.nmax + (uint32_t)n;
+    const uint32_t s = v ? (uint32_t)I.np + c : c;
+    f.kc = G(I.kcuv)[s]; f.kf = kf0[s];
+    f.za = zs[c]; f.zb = zs[v ? c + 1u : c + (uint32_t)I.nmax];
+    f.floor = uv_floor<SG>(I, (int)s);
+  }
+  return f;
+}
+
+// One face (uv-point) of plane VP between cell (n, m) and its right (0) or upper (1) neighbour.
+// Returns its discharge after the sweep; stores it, the velocity and kfuv when `own`.
+template <bool SG, int VP>
+__device__ __forceinline__ float step_face(const DevInst& I, const FaceIn& f, int n, bool own, float dt,
+                                           GA<const double> vol, GA<const float> zsd, GA<int8_t> kf1,
+                                           GA<const float> q0, GA<const float> u0, GA<float> q1, GA<float> u1,
+                                           float& mden, bool& act) {
+  const uint32_t c = (uint32_t)f.m * (uint32_t)I.nmax + (uint32_t)n;
+  const uint32_t s = VP ? (uint32_t)I.np + c : c;
+  sfx::UvIn<float> in;
+  in.zs_nm = f.za;
+  in.zs_nmu = f.zb;
+  sfx::UvTables tb;
+  if (SG) tb.zmin = f.floor;
+  else tb.zbuvmx = f.floor;
+  if (f.kc != 1) {   // a boundary point's value of this step, or a closed point's
+    const float q = q0[s], u = u0[s];
+    if (own) { q1[s] = q; u1[s] = u; }
+    return q;
+  }
+  float zsu;
+  if (!sfx::uv_wet<float, SG>(in, tb, I.c, zsu)) {
+    if (f.kf & 1) act = true;
+    if (own) {
+      if (!(f.kf & SF_ZERO2)) { q1[s] = 0.f; u1[s] = 0.f; }
+      kf1[s] = (f.kf & (SF_ZERO1 | SF_ZERO2)) ? SF_ZERO2 : SF_ZERO1;
+    }
+    return 0.f;
+  }
+  act = true;
+  point_stencil<float, SG, VP>(I, n, f.m, f.kf, q0, u0, vol, zsd, in);
+  if (SG) {
+    const float4 s4 = ldf4(G(I.uv_s4), s);
+    tb.zmax = s4.x; tb.havg_zmax = s4.y; tb.nrep_zmax = s4.z; tb.navg_w = s4.w; tb.fnfit = G(I.uv_fnfit)[s];
+  } else {
+    tb.gn2uv = G(I.gn2uv)[s];
+  }
+  const sfx::UvOut<float> o = sfx::uv_update<float, SG, true>(
+      in, tb, I.c, zsu, sfx::GRow<const float4>{G(I.uv_lev), SG ? s * (uint32_t)I.c.nl : 0u}, G(I.x73),
+      sfx::pow_tables_g(I.pw), dt);
+  if (own) { q1[s] = o.q; u1[s] = o.uv; kf1[s] = 1; }
+  if (o.den > mden) mden = o.den;
+  return o.q;
+}
+
+// One cell of the step: sources, the update from its four faces, the new side. Returns whether
+// anything changed. KCS_STEADY as in cont_update: the cell's last update, without inflow, rain or
+// source, changed nothing, so both sides hold its values and the same update again is skipped.
+template <bool SG>
+__device__ __forceinline__ bool step_cell(const DevInst& I, uint32_t c, const Scalars& n, float q_md, float q_mu,
+                                          float q_nd, float q_nu, bool dry_sky, GA<const double> zs0s, GA<double> zs1s,
+                                          GA<const double> vol0, GA<double> vol1, GA<const float> zsd0, GA<float> zsd1) {
+  const uint8_t kraw = G(I.kcs)[c];
+  const int kcs = kraw & KCS_MASK;
+  const float dt = n.dt;
+  const bool quiet = (kraw & (KCS_MASK | KCS_SOURCE)) == 1 && dry_sky && q_md == 0.f && q_mu == 0.f && q_nd == 0.f &&
+                     q_nu == 0.f && !(I.c.flags & sfx::F_QEXT);
+  if (quiet && (kraw & KCS_STEADY)) return false;
+  double zs = zs0s[c];
+  const double zs_in = zs;
+  const auto zsmaxp = G((float*)I.zsmax);
+  float zsmax = zsmaxp[c];
+  const float zsmax_in = zsmax;
+  const float qx = (I.c.flags & sfx::F_QEXT) ? G(I.qext)[c] : 0.f;
+  if (qx != 0.f && kcs == 1) atomicAdd(I.bal + 3, (double)(qx * dt) * (double)I.c.cell_area[0]);
+  const int itsel = (kraw & KCS_SOURCE) ? (int)n.itsrclast : 0;   // the sample before this step's time, 0: past the series
+  bool changed;
+  if (SG) {
+    double vol = vol0[c];
+    const double vol_in = vol;
+    if (kraw & KCS_SOURCE) {   // point sources of this cell, in source order (sfincs_continuity.f90:311-325)
+      double applied = 0.0;
+      for (int s = 0; s < I.nsrc; ++s)
+        if (G(I.src_cell)[s] == (int)c) {
+          const float qs = n.ahead ? source_at(I, n.t, itsel + 1, s) : G(I.qtsrc)[s];
+          if (vol >= 0) {
+            vol = vol + (double)(qs * dt);
+            applied += (double)(qs * dt);
+          }
+        }
+      if (applied != 0.0) atomicAdd(I.bal + 1, applied);
+    }
+    const auto zs0p = G((float*)I.zs0);
+    float zs0 = zs0p[c], zsd = zsd0[c], stor = 0.f;
+    const float zs0_in = zs0, zsd_in = zsd;
+    sfx::cell_subgrid<float, true>(zs, vol, zs0, zsd, zsmax, kcs, q_md, q_mu, q_nd, q_nu, n.netprcp, qx, stor, 1,
+                                   G(I.z_zmin)[c], G(I.z_zmax)[c], G(I.z_volmax)[c],
+                                   sfx::GRow<const float>{G(I.z_dep), c * (uint32_t)I.c.nl}, I.c, dt);
+    vol1[c] = vol;
+    zsd1[c] = zsd;
+    changed = !same_bits(vol, vol_in) || !same_bits(zs0, zs0_in) || !same_bits(zsd, zsd_in);
+    if (!same_bits(zs0, zs0_in)) zs0p[c] = zs0;
+  } else {
+    changed = false;
+    if (kraw & KCS_SOURCE) {   // (:87-106)
+      const double before = zs;
+      for (int s = 0; s < I.nsrc; ++s)
+        if (G(I.src_cell)[s] == (int)c) {
+          const float inc = (n.ahead ? source_at(I, n.t, itsel + 1, s) : G(I.qtsrc)[s]) * dt / I.c.cell_area[0];
+          zs = sfx::vmax<double>(zs + (double)inc, (double)G(I.zb)[c]);
+        }
+      if (zs != before) atomicAdd(I.bal + 1, (zs - before) * (double)I.c.cell_area[0]);
+    }
+    sfx::cell_regular<float, true>(zs, zsmax, kcs, q_md, q_mu, q_nd, q_nu, n.netprcp, qx, 1, I.c, dt);
+  }
+  zs1s[c] = zs;
+  if (!same_bits(zsmax, zsmax_in)) { zsmaxp[c] = zsmax; changed = true; }
+  changed = changed || !same_bits(zs, zs_in);
+  const bool steady = quiet && !changed;
+  if (steady != ((kraw & KCS_STEADY) != 0)) G(I.kcs)[c] = (uint8_t)((kraw & ~KCS_STEADY) | (steady ? KCS_STEADY : 0));
+  return changed;
+}
+
+template <bool SG>
+__global__ void __launch_bounds__(BLOCK, SG ? 7 : 8) k_step(const DevInst* __restrict__ insts, WorkList L, int flip) {
+  extern __shared__ float lq[];   // u faces of rows -1 .. frows-1, then v faces of rows 0 .. frows-1, a wave wide
+  __shared__ uint32_t lkey[BLOCK / WAVE];
+  int tile, inst;
+  if (!work_item(L, blockIdx.x, gridDim.x, tile, inst)) return;
+  const DevInst& I = insts[inst];
+  ScalarBlock* SB = (ScalarBlock*)(L.direct ? L.sc : I.sc);
+  const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  constexpr int W = BLOCK / WAVE;
+
+  // the step's scalars, in every wave
+  Scalars n;
+  {
+    const auto src = G((const uint32_t*)&SB->s[flip]);
+    uint32_t words[sizeof(Scalars) / 4];
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(Scalars) / 4); ++k) words[k] = src[k];
+    __builtin_memcpy(&n, words, sizeof(Scalars));
+  }
+  const int kset = n.kset, side = n.side, cur = n.cur;
+  const uint8_t flag = G(I.fflag)[tile], woken = G(I.fwake)[(uint32_t)(side * I.fnt + tile)];
+  const uint32_t quiet = G((const uint32_t*)I.fquiet)[tile];   // one byte per wave
+  const bool asleep = !woken && !(flag & FT_RUN) && quiet == 0x02020202u && !(I.c.flags & sfx::F_QEXT);
+  if (asleep && !(I.c.flags & sfx::F_PRECIP)) return;
+
+  const auto zs0 = G((const double*)I.zs_s[side]);
+  const auto zs1 = G(I.zs_s[side ^ 1]);
+  const auto vol0 = G((const double*)I.vol_s[side]);
+  const auto vol1 = G(I.vol_s[side ^ 1]);
+  const auto zsd0 = G((const float*)I.zsd_s[side]);
+  const auto zsd1 = G(I.zsd_s[side ^ 1]);
+  const auto kf0 = G((const int8_t*)I.kf_s[side]);
+  const auto kf1 = G(I.kf_s[side ^ 1]);
+  const auto q0 = G((const float*)I.q[cur]);
+  const auto u0 = G((const float*)I.uv[cur]);
+  const auto q1 = G((float*)I.q[cur ^ 1]);
+  const auto u1 = G((float*)I.uv[cur ^ 1]);
+  const int nmax = I.nmax, mmax = I.mmax, fr = I.frows;
+  const int j = tile * STEP_COLS + lane - 1;
+  const bool jok = j >= 0 && j < I.fcols;
+  const int mb = tile_div(max(j, 0), nmax, I.fmagic), cn = j - mb * nmax, m0 = mb * fr;
+  FaceIn f = step_load<SG>(I, w, cn, m0, jok, lane, zs0, kf0);   // in flight while the scalars are worked out
+
+  if (n.pend) {
+    uint32_t k = wave_max_last(G(SB->key[kset])[lane * KEY_STRIDE]);
+    n.min_dt = key_step((uint32_t)__builtin_amdgcn_readlane((int)k, WAVE - 1), 0, I.c.dtmax);
+    n.pend = 0;
+  }
+  const int go = advance(I.c, n);
+  const int k1 = kset == 2 ? 0 : kset + 1, k2 = k1 == 2 ? 0 : k1 + 1;
+  int itb0 = 1, itb1 = 1;
+  float tbfac = 0.f;
+  if (go) {
+    if ((I.c.flags & sfx::F_PRECIP) && I.ntprcp > 0) n.netprcp = rain_at(I, n.t, n.itprcplast);
+    n.ahead = 0;   // here: whether this step's time lies inside the discharge series
+    if (flag & FT_RUN) {
+      if (I.nbnd > 0) tbfac = boundary_at(I, n.t, n.itbndlast, itb0, itb1);
+      if (I.nsrc > 0) n.ahead = sources_at(I, n.t, n.itsrclast) != 0;
+      n.factime = sfx::vmin<float>(n.dt / I.c.btfilter, 1.0f);
+      n.one_minus_factime = 1.0f - n.factime;
+      n.facrel = 1.0f - sfx::vmin<float>(n.dt / I.c.btrelax, 1.0f);
+    }
+  }
+  if (tile == 0) {
+    if (go) {
+      if (w == 0) G(SB->key[k2])[lane * KEY_STRIDE] = 0u;
+      if (n.ahead)
+        for (int k = threadIdx.x; k < I.nsrc; k += BLOCK) G(I.qtsrc)[k] = source_at(I, n.t, n.itsrclast + 1, k);
+      if (threadIdx.x == 0 && (I.c.flags & sfx::F_PRECIP)) I.bal[2] = I.bal[2] + (double)(n.netprcp * n.dt) * I.rain_area;
+    }
+    Scalars o = n;
+    o.ahead = 0; o.mom_done = 0;
+    if (go) { o.pend = 1; o.kset = k1; o.side = side ^ 1; o.cur = cur ^ 1; }
+    if (threadIdx.x == 0) SB->s[flip ^ 1] = o;
+  }
+  const bool dry_sky = !(I.c.flags & sfx::F_PRECIP) || n.netprcp == 0.f;
+  if (!go || (asleep && dry_sky)) return;
+
+  if (flag & FT_BND) {   // the boundary points this block reads, at the step's time (see above)
+    const BndStep<float> B{itb0, itb1, tbfac, n.t, n.factime, n.facrel, n.one_minus_factime, MeteoNow{}};
+    const auto um0 = G((const float*)I.um_s[side]);
+    const auto um1 = G(I.um_s[side ^ 1]);
+    const int e1 = G(I.fb_ptr)[tile + 1];
+    for (int e = G(I.fb_ptr)[tile] + (int)threadIdx.x; e < e1; e += BLOCK) {
+      const int ent = G(I.fb_ent)[e];
+      BndPt<float> p;
+      bnd_load<float>(I, B, ent >> 1, p, zs0, vol0, um0);
+      float qb, ub, um;
+      bnd_flux<float>(I, B, p, qb, ub, um);
+      G((float*)I.q[cur])[p.ip] = qb;
+      G((float*)I.uv[cur])[p.ip] = ub;
+      G(I.zs_s[side])[p.nmb] = (double)p.zsb1;
+      if (ent & 1) um1[p.ib] = um;
+    }
+    __syncthreads();
+  }
+
+  float mden = 0.f;
+  bool act = false;
+  for (int i = w; i < 2 * fr + 1; i += W) {
+    const FaceIn next = step_load<SG>(I, i + W, cn, m0, jok, lane, zs0, kf0);
+    float q = 0.f;
+    if (i <= fr) {
+      if (f.ok) q = step_face<SG, 0>(I, f, cn, i > 0, n.dt, vol0, zsd0, kf1, q0, u0, q1, u1, mden, act);
+    } else {
+      if (f.ok) q = step_face<SG, 1>(I, f, cn, lane > 0, n.dt, vol0, zsd0, kf1, q0, u0, q1, u1, mden, act);
+    }
+    lq[i * WAVE + lane] = q;
+    f = next;
+  }
+  const uint32_t key = wave_max_last(step_key<float>(mden, I.c.dtmax));
+  if (lane == WAVE - 1) lkey[w] = key;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t k = lkey[0];
+    for (int i = 1; i < W; ++i) k = lkey[i] > k ? lkey[i] : k;
+    if (k) atomicMax(&SB->key[k1][(tile & (NKEY - 1)) * KEY_STRIDE], k);
+    if (woken) G(I.fwake)[(uint32_t)(side * I.fnt + tile)] = 0;   // every wave has read it
+  }
+  const float* lv = lq + (fr + 1) * WAVE;
+  for (int r = w; r < fr; r += W) {
+    const int m = m0 + r;
+    if (jok && lane > 0 && m < mmax)
+      if (step_cell<SG>(I, (uint32_t)m * (uint32_t)nmax + (uint32_t)cn, n, lq[r * WAVE + lane], lq[(r + 1) * WAVE + lane],
+                        lv[r * WAVE + lane - 1], lv[r * WAVE + lane], dry_sky, zs0, zs1, vol0, vol1, zsd0, zsd1))
+        act = true;
+  }
+  if ((flag & FT_BAL) && w == 0) {   // volume into the interior cells through this block's balance faces
+    double acc = 0.0;
+    const int e1 = G(I.ff_ptr)[tile + 1];
+    for (int e = G(I.ff_ptr)[tile] + lane; e < e1; e += WAVE) {
+      const int f = G(I.ff_ent)[e];
+      acc += G(I.bf_coef)[f] * (double)q1[G(I.bf_slot)[f]];
+    }
+    for (int o = WAVE / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, WAVE);
+    if (lane == 0 && acc != 0.0) atomicAdd(I.bal, acc * (double)n.dt);
+  }
+  if (__ballot(act)) {   // wake the blocks around this one for the next step
+    if (lane == 0) G(I.fquiet)[(uint32_t)(tile * W + w)] = 0;
+    const int below = tile * STEP_COLS - 1 - nmax, above = tile * STEP_COLS - 1 + nmax;   // first column of the rows around
+    const int t = lane < 2 ? tile - 1 + 2 * lane
+                           : (lane < 5 ? (below >= 0 ? below / STEP_COLS : 0) + lane - 2 : above / STEP_COLS + lane - 5);
+    if (lane < 8 && t >= 0 && t < I.fnt) G(I.fwake)[(uint32_t)((side ^ 1) * I.fnt + t)] = 1;
+  } else if (lane == 0) {
+    const uint8_t k = (uint8_t)(quiet >> (8 * w));
+    G(I.fquiet)[(uint32_t)(tile * W + w)] = k < 2 ? k + 1 : 2;
+  }
+}
+
+// Brings the scalars back to the first set after an odd number of steps.
+__global__ void __launch_bounds__(WAVE) k_step_scalars(const DevInst* __restrict__ insts, const int32_t* __restrict__ ids) {
+  const DevInst& I = insts[ids[blockIdx.x]];
+  copy_words(&I.sb->s[0], &I.sb->s[1]);
+}
+
+// The levels back to their first side (after an odd number of steps), for the kernels that work
+// on one side only.
+__global__ void __launch_bounds__(BLOCK) k_step_settle(const DevInst* __restrict__ I0) {
+  const DevInst& I = *I0;
+  for (uint32_t c = blockIdx.x * BLOCK + threadIdx.x; c < (uint32_t)I.nslot; c += gridDim.x * BLOCK) {
+    I.kf_s[0][c] = I.kf_s[1][c];
+    if (c < (uint32_t)I.np) {
+      I.zs_s[0][c] = I.zs_s[1][c];
+      if (I.subgrid) { I.vol_s[0][c] = I.vol_s[1][c]; I.zsd_s[0][c] = I.zsd_s[1][c]; }
+    }
+    if (c < (uint32_t)I.nkcuv2) I.um_s[0][c] = I.um_s[1][c];
+  }
+}
+
+// No cell keeps its steady bit, and with uv set no uv-point its zero flags (host writes, and changes
+// between the step kernel and the separate ones, whose flags mean different things).
+__global__ void __launch_bounds__(BLOCK) k_clear_marks(const DevInst* __restrict__ I0, int uv) {
+  const DevInst& I = *I0;
+  for (uint32_t c = blockIdx.x * BLOCK + threadIdx.x; c < (uint32_t)I.nslot; c += gridDim.x * BLOCK) {
+    if (c < (uint32_t)I.np) I.kcs[c] &= (uint8_t)~KCS_STEADY;
+    if (uv) {
+      I.kf_s[0][c] &= 1;
+      if (I.fnt) I.kf_s[1][c] &= 1;
+    }
+  }
+}
+
 // FP64 volume accumulator: sum over active cells of V (subgrid) or zs*A (regular).
 __global__ void __launch_bounds__(BLOCK) k_volume(const DevInst* __restrict__ I0, double* out) {
   const DevInst& I = *I0;
   double acc = 0.0;
+  const auto zs = G(I.zs_s[I.sc->side]), vol = G(I.vol_s[I.sc->side]);
   for (int c = blockIdx.x * BLOCK + threadIdx.x; c < I.np; c += gridDim.x * BLOCK) {
     const int k = G(I.kcs)[c] & KCS_MASK;
     if (k == 0) continue;
     const int iref = I.dense ? 1 : G(I.z_iref)[c];
-    if (I.subgrid) acc += G(I.vol)[c];
-    else acc += G(I.zs)[c] * (double)I.c.cell_area[iref - 1];
+    if (I.subgrid) acc += vol[c];
+    else acc += zs[c] * (double)I.c.cell_area[iref - 1];
   }
   for (int o = WAVE / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, WAVE);
   __shared__ double red[BLOCK / WAVE];
@@ -1931,10 +2369,11 @@ __global__ void k_zero_f64(double* p) { *p = 0.0; }
 __global__ void __launch_bounds__(BLOCK) k_balance_volume(const DevInst* __restrict__ I0) {
   const DevInst& I = *I0;
   double v = 0.0, st = 0.0;
+  const auto zs = G(I.zs_s[I.sc->side]), vol = G(I.vol_s[I.sc->side]);
   for (int c = blockIdx.x * BLOCK + threadIdx.x; c < I.np; c += gridDim.x * BLOCK) {
     if ((G(I.kcs)[c] & KCS_MASK) != 1) continue;
     const int iref = I.dense ? 1 : G(I.z_iref)[c];
-    v += I.subgrid ? G(I.vol)[c] : G(I.zs)[c] * (double)I.c.cell_area[iref - 1];
+    v += I.subgrid ? vol[c] : zs[c] * (double)I.c.cell_area[iref - 1];
     if (I.c.flags & sfx::F_STORAGE)
       st += I.fp64 ? G((const double*)I.storage)[c] : (double)G((const float*)I.storage)[c];
   }
@@ -1996,10 +2435,13 @@ struct sfx_handle {
   int tile_tn = CELL_SHAPES[0][0], tile_tm = CELL_SHAPES[0][1];
   int mtile_tn = 32, mtile_tm = 8, strip_rows = -1;   // per-point kernel on 32 x 8 tiles
   int xchunk = 64, xchunk_c = 0;
-  size_t nmt_cap = 0;            // capacity of blkmin (tiles of the largest tile count)
+  size_t nmt_cap = 0;            // capacity of blkkey (tiles of the largest tile count)
   size_t nct_cap = 0;            // continuity tiles of the largest tile count (cntstore)
   int in_batches = 0;            // user batches holding this scenario (tile shape is frozen)
   double* dvol = nullptr;
+  // step kernel: whether the handle may use it (step_rule), is meant to (not pinned to other
+  // shapes) and is using it now (on_step: the state lies on Scalars::side of the level arrays)
+  bool stepable = false, use_step = false, on_step = false;
   template <typename T> T* upload(const T* src, size_t n);
   template <typename T> T* alloc(size_t n);
 };
@@ -2022,6 +2464,11 @@ template <typename T> T* sfx_handle::upload(const T* src, size_t n) {
 // Momentum work lists of a batch, one per (kernel, mesh kind): [cell sg, cell reg, strip sg,
 // strip reg, idx sg, idx reg, point P=1 sg, reg, point P=2 sg, reg, point P=4 sg, reg].
 constexpr int NLIST_M = 12;
+// Runs in which the step kernel's tiles are dealt to the XCDs (16 to 128 measure within 1% on every
+// size; runs of 1 to 4 lose up to 12%, one band per XCD up to 25%: the wet tiles are clustered).
+constexpr int STEP_RUN = 32;
+// The step kernel as a momentum kernel number of sfx_get_tuning / sfx_set_tuning.
+constexpr int STEP_KERNEL = -8;
 
 // Momentum list of a scenario's kernel choice.
 inline int mom_list(const DevInst& I) {
@@ -2053,6 +2500,12 @@ struct sfx_batch {
   size_t off_m[NLIST_M] = {}, n_m[NLIST_M] = {};
   WorkList wl_m[NLIST_M] = {}, wl_cuv = {}, wl_cd = {}, wl_ci = {};   // launch arguments of the lists
   size_t off_cuv = 0, n_cuv = 0, off_cd = 0, n_cd = 0, off_ci = 0, n_ci = 0;
+  // step kernel lists (subgrid, regular), the scenarios in them (dIds + n_live onwards), and which
+  // scalar set the next launch reads
+  size_t off_s[2] = {}, n_s[2] = {};
+  WorkList wl_s[2] = {};
+  int n_step = 0, flip = 0;
+  std::vector<char> built_step;  // per member: in the step lists
   bool dirty = true;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -2176,9 +2629,15 @@ extern "C" int sfx_model_footprint(const sfx_model* M, size_t* bytes) {
   size_t b = np * (8 + 4 * 3 + 1) + nslot * (4 * 4 + 3);
   if (M->subgrid) b += np * (8 + 12 + 4 * (size_t)M->nl) + nslot * (4 + 16 + 4 + 16 * (size_t)M->nl);
   else b += np * 4 + nslot * 8;
+  if (M->dense) b += np * (8 + (M->subgrid ? 12 : 0)) + nslot;   // the step kernel's second side
   if (!M->dense) b += (size_t)M->npuv * (40 + 1) + np * 17 + (size_t)M->ncuv * 12;
   *bytes = b + (1 << 20);
   return SFX_OK;
+}
+
+namespace {
+bool step_rule(const DevInst& I, const sfx_model* M);
+void build_step(sfx_handle* H, const sfx_model* M, const std::vector<int32_t>& bf);
 }
 
 extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, sfx_handle** out);
@@ -2394,7 +2853,9 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
   s.dt = 1.0e-6f; s.min_dt = 1.0e-6f;   // sfincs_lib.f90:281-282
   s.itbndlast = 1; s.itsrclast = 1; s.itwndlast = 1; s.itprcplast = 1;
   s.twindupd = M->p.t0; s.mwin = -1; s.momtw = 1.0f; s.msm = 1.0f;   // sfincs_lib.f90:290
-  H->dS = H->upload(&s, 1);
+  I.sb = H->alloc<ScalarBlock>(1);
+  H->dS = (Scalars*)I.sb;
+  if (I.sb) (void)hipMemcpy(H->dS, &s, sizeof(s), hipMemcpyHostToDevice);
   I.sc = H->dS;
   // tiles
   I.tn = H->tile_tn; I.tm = H->tile_tm;
@@ -2407,6 +2868,7 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
   I.tn_sh = ilog2(I.tn); I.mtn_sh = ilog2(I.mtn);
   I.mrow_sh = ilog2(I.mtm * (I.sk < 0 ? -I.sk : 1));
   I.nmt = (int32_t)mom_tiles(I);
+  I.mmagic = div_magic(I.mntn, (size_t)I.nmt);
   H->nmt_cap = I.nmt;
   if (M->dense) {
     for (int k = 0; k < N_STRIP_ROWS; ++k) H->nmt_cap = std::max(H->nmt_cap, strip_tiles(I, STRIP_ROWS[k]));
@@ -2414,8 +2876,7 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
       H->nmt_cap = std::max(H->nmt_cap, 2 * cell_tiles(I, CELL_SHAPES[k][0], CELL_SHAPES[k][1]));
   }
   {
-    std::vector<float> init(H->nmt_cap, I.c.dtmax);
-    I.blkmin = H->upload(init.data(), init.size());
+    I.blkkey = H->alloc<uint32_t>(H->nmt_cap);
   }
   I.blkcnt = H->alloc<uint32_t>(NCNT * H->nmt_cap);
   I.mq = H->alloc<uint32_t>(H->nmt_cap);
@@ -2453,6 +2914,12 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
     I.bf_coef = H->upload(coef.data(), coef.size());
     I.rain_area = rain_area;
     I.bal = H->alloc<double>(NBAL);
+    for (int k = 0; k < 2; ++k) {
+      I.zs_s[k] = I.zs; I.vol_s[k] = I.vol; I.zsd_s[k] = (float*)I.zsderv; I.kf_s[k] = I.kfuv; I.um_s[k] = (float*)I.uvmean;
+    }
+    H->stepable = step_rule(I, M);
+    H->use_step = H->stepable;
+    if (H->stepable) build_step(H, M, slot);
   }
   H->dI = H->upload(&I, 1);
   for (void* p : H->allocs) if (!p) { set_error("hipMalloc failed"); return SFX_ERR_MEMORY; }
@@ -2461,6 +2928,87 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
   *out = H;
   return rc;
 }
+
+namespace {
+// Whether a scenario may take its steps in one launch each (k_step): a full rectangle in FP32
+// with the default physics, whose boundary is made of flux points only (no Neumann copies, no
+// weirs, no drainage structures), driven by uniform rain, discharges and external sources at
+// most. Everything else takes the separate kernels.
+bool step_rule(const DevInst& I, const sfx_model* M) {
+  return I.dense && !I.fp64 && sfx::std_physics(I.c) && I.n6 == 0 && I.ndrn == 0 && M->structure_uv_index.empty() &&
+         (size_t)M->mmax * (size_t)M->nmax < ((size_t)1 << 30);
+}
+
+// Rows of a step kernel tile. Its 4 waves compute 2 frows + 1 wave-rows of faces, one of them for
+// the neighbour's benefit, so few rows repeat more work; but the rows of a wave follow each other,
+// and a small mesh has waves to spare. The lines lie where the waves (4 np / (63 frows)) pass the
+// 8192 that the chip holds at once. Measured, us per step, regular / subgrid meshes (as separate
+// kernels about 16 / 17 at 64K cells, 19 / 22 at 256K, 62 / 60 at 1M, 93 / 98 at 3.1M / 4.2M):
+//    cells        frows 1        3            5            7
+//    64K         8.8 / 10.2  10.5 / 12.3  12.3 / 15.7  14.4 / 19.9
+//    130K / 176K 10.6 / 14.2 11.1 / 13.6  13.0 / 19.2  15.5 / 19.7
+//    256K / 358K 17.4 / 20.5 13.3 / 16.4  14.5 / 20.3  16.0 / 25.2
+//    1M          39.6 / 49   25.7 / 32.4  25.3 / 32.5  23.8 / 35.2
+//    3.1M / 4.2M  150 / 165  79.5 / 99.9  67.6 / 92.6  62.4 / 89.4
+int step_rows(size_t np) {
+  return np <= 150000 ? 1 : (np <= 750000 ? 3 : (np <= 2000000 ? 5 : 7));
+}
+
+// The step kernel's second side and per-tile tables. bf: the balance faces' slots.
+void build_step(sfx_handle* H, const sfx_model* M, const std::vector<int32_t>& bf) {
+  DevInst& I = H->hI;
+  const int nmax = I.nmax, mmax = I.mmax, np = I.np, fr = step_rows((size_t)np);
+  I.frows = fr;
+  I.fcols = nmax * ((mmax + fr - 1) / fr);
+  I.fnt = (I.fcols + STEP_COLS - 1) / STEP_COLS;
+  I.fmagic = div_magic(nmax, (size_t)I.fnt * STEP_COLS + WAVE);
+  auto tile_of = [&](int n, int m) { return ((m / fr) * nmax + n) / STEP_COLS; };
+  std::vector<uint8_t> flag(I.fnt, 0);
+  flag[0] |= FT_RUN;
+  for (int c = 0; c < np; ++c)
+    if (M->kcs[c] != 1) flag[tile_of(c % nmax, c / nmax)] |= FT_RUN;
+  for (int k = 0; k < M->nsrc; ++k) {
+    const int c = M->nmindsrc[k] - 1;
+    flag[tile_of(c % nmax, c / nmax)] |= FT_RUN;
+  }
+  // a tile reads the values of points up to two rows and columns from its cells (its own faces and
+  // the repeated ones, and their stencils), and sets the levels of its boundary cells
+  std::vector<std::vector<int32_t>> pts(I.fnt), faces(I.fnt);
+  for (int i = 0; i < M->nkcuv2; ++i) {
+    if (M->kcs[M->nmbkcuv2[i] - 1] == 6) continue;
+    const int s = H->ref2slot[M->index_kcuv2[i] - 1], c = s % np, n = c % nmax, m = c / nmax, own = tile_of(n, m);
+    for (int dm = -2; dm <= 2; ++dm)
+      for (int dn = -2; dn <= 2; ++dn) {
+        if (n + dn < 0 || n + dn >= nmax || m + dm < 0 || m + dm >= mmax) continue;
+        const int t = tile_of(n + dn, m + dm), ent = 2 * i + (t == own ? 1 : 0);
+        if (std::find(pts[t].rbegin(), pts[t].rend(), ent) == pts[t].rend()) pts[t].push_back(ent);
+      }
+  }
+  for (size_t f = 0; f < bf.size(); ++f) {
+    const int c = bf[f] % np;
+    faces[tile_of(c % nmax, c / nmax)].push_back((int32_t)f);
+  }
+  auto csr = [&](const std::vector<std::vector<int32_t>>& v, uint8_t bit, const int32_t*& ptr, const int32_t*& ent) {
+    std::vector<int32_t> p(1, 0), e;
+    for (int t = 0; t < I.fnt; ++t) {
+      e.insert(e.end(), v[t].begin(), v[t].end());
+      p.push_back((int32_t)e.size());
+      if (!v[t].empty()) flag[t] |= bit | FT_RUN;
+    }
+    ptr = H->upload(p.data(), p.size());
+    ent = H->upload(e.data(), e.size());
+  };
+  csr(pts, FT_BND, I.fb_ptr, I.fb_ent);
+  csr(faces, FT_BAL, I.ff_ptr, I.ff_ent);
+  I.fflag = H->upload(flag.data(), flag.size());
+  I.fquiet = H->alloc<uint8_t>((size_t)I.fnt * (BLOCK / WAVE));
+  I.fwake = H->alloc<uint8_t>((size_t)I.fnt * 2);
+  I.zs_s[1] = H->alloc<double>(np);
+  if (I.subgrid) { I.vol_s[1] = H->alloc<double>(np); I.zsd_s[1] = H->alloc<float>(np); }
+  I.kf_s[1] = H->alloc<int8_t>((size_t)H->nslot + 1);
+  I.um_s[1] = H->alloc<float>(M->uvmean.size());
+}
+}  // namespace
 
 extern "C" int sfx_batch_destroy(sfx_batch* b);
 
@@ -2495,6 +3043,16 @@ int write_scalars(sfx_handle* H, const Scalars& s) {
 // `cur` holds the latest q/uv and min_dt the sweep's minimum.
 int normalise(sfx_handle* H, Scalars& s) {
   int rc = read_scalars(H, s);
+  if (!rc && s.pend) {   // the step kernel's last sweep (its buffers have flipped already)
+    uint32_t key[NKEY * KEY_STRIDE], k = 0u;
+    HIPCHK(hipMemcpy(key, H->hI.sb->key[s.kset], sizeof(key), hipMemcpyDeviceToHost));
+    for (uint32_t v : key) k = std::max(k, v);
+    float den;
+    std::memcpy(&den, &k, 4);
+    s.min_dt = k ? std::fmin(H->hI.c.dtmax, 1.0f / den) : H->hI.c.dtmax;
+    s.pend = 0;
+    return SFX_OK;
+  }
   if (rc || !s.mom_done) return rc;
   hipLaunchKernelGGL(k_fold, dim3(1), dim3(FBLOCK), 0, H->stream, H->dI, (const int32_t*)nullptr);
   HIPCHK(hipGetLastError());
@@ -2576,7 +3134,7 @@ extern "C" int sfx_get_state(sfx_handle* H, const char* name, void* dst, size_t 
   const std::string k = name;
   const size_t np = H->hI.np;
   DevInst& I = H->hI;
-  if (k == "zs") { if (nbytes != np * 8) { set_error("size mismatch"); return SFX_ERR_ARG; } HIPCHK(hipMemcpy(dst, I.zs, nbytes, hipMemcpyDeviceToHost)); return SFX_OK; }
+  if (k == "zs") { if (nbytes != np * 8) { set_error("size mismatch"); return SFX_ERR_ARG; } HIPCHK(hipMemcpy(dst, I.zs_s[s.side], nbytes, hipMemcpyDeviceToHost)); return SFX_OK; }
   if (k == "zb") {
     if (!I.zb || nbytes != np * 4) { set_error("sfx_get_state: zb needs a regular (not subgrid) mesh and np f32 values"); return SFX_ERR_ARG; }
     HIPCHK(hipMemcpy(dst, I.zb, nbytes, hipMemcpyDeviceToHost));
@@ -2584,7 +3142,7 @@ extern "C" int sfx_get_state(sfx_handle* H, const char* name, void* dst, size_t 
   }
   if (k == "z_volume") {
     if (!I.vol || nbytes != np * 8) { set_error("no z_volume / size mismatch"); return SFX_ERR_ARG; }
-    HIPCHK(hipMemcpy(dst, I.vol, nbytes, hipMemcpyDeviceToHost)); return SFX_OK;
+    HIPCHK(hipMemcpy(dst, I.vol_s[s.side], nbytes, hipMemcpyDeviceToHost)); return SFX_OK;
   }
   if (k == "q" || k == "uv") {
     void* src = k == "q" ? I.q[s.cur] : I.uv[s.cur];
@@ -2594,12 +3152,12 @@ extern "C" int sfx_get_state(sfx_handle* H, const char* name, void* dst, size_t 
     const size_t n = H->sz.npuv;
     if (nbytes != n) { set_error("size mismatch"); return SFX_ERR_ARG; }
     std::vector<int8_t> b(H->nslot + 1);
-    HIPCHK(hipMemcpy(b.data(), I.kfuv, b.size(), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(b.data(), I.kf_s[s.side], b.size(), hipMemcpyDeviceToHost));
     for (size_t i = 0; i < n; ++i) ((int8_t*)dst)[i] = (int8_t)(b[H->ref2slot[i]] & 1);
     return SFX_OK;
   }
   if (k == "zs0" || k == "zsderv" || k == "zsmax") {
-    void* src = k == "zs0" ? I.zs0 : (k == "zsderv" ? I.zsderv : I.zsmax);
+    void* src = k == "zs0" ? I.zs0 : (k == "zsderv" ? (void*)I.zsd_s[s.side] : I.zsmax);
     return H->fp64 ? get_cell_r<double>(H, src, dst, nbytes, np) : get_cell_r<float>(H, src, dst, nbytes, np);
   }
   if (k == "tsa_sum" || k == "tsa_wet" || k == "tsa_lim") {   // timestep analysis, per uv-point
@@ -2618,7 +3176,7 @@ extern "C" int sfx_get_state(sfx_handle* H, const char* name, void* dst, size_t 
   }
   if (k == "uvmean") {
     const size_t n = H->sz.nkcuv2;
-    return H->fp64 ? get_cell_r<double>(H, I.uvmean, dst, nbytes, n) : get_cell_r<float>(H, I.uvmean, dst, nbytes, n);
+    return H->fp64 ? get_cell_r<double>(H, I.uvmean, dst, nbytes, n) : get_cell_r<float>(H, I.um_s[s.side], dst, nbytes, n);
   }
   if (k == "cumprcp" || k == "cuminf") {   // curve-number cumulative rain and infiltration, f32 per cell
     const float* src = k == "cumprcp" ? I.cumprcp : I.cuminf;
@@ -2636,15 +3194,22 @@ extern "C" int sfx_get_state(sfx_handle* H, const char* name, void* dst, size_t 
   return SFX_ERR_ARG;
 }
 
-namespace { int reset_tile_flags(sfx_handle* H); }
+namespace {
+int reset_tile_flags(sfx_handle* H);
+
+int clear_marks(sfx_handle* H, int uv) {
+  const int nb = std::min(4096, (H->hI.nslot + BLOCK - 1) / BLOCK);
+  hipLaunchKernelGGL(k_clear_marks, dim3(nb), dim3(BLOCK), 0, H->stream, H->dI, uv);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(H->stream));
+  return SFX_OK;
+}
+}  // namespace
 
 // A host write of cell state: no cell keeps its steady bit and no tile is quiescent.
 int clear_steady(sfx_handle* H) {
-  std::vector<uint8_t> b(H->hI.np);
-  HIPCHK(hipMemcpy(b.data(), H->hI.kcs, b.size(), hipMemcpyDeviceToHost));
-  for (auto& v : b) v = (uint8_t)(v & ~KCS_STEADY);
-  HIPCHK(hipMemcpy(H->hI.kcs, b.data(), b.size(), hipMemcpyHostToDevice));
-  return reset_tile_flags(H);
+  const int rc = clear_marks(H, 0);
+  return rc ? rc : reset_tile_flags(H);
 }
 
 extern "C" int sfx_set_state(sfx_handle* H, const char* name, const void* src, size_t nbytes) {
@@ -2658,12 +3223,12 @@ extern "C" int sfx_set_state(sfx_handle* H, const char* name, const void* src, s
   DevInst& I = H->hI;
   if (k == "zs") {
     if (nbytes != np * 8) { set_error("size mismatch"); return SFX_ERR_ARG; }
-    HIPCHK(hipMemcpy(I.zs, src, nbytes, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(I.zs_s[s.side], src, nbytes, hipMemcpyHostToDevice));
     return clear_steady(H);
   }
   if (k == "z_volume") {
     if (!I.vol || nbytes != np * 8) { set_error("no z_volume / size mismatch"); return SFX_ERR_ARG; }
-    HIPCHK(hipMemcpy(I.vol, src, nbytes, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(I.vol_s[s.side], src, nbytes, hipMemcpyHostToDevice));
     return clear_steady(H);
   }
   if (k == "zb") {   // bed level of a regular mesh, e.g. written by a coupler through the BMI
@@ -2676,23 +3241,21 @@ extern "C" int sfx_set_state(sfx_handle* H, const char* name, const void* src, s
     rc = H->fp64 ? set_uv_field<double>(H, dst, src, nbytes) : set_uv_field<float>(H, dst, src, nbytes);
     if (rc) return rc;
     // only the current buffer changed: the momentum kernels' zero flags no longer hold
-    std::vector<int8_t> b(H->nslot + 1);
-    HIPCHK(hipMemcpy(b.data(), I.kfuv, b.size(), hipMemcpyDeviceToHost));
-    for (auto& v : b) v = (int8_t)(v & 1);
-    HIPCHK(hipMemcpy(I.kfuv, b.data(), b.size(), hipMemcpyHostToDevice));
+    if ((rc = clear_marks(H, 1))) return rc;
     return reset_tile_flags(H);
   }
   if (k == "kfuv") {
     const size_t n = H->sz.npuv;
     if (nbytes != n) { set_error("size mismatch"); return SFX_ERR_ARG; }
     std::vector<int8_t> b(H->nslot + 1, 0);
-    HIPCHK(hipMemcpy(b.data(), I.kfuv, b.size(), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(b.data(), I.kf_s[s.side], b.size(), hipMemcpyDeviceToHost));
     for (size_t i = 0; i < n; ++i) b[H->ref2slot[i]] = ((const int8_t*)src)[i];
-    HIPCHK(hipMemcpy(I.kfuv, b.data(), b.size(), hipMemcpyHostToDevice));
+    for (int sd = 0; sd < (H->on_step ? 2 : 1); ++sd)   // points that no step writes keep it on both sides
+      HIPCHK(hipMemcpy(I.kf_s[sd], b.data(), b.size(), hipMemcpyHostToDevice));
     return reset_tile_flags(H);
   }
   if (k == "zs0" || k == "zsderv" || k == "zsmax") {
-    void* dst = k == "zs0" ? I.zs0 : (k == "zsderv" ? I.zsderv : I.zsmax);
+    void* dst = k == "zs0" ? I.zs0 : (k == "zsderv" ? (void*)I.zsd_s[s.side] : I.zsmax);
     rc = H->fp64 ? set_cell_r<double>(H, dst, src, nbytes, np) : set_cell_r<float>(H, dst, src, nbytes, np);
     if (rc) return rc;
     return clear_steady(H);
@@ -2787,9 +3350,10 @@ int rebuild(sfx_batch* B) {
   HIPCHK(hipSetDevice(B->device));
   const size_t nm = B->members.size();
   std::vector<DevInst> insts(nm);
-  std::vector<Item> mom[NLIST_M], cu, cd, ci;
-  std::vector<int32_t> ids;
+  std::vector<Item> mom[NLIST_M], cu, cd, ci, st[2];
+  std::vector<int32_t> ids, ids_step;
   int fp64 = -1;
+  B->built_step.assign(nm, 0);
   if (B->live.size() != nm) B->live.assign(nm, 1);
   for (size_t i = 0; i < nm; ++i) {
     sfx_handle* H = B->members[i];
@@ -2797,8 +3361,14 @@ int rebuild(sfx_batch* B) {
     if (fp64 < 0) fp64 = H->fp64;
     if (fp64 != H->fp64) { set_error("a batch cannot mix FP32 and FP64 members"); return SFX_ERR_ARG; }
     if (!B->live[i]) continue;
-    ids.push_back((int32_t)i);
     const DevInst& I = H->hI;
+    if (H->on_step) {
+      B->built_step[i] = 1;
+      ids_step.push_back((int32_t)i);
+      for (int t = 0; t < I.fnt; ++t) st[I.subgrid ? 0 : 1].push_back(Item{(int)i, t});
+      continue;
+    }
+    ids.push_back((int32_t)i);
     std::vector<Item>& mv = mom[mom_list(I)];
     const size_t tm = mom_tiles(I), tc = cont_tiles(I);
     for (size_t t = 0; t < tm; ++t) mv.push_back(Item{(int)i, (int)t});
@@ -2831,6 +3401,12 @@ int rebuild(sfx_batch* B) {
   if (cu.size()) { xcd_order(cu, 0); xcd_major(cu); }
   if (cd.size()) { xcd_order(cd, xchunk_c); xcd_major(cd); }
   if (ci.size()) { xcd_order(ci, xchunk_c); xcd_major(ci); }
+  Src src_s[2];
+  for (int k = 0; k < 2; ++k) {
+    src_s[k] = source(st[k], STEP_RUN);
+    if (st[k].size()) { xcd_order(st[k], STEP_RUN); xcd_major(st[k]); }
+    B->off_s[k] = all.size(); all.insert(all.end(), st[k].begin(), st[k].end()); B->n_s[k] = st[k].size();
+  }
   B->off_cuv = all.size(); all.insert(all.end(), cu.begin(), cu.end()); B->n_cuv = cu.size();
   B->off_cd = all.size(); all.insert(all.end(), cd.begin(), cd.end()); B->n_cd = cd.size();
   B->off_ci = all.size(); all.insert(all.end(), ci.begin(), ci.end()); B->n_ci = ci.size();
@@ -2851,8 +3427,10 @@ int rebuild(sfx_batch* B) {
   }
   if (nm) HIPCHK(hipMemcpy(B->dInsts, insts.data(), nm * sizeof(DevInst), hipMemcpyHostToDevice));
   if (all.size()) HIPCHK(hipMemcpy(B->dItems, all.data(), all.size() * sizeof(Item), hipMemcpyHostToDevice));
-  if (ids.size()) HIPCHK(hipMemcpy(B->dIds, ids.data(), ids.size() * sizeof(int32_t), hipMemcpyHostToDevice));
   B->n_live = (int)ids.size();
+  B->n_step = (int)ids_step.size();
+  ids.insert(ids.end(), ids_step.begin(), ids_step.end());   // the step kernel's scenarios follow the others
+  if (ids.size()) HIPCHK(hipMemcpy(B->dIds, ids.data(), ids.size() * sizeof(int32_t), hipMemcpyHostToDevice));
   auto wl = [&](size_t off, const Src& r) {
     WorkList w{};
     w.items = B->dItems + off;
@@ -2862,6 +3440,7 @@ int rebuild(sfx_batch* B) {
     return w;
   };
   for (int k = 0; k < NLIST_M; ++k) B->wl_m[k] = wl(B->off_m[k], src_m[k]);
+  for (int k = 0; k < 2; ++k) B->wl_s[k] = wl(B->off_s[k], src_s[k]);
   B->wl_cuv = wl(B->off_cuv, src_cu); B->wl_cd = wl(B->off_cd, src_cd); B->wl_ci = wl(B->off_ci, src_ci);
   if (B->exec) { hipGraphExecDestroy(B->exec); B->exec = nullptr; }
   if (B->graph) { hipGraphDestroy(B->graph); B->graph = nullptr; }
@@ -2885,10 +3464,10 @@ __global__ void __launch_bounds__(FBLOCK) k_tsa_min(const DevInst* __restrict__ 
                                                    const int32_t* __restrict__ ids) {
   const DevInst& I = insts[ids[blockIdx.x]];
   if (!(I.c.flags & sfx::F_TSA) || !G(I.sc)->mom_done) return;
-  float v = I.c.dtmax;
-  for (int i = threadIdx.x; i < I.nmt; i += FBLOCK) v = fminf(v, G(I.blkmin)[i]);
-  v = block_min<FBLOCK>(v);
-  if (threadIdx.x == 0) G(I.tsa_min)[0] = v;
+  uint32_t v = 0u;
+  for (int i = threadIdx.x; i < I.nmt; i += FBLOCK) v = max(v, G(I.blkkey)[i]);
+  v = block_max<FBLOCK>(v);
+  if (threadIdx.x == 0) G(I.tsa_min)[0] = key_step(v, I.fp64, I.c.dtmax);
 }
 
 __global__ void __launch_bounds__(BLOCK) k_tsa_update(const DevInst* __restrict__ insts,
@@ -2911,6 +3490,18 @@ template <typename R>
 void launch_phases(sfx_batch* B, int what, int forcing_mode) {
   hipStream_t st = B->stream;
   const int nm = B->n_live;
+  if (what == 7 && forcing_mode == 0 && B->n_step) {   // scenarios that step in one launch
+    size_t lds[2] = {0, 0};
+    for (sfx_handle* H : B->members)
+      if (H->on_step) {
+        size_t& b = lds[H->hI.subgrid ? 0 : 1];
+        b = std::max(b, (size_t)(2 * H->hI.frows + 1) * WAVE * sizeof(float));
+      }
+    if (B->n_s[0]) hipLaunchKernelGGL((k_step<true>), dim3(B->n_s[0]), dim3(BLOCK), lds[0], st, base_of(B, B->wl_s[0]), B->wl_s[0], B->flip);
+    if (B->n_s[1]) hipLaunchKernelGGL((k_step<false>), dim3(B->n_s[1]), dim3(BLOCK), lds[1], st, base_of(B, B->wl_s[1]), B->wl_s[1], B->flip);
+    B->flip ^= 1;
+  }
+  if (nm == 0) return;
   if ((what & 1) && nm) hipLaunchKernelGGL(k_forcing<R>, dim3(nm), dim3(FBLOCK), 0, st, B->dInsts, B->dIds, forcing_mode);
   if (what & 2) {
     if (B->n_m[0]) hipLaunchKernelGGL((k_mom_cell<R, true>), dim3(B->n_m[0]), dim3(BLOCK), 0, st, base_of(B, B->wl_m[0]), B->wl_m[0]);
@@ -2927,7 +3518,7 @@ void launch_phases(sfx_batch* B, int what, int forcing_mode) {
 #undef SFX_MOM_POINT
     if (B->n_cuv) hipLaunchKernelGGL(k_cuv<R>, dim3(B->n_cuv), dim3(BLOCK), 0, st, base_of(B, B->wl_cuv), B->wl_cuv);
     int tsa_slots = 0;   // timestep analysis of the members that have it on (not while tuning)
-    for (sfx_handle* H : B->members)
+    for (sfx_handle* H : B->members)   // (the step kernel's rule leaves members with it to these kernels)
       if (H->hI.tsa_req && !H->tsa_paused) tsa_slots = std::max(tsa_slots, (int)H->hI.nslot);
     if (tsa_slots && nm) {
       hipLaunchKernelGGL(k_tsa_min, dim3(nm), dim3(FBLOCK), 0, st, B->dInsts, B->dIds);
@@ -2961,6 +3552,12 @@ void launch(sfx_batch* B, int what, int mode) {
   else launch_phases<float>(B, what, mode);
 }
 
+// After a run of steps: the step kernel's scalars are in the first set again.
+void end_steps(sfx_batch* B) {
+  if (B->flip) hipLaunchKernelGGL(k_step_scalars, dim3(B->n_step), dim3(WAVE), 0, B->stream, B->dInsts, B->dIds + B->n_live);
+  B->flip = 0;
+}
+
 int ensure_graph(sfx_batch* B, int steps) {
   if (B->dirty) { int rc = rebuild(B); if (rc) return rc; }
   if (B->exec && B->graph_steps == steps) return SFX_OK;
@@ -2968,6 +3565,7 @@ int ensure_graph(sfx_batch* B, int steps) {
   if (B->graph) { hipGraphDestroy(B->graph); B->graph = nullptr; }
   HIPCHK(hipStreamBeginCapture(B->stream, hipStreamCaptureModeThreadLocal));
   for (int s = 0; s < steps; ++s) launch(B, 7, 0);
+  end_steps(B);
   HIPCHK(hipStreamEndCapture(B->stream, &B->graph));
   HIPCHK(hipGraphInstantiate(&B->exec, B->graph, nullptr, nullptr, 0));
   B->graph_steps = steps;
@@ -2987,14 +3585,48 @@ sfx_batch* solo(sfx_handle* H) {
   return H->solo;
 }
 
+// Moves a handle to the step kernel, or back to the separate ones. Both sides then hold what no
+// step writes, no tile is taken for quiet, and the separate kernels' marks are cleared.
+int enter_step(sfx_handle* H) {
+  if (!H->use_step || H->hI.count || H->on_step) return SFX_OK;
+  Scalars s;
+  int rc = normalise(H, s);
+  if (rc) return rc;
+  const DevInst& I = H->hI;
+  HIPCHK(hipMemcpyAsync(I.kf_s[1], I.kf_s[0], (size_t)H->nslot + 1, hipMemcpyDeviceToDevice, H->stream));
+  if (I.nkcuv2) HIPCHK(hipMemcpyAsync(I.um_s[1], I.um_s[0], (size_t)I.nkcuv2 * 4, hipMemcpyDeviceToDevice, H->stream));
+  HIPCHK(hipMemsetAsync(I.fwake, 0, (size_t)I.fnt * 2, H->stream));
+  HIPCHK(hipMemsetAsync(I.fquiet, 0, (size_t)I.fnt * (BLOCK / WAVE), H->stream));
+  HIPCHK(hipMemsetAsync(I.sb->key, 0, sizeof(I.sb->key), H->stream));
+  if ((rc = write_scalars(H, s)) || (rc = clear_marks(H, 1))) return rc;
+  H->on_step = true;
+  if (H->solo) H->solo->dirty = true;
+  return SFX_OK;
+}
+
+int enter_general(sfx_handle* H) {
+  if (!H->on_step) return SFX_OK;
+  Scalars s;
+  int rc = normalise(H, s);
+  if (rc) return rc;
+  const int nb = std::min(4096, (H->hI.nslot + BLOCK - 1) / BLOCK);
+  if (s.side) hipLaunchKernelGGL(k_step_settle, dim3(nb), dim3(BLOCK), 0, H->stream, H->dI);
+  HIPCHK(hipGetLastError());
+  s.side = 0;
+  if ((rc = write_scalars(H, s)) || (rc = clear_marks(H, 1))) return rc;
+  H->on_step = false;
+  if (H->solo) H->solo->dirty = true;
+  return reset_tile_flags(H);
+}
+
 }  // namespace
 
 extern "C" int sfx_compute_fluxes(sfx_handle* H, float dt, float* min_dt) {
   if (!H) { set_error("null"); return SFX_ERR_ARG; }
   HIPCHK(hipSetDevice(H->device));
   Scalars s;
-  int rc = normalise(H, s);
-  if (rc) return rc;
+  int rc = enter_general(H);
+  if (rc || (rc = normalise(H, s))) return rc;
   s.dt = dt; s.active = 1;
   if ((rc = write_scalars(H, s))) return rc;
   sfx_batch* B = solo(H);
@@ -3010,8 +3642,8 @@ extern "C" int sfx_compute_water_levels(sfx_handle* H, double t, float dt) {
   if (!H) { set_error("null"); return SFX_ERR_ARG; }
   HIPCHK(hipSetDevice(H->device));
   Scalars s;
-  int rc = read_scalars(H, s);
-  if (rc) return rc;
+  int rc = enter_general(H);
+  if (rc || (rc = read_scalars(H, s))) return rc;
   s.t = t; s.dt = dt; s.active = 1;
   if ((rc = write_scalars(H, s))) return rc;
   sfx_batch* B = solo(H);
@@ -3026,8 +3658,8 @@ extern "C" int sfx_update_forcing(sfx_handle* H, double t, float dt) {
   if (!H) { set_error("null"); return SFX_ERR_ARG; }
   HIPCHK(hipSetDevice(H->device));
   Scalars s;
-  int rc = normalise(H, s);
-  if (rc) return rc;
+  int rc = enter_general(H);
+  if (rc || (rc = normalise(H, s))) return rc;
   s.t = t; s.dt = dt;
   if ((rc = write_scalars(H, s))) return rc;
   sfx_batch* B = solo(H);
@@ -3045,8 +3677,8 @@ int update_loop(sfx_handle* H, int mode, double arg, sfx_step_stats* st) {
   HIPCHK(hipSetDevice(H->device));
   auto t_start = std::chrono::steady_clock::now();
   Scalars s;
-  int rc = read_scalars(H, s);
-  if (rc) return rc;
+  int rc = enter_step(H);
+  if (rc || (rc = H->on_step ? normalise(H, s) : read_scalars(H, s))) return rc;
   if (s.error_pending) { s.error = 1; s.error_pending = 0; s.t = (double)H->hI.c.t1 + 1.0; }
   const int64_t nt0 = s.nt;
   bool single = false;
@@ -3059,6 +3691,7 @@ int update_loop(sfx_handle* H, int mode, double arg, sfx_step_stats* st) {
   if (B->dirty && (rc = rebuild(B))) return rc;
   if (single) {
     launch(B, 7, 0);
+    end_steps(B);
     HIPCHK(hipGetLastError());
   } else {
     const int K = 32;
@@ -3093,6 +3726,10 @@ extern "C" int sfx_update_to(sfx_handle* H, double t_end, sfx_step_stats* st) {
 extern "C" int sfx_set_counting(sfx_handle* H, int32_t on) {
   if (!H) { set_error("null"); return SFX_ERR_ARG; }
   HIPCHK(hipSetDevice(H->device));
+  if (on) {   // the separate kernels count
+    const int rc = enter_general(H);
+    if (rc) return rc;
+  }
   H->hI.count = on ? 1 : 0;
   HIPCHK(hipStreamSynchronize(H->stream));
   HIPCHK(hipMemcpy(H->dI, &H->hI, sizeof(DevInst), hipMemcpyHostToDevice));
@@ -3190,11 +3827,12 @@ __global__ void __launch_bounds__(BLOCK) k_volume_partial(const DevInst* __restr
   const int c0 = blockIdx.x * VOL_CHUNK;
   const int c1 = std::min(I.np, c0 + VOL_CHUNK);
   double acc = 0.0;
+  const auto zs = G(I.zs_s[I.sc->side]), vol = G(I.vol_s[I.sc->side]);
   for (int c = c0 + (int)threadIdx.x; c < c1; c += BLOCK) {
     const int k = G(I.kcs)[c] & KCS_MASK;
     if (k == 0) continue;
     const int iref = I.dense ? 1 : G(I.z_iref)[c];
-    acc += I.subgrid ? G(I.vol)[c] : G(I.zs)[c] * (double)I.c.cell_area[iref - 1];
+    acc += I.subgrid ? vol[c] : zs[c] * (double)I.c.cell_area[iref - 1];
   }
   for (int o = WAVE / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, WAVE);
   __shared__ double red[BLOCK / WAVE];
@@ -3319,12 +3957,17 @@ extern "C" int sfx_batch_advance(sfx_batch* B, int32_t nsteps, int32_t* n_active
   HIPCHK(hipSetDevice(B->device));
   int rc;
   if (B->members.empty()) { if (n_active) *n_active = 0; return SFX_OK; }
+  for (size_t i = 0; i < B->members.size(); ++i) {
+    if ((rc = enter_step(B->members[i]))) return rc;
+    if (i >= B->built_step.size() || i >= B->live.size() || (B->live[i] && B->built_step[i] != (char)B->members[i]->on_step)) B->dirty = true;
+  }
   if (B->dirty && (rc = rebuild(B))) return rc;
-  if (B->n_live > 0) {
+  if (B->n_live + B->n_step > 0) {
     const int K = std::max(1, std::min(nsteps, 64));
     if ((rc = ensure_graph(B, K))) return rc;
     for (int r = 0; r < nsteps / K; ++r) HIPCHK(hipGraphLaunch(B->exec, B->stream));
     for (int r = 0; r < nsteps % K; ++r) launch(B, 7, 0);
+    end_steps(B);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(B->stream));
   }
@@ -3353,7 +3996,7 @@ extern "C" int sfx_batch_done(sfx_batch* B, sfx_handle* H, int32_t* done) {
 extern "C" int sfx_get_tuning(sfx_handle* H, int32_t out[8]) {
   if (!H || !out) { set_error("null"); return SFX_ERR_ARG; }
   const DevInst& I = H->hI;
-  out[0] = I.dense; out[1] = I.sk; out[2] = I.mtn; out[3] = I.mtm; out[4] = I.tn; out[5] = I.tm; out[6] = I.xchunk;
+  out[0] = I.dense; out[1] = H->use_step ? STEP_KERNEL : I.sk; out[2] = I.mtn; out[3] = I.mtm; out[4] = I.tn; out[5] = I.tm; out[6] = I.xchunk;
   out[7] = I.xchunk_c;
   return SFX_OK;
 }
@@ -3384,14 +4027,14 @@ int time_phases(sfx_handle* H, int what, int trials, hipEvent_t e0, hipEvent_t e
 // No per-point tile is quiescent (after host writes of state and tile-shape changes).
 int reset_tile_flags(sfx_handle* H) {
   HIPCHK(hipMemset(H->hI.mq, 0, H->nmt_cap * sizeof(uint32_t)));
+  if (H->stepable) HIPCHK(hipMemset(H->hI.fquiet, 0, (size_t)H->hI.fnt * (BLOCK / WAVE)));
   return SFX_OK;
 }
 
-// Tile minima back to dtmax (after sweeps that were not folded, e.g. timing runs), and no
-// tile quiescent.
-int reset_blkmin(sfx_handle* H) {
-  std::vector<float> init(H->nmt_cap, H->hI.c.dtmax);
-  HIPCHK(hipMemcpy(H->hI.blkmin, init.data(), init.size() * sizeof(float), hipMemcpyHostToDevice));
+// Tile keys back to 0 (after sweeps that were not folded, e.g. timing runs), and no tile
+// quiescent.
+int reset_keys(sfx_handle* H) {
+  HIPCHK(hipMemset(H->hI.blkkey, 0, H->nmt_cap * sizeof(uint32_t)));
   return reset_tile_flags(H);
 }
 
@@ -3403,12 +4046,14 @@ void set_shapes(sfx_handle* H, int sk, int mtn, int mtm, int tn, int tm) {
   I.tn_sh = ilog2(tn); I.mtn_sh = ilog2(mtn);
   I.mrow_sh = ilog2(mtm * (sk < 0 ? -sk : 1));
   I.nmt = (int32_t)mom_tiles(I);
+  I.mmagic = div_magic(I.mntn, (size_t)I.nmt);
 }
 }  // namespace
 
 extern "C" int sfx_set_tuning(sfx_handle* H, const int32_t in[5]) {
   if (!H || !in) { set_error("null"); return SFX_ERR_ARG; }
-  const int sk = in[0], mtn = in[1], mtm = in[2], tn = in[3], tm = in[4];
+  const bool step = in[0] == STEP_KERNEL && H->stepable;
+  const int sk = step ? H->hI.sk : in[0], mtn = in[1], mtm = in[2], tn = in[3], tm = in[4];
   const bool sk_ok = sk == -1 || sk == -2 || sk == -4 || (sk >= 0 && sk <= 256);
   if (!sk_ok || mtn <= 0 || mtm <= 0 || mtn * mtm != BLOCK || tn <= 0 || tm <= 0 || tn * tm != BLOCK) {
     set_error("sfx_set_tuning: the momentum kernel must be -1, -2, -4 (per-point), 0 (per-cell) or 1..256 strip rows, "
@@ -3419,8 +4064,8 @@ extern "C" int sfx_set_tuning(sfx_handle* H, const int32_t in[5]) {
   if (!H->hI.dense) return SFX_OK;
   HIPCHK(hipSetDevice(H->device));
   Scalars s;
-  int rc = normalise(H, s);
-  if (rc) return rc;
+  int rc = enter_general(H);
+  if (rc || (rc = normalise(H, s))) return rc;
   const DevInst keep = H->hI;
   set_shapes(H, sk, mtn, mtm, tn, tm);
   if (mom_tiles(H->hI) > H->nmt_cap) {
@@ -3430,7 +4075,8 @@ extern "C" int sfx_set_tuning(sfx_handle* H, const int32_t in[5]) {
   }
   HIPCHK(hipMemcpy(H->dI, &H->hI, sizeof(DevInst), hipMemcpyHostToDevice));
   H->tile_tn = tn; H->tile_tm = tm; H->strip_rows = sk; H->mtile_tn = mtn; H->mtile_tm = mtm;
-  if ((rc = reset_blkmin(H))) return rc;
+  H->use_step = step;
+  if ((rc = reset_keys(H))) return rc;
   if (H->solo) H->solo->dirty = true;
   return SFX_OK;
 }
@@ -3459,8 +4105,8 @@ extern "C" int sfx_autotune(sfx_handle* H, int32_t trials) {
   struct Pause { sfx_handle* h; ~Pause() { h->tsa_paused = false; } } pause{H};
   H->tsa_paused = true;   // timed sweeps are not steps of the run
   Scalars s0;
-  int rc = normalise(H, s0);
-  if (rc) return rc;
+  int rc = enter_general(H);
+  if (rc || (rc = normalise(H, s0))) return rc;
   // momentum and continuity write state: time on a snapshot and restore it afterwards
   std::vector<std::string> fields = {"zs", "q", "uv", "kfuv", "zs0", "zsderv", "zsmax"};
   if (H->hI.vol) fields.push_back("z_volume");
@@ -3482,7 +4128,10 @@ extern "C" int sfx_autotune(sfx_handle* H, int32_t trials) {
   HIPCHK(hipMemcpy(bal_keep, H->hI.bal, sizeof(bal_keep), hipMemcpyDeviceToHost));
   Scalars s = s0;
   s.active = 1; s.dt = std::max(s0.dt, 1.0e-3f);
+  s.tend = 1.0e30;
   if ((rc = write_scalars(H, s))) return rc;
+  std::vector<char> um((size_t)H->sz.nkcuv2 * (H->fp64 ? 8 : 4));   // whole steps are timed too
+  if (!um.empty()) HIPCHK(hipMemcpy(um.data(), H->hI.uvmean, um.size(), hipMemcpyDeviceToHost));
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
@@ -3536,6 +4185,18 @@ extern "C" int sfx_autotune(sfx_handle* H, int32_t trials) {
     if (!rc && ms < best) { best = ms; bxc = chunks[k]; }
   }
   H->hI.xchunk_c = bxc;
+  // the step kernel against the separate kernels, forcing included
+  if (H->stepable && !rc) {
+    float apart = 0.f, step = 0.f;
+    H->use_step = false;
+    rc = time_phases(H, 7, trials, e0, e1, apart);
+    H->use_step = true;
+    if (!rc) rc = enter_step(H);
+    if (!rc) rc = time_phases(H, 7, trials, e0, e1, step);
+    end_steps(solo(H));
+    if (!rc) rc = enter_general(H);
+    H->use_step = !rc && step <= apart;
+  }
   hipEventDestroy(e0);
   hipEventDestroy(e1);
   if (rc) return rc;
@@ -3543,10 +4204,11 @@ extern "C" int sfx_autotune(sfx_handle* H, int32_t trials) {
   H->tile_tn = H->hI.tn; H->tile_tm = H->hI.tm; H->strip_rows = H->hI.sk;
   H->mtile_tn = H->hI.mtn; H->mtile_tm = H->hI.mtm; H->xchunk = H->hI.xchunk; H->xchunk_c = H->hI.xchunk_c;
   if ((rc = write_scalars(H, s0))) return rc;
-  if ((rc = reset_blkmin(H))) return rc;
+  if ((rc = reset_keys(H))) return rc;
   for (auto& f : fields)
     if ((rc = sfx_set_state(H, f.c_str(), snap[f].data(), snap[f].size()))) return rc;
   HIPCHK(hipMemcpy(H->hI.bal, bal_keep, sizeof(bal_keep), hipMemcpyHostToDevice));
+  if (!um.empty()) HIPCHK(hipMemcpy(H->hI.uvmean, um.data(), um.size(), hipMemcpyHostToDevice));
   if (H->solo) H->solo->dirty = true;
   return SFX_OK;
 }
@@ -3558,11 +4220,12 @@ extern "C" int sfx_autotune(sfx_handle* H, int32_t trials) {
 extern "C" int sfx_profile_steps(sfx_handle* H, int32_t nsteps, double ms[3]) {
   if (!H || !ms || nsteps < 1) { set_error("sfx_profile_steps: bad args"); return SFX_ERR_ARG; }
   HIPCHK(hipSetDevice(H->device));
+  int rc = enter_step(H);
+  if (rc) return rc;
   sfx_batch* B = solo(H);
-  int rc;
   if (B->dirty && (rc = rebuild(B))) return rc;
   Scalars s;
-  if ((rc = read_scalars(H, s))) return rc;
+  if ((rc = H->on_step ? normalise(H, s) : read_scalars(H, s))) return rc;
   s.tend = 1.0e30;
   if ((rc = write_scalars(H, s))) return rc;
   hipEvent_t ev[4];
@@ -3570,11 +4233,11 @@ extern "C" int sfx_profile_steps(sfx_handle* H, int32_t nsteps, double ms[3]) {
   double acc[3] = {0, 0, 0};
   for (int i = 0; i < nsteps; ++i) {
     HIPCHK(hipEventRecord(ev[0], B->stream));
-    launch(B, 1, 0);
+    if (!H->on_step) launch(B, 1, 0);
     HIPCHK(hipEventRecord(ev[1], B->stream));
-    launch(B, 2, 0);
+    launch(B, H->on_step ? 7 : 2, 0);
     HIPCHK(hipEventRecord(ev[2], B->stream));
-    launch(B, 4, 0);
+    if (!H->on_step) launch(B, 4, 0);
     HIPCHK(hipEventRecord(ev[3], B->stream));
     HIPCHK(hipEventSynchronize(ev[3]));
     for (int k = 0; k < 3; ++k) {
@@ -3583,6 +4246,7 @@ extern "C" int sfx_profile_steps(sfx_handle* H, int32_t nsteps, double ms[3]) {
       acc[k] += t;
     }
   }
+  end_steps(B);
   for (auto& e : ev) hipEventDestroy(e);
   for (int k = 0; k < 3; ++k) ms[k] = acc[k] / nsteps;
   return SFX_OK;

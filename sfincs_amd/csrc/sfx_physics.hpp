@@ -46,6 +46,10 @@ struct GA {
   __device__ __forceinline__ GA operator+(uint32_t i) const {
     return GA{(gptr<T>)((gptr<char>)(gptr<void>)p + i * (uint32_t)sizeof(T))};
   }
+  // element i + k, k a small constant: the distance goes into the instruction's offset field
+  __device__ __forceinline__ __attribute__((address_space(1))) T& at(uint32_t i, int k) const {
+    return *((gptr<T>)((gptr<char>)(gptr<void>)p + i * (uint32_t)sizeof(T)) + k);
+  }
   __device__ __forceinline__ gptr<T> operator->() const { return p; }
 };
 template <typename T> __device__ __forceinline__ GA<T> ga(T* p) { return GA<T>{(gptr<T>)p}; }
@@ -164,12 +168,24 @@ __device__ __forceinline__ R power7over3(P x73, R hu) {
   return rpow<R>(R(10000.0f), R(7.0f / 3.0f));
 }
 
+// The physics switches of a default run that the STD instantiations of the updates take as
+// fixed: first-order upwind advection, two-dimensional friction, wiggle suppression on subgrid
+// meshes, the maximum level kept; no viscosity, Coriolis, theta smoothing, slope limit, h^(7/3)
+// table, wind, pressure or timestep analysis. std_physics() is the rule.
+constexpr uint32_t STD_ON = F_ADVECTION | F_UPW1 | F_FRICTION2D | F_NBRS | F_ZSMAX;
+constexpr uint32_t STD_OFF = F_VISCOSITY | F_CORIOLIS | F_THETA | F_H73 | F_WIND | F_TSA | F_MWIND | F_PATM | F_METEO3D |
+                             F_MPRCP | F_MSPIN | F_INFIL | F_CNA | F_STORE | F_STORAGE | F_QUADTREE;
+inline bool std_physics(const Consts& c) {
+  return (c.flags & STD_ON) == STD_ON && (c.flags & STD_OFF) == 0 && (!(c.flags & F_SUBGRID) || (c.flags & F_WIGGLE)) &&
+         !(c.slopelim < 9999.0f);
+}
+
 // One wet uv-point (sfincs_momentum.f90:189-742). `lev` points at the 2 levels
 // {havg,nrep,pwet,-} bracketing zsu for partially wet subgrid points.
-template <typename R, bool SUBGRID, typename LevP, typename X73P>
+template <typename R, bool SUBGRID, bool STD = false, typename LevP, typename X73P>
 __device__ __forceinline__ UvOut<R> uv_update(const UvIn<R>& in, const UvTables& tb, const Consts& c, R zsu,
                                               LevP lev_row, X73P x73, const PowTablesG& pw, R dt) {
-  const uint32_t F = c.flags;
+  const uint32_t F = STD ? STD_ON | (SUBGRID ? (uint32_t)F_WIGGLE : 0u) : c.flags;
   UvOut<R> o;
   const int iref = in.iref - 1;
   R dxuvinv, dxuv2inv, dyuv2inv;
@@ -209,21 +225,21 @@ __device__ __forceinline__ UvOut<R> uv_update(const UvIn<R>& in, const UvTables&
     hu = vmax<R>(zsu - (R)tb.zbuvmx, (R)c.huthresh);
     gnavg2 = tb.gn2uv;
   }
-  R dzdx;
-  if (c.slopelim < 9999.0f) {
-    double d = (in.zs_nmu - in.zs_nm) * (double)dxuvinv;
-    if (d < (double)(-c.slopelim)) d = (double)(-c.slopelim);
-    if (d > (double)c.slopelim) d = (double)c.slopelim;
-    dzdx = (R)d;
-  } else {
-    dzdx = (R)((in.zs_nmu - in.zs_nm) * (double)dxuvinv);
+  double slope = (in.zs_nmu - in.zs_nm) * (double)dxuvinv;
+  if (!STD && c.slopelim < 9999.0f) {
+    asm volatile("");   // off by default: a branch, not a select that every point pays for
+    if (slope < (double)(-c.slopelim)) slope = (double)(-c.slopelim);
+    if (slope > (double)c.slopelim) slope = (double)c.slopelim;
   }
+  const R dzdx = (R)slope;
   const R g = c.g;
   R frc = -(g * hu * dzdx);
+  // read with the rest of the stencil, not after the advection test (a round trip later)
+  R qy_nm = in.qy_nm, qy_nmu = in.qy_nmu, qy_ndm = in.qy_ndm, qy_ndmu = in.qy_ndmu;
+  asm volatile("" : "+v"(qy_nm), "+v"(qy_nmu), "+v"(qy_ndm), "+v"(qy_ndmu));
   if ((F & F_ADVECTION) && in.mask_adv == 1) {
     R dqxudx = R(0), dqyudy = R(0);
-    const R qx_nmd = in.qx_nmd, qx_nmu = in.qx_nmu, qy_nm = in.qy_nm, qy_nmu = in.qy_nmu;
-    const R qy_ndm = in.qy_ndm, qy_ndmu = in.qy_ndmu;
+    const R qx_nmd = in.qx_nmd, qx_nmu = in.qx_nmu;
     const R uu_nm = in.uu_nm, uu_nmd = in.uu_nmd, uu_nmu = in.uu_nmu, uu_ndm = in.uu_ndm, uu_num = in.uu_num;
     const R eps = R(1.0e-6f);
     if (F & F_UPW1) {
@@ -308,7 +324,7 @@ __device__ __forceinline__ UvOut<R> uv_update(const UvIn<R>& in, const UvTables&
 }
 
 // Cell update of the regular continuity (sfincs_continuity.f90:112-155, 239-255).
-template <typename R>
+template <typename R, bool STD = false>
 __device__ __forceinline__ void cell_regular(double& zs, R& zsmax, int kcs, R q_md, R q_mu, R q_nd, R q_nu,
                                              R netprcp, R qext, int iref, const Consts& c, R dt) {
   if (kcs == 1) {
@@ -317,18 +333,18 @@ __device__ __forceinline__ void cell_regular(double& zs, R& zsmax, int kcs, R q_
     const R d = ((q_md - q_mu) * (R)c.dxrinv[iref - 1] + (q_nd - q_nu) * (R)c.dyrinv[iref - 1]) * dt;
     zs = zs + (double)d;
   }
-  if (c.flags & F_ZSMAX) zsmax = (R)vmax<double>((double)zsmax, zs);
+  if (STD || (c.flags & F_ZSMAX)) zsmax = (R)vmax<double>((double)zsmax, zs);
 }
 
 // Cell update of the subgrid continuity (sfincs_continuity.f90:337-618).
-template <typename R, typename DepP>
+template <typename R, bool STD = false, typename DepP>
 __device__ __forceinline__ void cell_subgrid(double& zs, double& vol, R& zs0, R& zsderv, R& zsmax, int kcs,
                                              R q_md, R q_mu, R q_nd, R q_nu, R netprcp, R qext, R& stor, int iref,
                                              float zmin, float zmax, float volmax, DepP dep,
                                              const Consts& c, R dt) {
   R dvol = R(0);
   if (kcs == 1) {
-    if (c.flags & F_QUADTREE)
+    if (!STD && (c.flags & F_QUADTREE))
       dvol = dvol + ((q_md - q_mu) * (R)c.dyrm[iref - 1] + (q_nd - q_nu) * (R)c.dxrm[iref - 1]) * dt;
     else
       dvol = dvol + ((q_md - q_mu) * (R)c.dy + (q_nd - q_nu) * (R)c.dx) * dt;
@@ -341,14 +357,14 @@ __device__ __forceinline__ void cell_subgrid(double& zs, double& vol, R& zs0, R&
       if (c.flags & F_QEXT) dzsdt = dzsdt + qext;
       dvol = dvol + dzsdt * a * dt;
     }
-    if ((c.flags & F_STORAGE) && stor > R(1.0e-6f) && dvol > R(0)) {   // :499-523: storage fills first
+    if (!STD && (c.flags & F_STORAGE) && stor > R(1.0e-6f) && dvol > R(0)) {   // :499-523: storage fills first
       const R dv = stor - dvol;
       stor = vmax<R>(dv, R(0));
       dvol = dv < R(0) ? -dv : R(0);
     }
     vol = vol + (double)dvol;
     R zs00 = R(0), zs11 = R(0);
-    if (c.flags & F_WIGGLE) { zs00 = zs0; zs11 = (R)zs; zs0 = zs11; }
+    if (STD || (c.flags & F_WIGGLE)) { zs00 = zs0; zs11 = (R)zs; zs0 = zs11; }
     const float vmx = volmax;
     if (vol >= (double)(vmx * 0.999f)) {
       zs = (double)vmax<float>(zmax, -20.0f) + (vol - (double)vmx) / (double)a;
@@ -362,9 +378,9 @@ __device__ __forceinline__ void cell_subgrid(double& zs, double& vol, R& zs0, R&
       const R d0 = dep[iuv - 1], d1 = dep[iuv];
       zs = (double)(d0 + (d1 - d0) * facint);
     }
-    if (c.flags & F_WIGGLE) zsderv = (R)((zs - (double)(R(2) * zs11)) + (double)zs00);
+    if (STD || (c.flags & F_WIGGLE)) zsderv = (R)((zs - (double)(R(2) * zs11)) + (double)zs00);
   }
-  if (c.flags & F_ZSMAX) zsmax = (R)vmax<double>((double)zsmax, zs);
+  if (STD || (c.flags & F_ZSMAX)) zsmax = (R)vmax<double>((double)zsmax, zs);
 }
 
 }  // namespace sfx

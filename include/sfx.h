@@ -345,7 +345,8 @@ int  sfx_compute_water_levels(sfx_handle* h, double t, float dt);
  * boundary points/conditions/fluxes, discharges, at time t with step dt. */
 int  sfx_update_forcing(sfx_handle* h, double t, float dt);
 /* sfincs_update(dtrange) (sfincs_lib.f90:337-683): dtrange < -999 runs to t1, dtrange <= 0
- * one step, dtrange > 0 runs to t + dtrange. Device-resident loop, graph-captured. */
+ * one step, dtrange > 0 runs to t + dtrange. Device-resident loop: t and dt stay on the GPU, and
+ * the host launches as many steps as it expects to remain (steps past the end do nothing). */
 int  sfx_update(sfx_handle* h, double dtrange, sfx_step_stats* st);
 /* Steps while t < t_end (an absolute model time): the form a host uses to stop at the
  * first step whose time reaches an output time, as the reference's output triggers fire
@@ -417,12 +418,14 @@ int  sfx_create_ex(const sfx_model* m, int32_t device, int32_t fp64, sfx_handle*
  * lengths), the tile
  * shapes of the dense continuity kernel, and for both sweeps (dense or indexed) the runs
  * in which tiles are dealt to the XCDs, and keeps the fastest by the median of `trials`
- * timed launches per candidate. Call it before the handle joins a batch (SFX_ERR_STATE
+ * timed launches per candidate; then whole steps of those against the step kernel where the
+ * scenario may use it (dense FP32 meshes with the default physics). Call it before the handle joins a batch (SFX_ERR_STATE
  * otherwise). */
 int  sfx_autotune(sfx_handle* h, int32_t trials);
 /* out = {dense, momentum kernel (-1, -2, -4: per uv-point with 1, 2 or 4 points per
  *        thread, the points of a thread momentum-tile-m rows apart; 0: per cell; k > 0:
- *        strip march of k rows per wave), momentum tile n, momentum tile m, continuity tile n, continuity
+ *        strip march of k rows per wave; -8: the step kernel, which takes forcing,
+ *        momentum and continuity in one launch and ignores the tile shapes), momentum tile n, momentum tile m, continuity tile n, continuity
  *        tile m, momentum and continuity work-list runs per XCD (0: one contiguous band
  *        per XCD)} */
 int  sfx_get_tuning(sfx_handle* h, int32_t out[8]);

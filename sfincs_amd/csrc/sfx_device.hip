@@ -16,12 +16,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "sfx_internal.hpp"
@@ -397,12 +399,6 @@ __device__ void fold_sweep(const DevInst& I) {
   v = block_max<FBLOCK>(v);
   if (threadIdx.x == 0) { S->cur ^= 1; S->mom_done = 0; S->min_dt = key_step(v, I.fp64, I.c.dtmax); }
   __syncthreads();
-}
-
-__global__ void __launch_bounds__(FBLOCK) k_fold(const DevInst* __restrict__ insts, const int32_t* __restrict__ ids) {
-  const DevInst& I = insts[ids ? ids[blockIdx.x] : blockIdx.x];
-  fold_sweep(I);
-  if (threadIdx.x == 0) G(I.sc)->ahead = 0;   // a staged next step folded this sweep too
 }
 
 // Raises md of the per-point tiles (both planes) covering cells [nlo, nhi] x [mlo, mhi]
@@ -2312,6 +2308,55 @@ __global__ void __launch_bounds__(WAVE) k_step_scalars(const DevInst* __restrict
   copy_words(&I.sb->s[0], &I.sb->s[1]);
 }
 
+// Host write of a scenario's step scalars.
+__global__ void __launch_bounds__(WAVE) k_put_scalars(Scalars* dst, Scalars s) { copy_words(dst, &s); }
+
+// Hands the step scalars of some scenarios to the host: `out` is pinned host memory, one entry per
+// block. With flip they are first brought back to the first set; with fold a finished sweep is
+// completed (min_dt from its keys, the buffers of a separate sweep flipped).
+__global__ void __launch_bounds__(FBLOCK) k_give_scalars(const DevInst* __restrict__ insts, const int32_t* __restrict__ ids,
+                                                        int flip, int fold, Scalars* out) {
+  const DevInst& I = insts[ids ? ids[blockIdx.x] : blockIdx.x];
+  __shared__ Scalars n;
+  copy_words(&n, flip ? &I.sb->s[1] : &I.sb->s[0]);
+  __syncthreads();
+  if (fold && n.pend) {
+    if (threadIdx.x < WAVE) {
+      const uint32_t k = wave_max_last(G(I.sb->key[n.kset])[threadIdx.x * KEY_STRIDE]);
+      if (threadIdx.x == WAVE - 1) { n.min_dt = key_step(k, 0, I.c.dtmax); n.pend = 0; }
+    }
+    __syncthreads();
+  }
+  if (fold && n.mom_done) {
+    fold_sweep(I);
+    copy_words(&n, I.sc);
+    __syncthreads();
+    if (threadIdx.x == 0) n.ahead = 0;   // a staged next step folded this sweep too
+    __syncthreads();
+  }
+  if (flip || fold) copy_words(&I.sb->s[0], &n);
+  copy_words(&out[blockIdx.x], &n);
+}
+
+// q or uv of a full rectangle in reference order (per cell the point on its right, then the one
+// above; the dummy, zero, last): elements [from, from + n) to `out`.
+__global__ void __launch_bounds__(BLOCK) k_give_uv(const DevInst* __restrict__ I0, const float* src, uint32_t from, uint32_t n,
+                                                  float* out) {
+  const DevInst& I = *I0;
+  const uint32_t nmax = I.nmax, mmax = I.mmax, per = 2 * nmax - 1, last = (mmax - 1) * per;
+  for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) {
+    const uint32_t k = from + i;
+    uint32_t slot = (uint32_t)I.nslot;
+    if (k < last) {
+      const uint32_t m = k / per, r = k - m * per;
+      slot = m * nmax + (r >> 1) + ((r & 1u) ? (uint32_t)I.np : 0u);
+    } else if (k < (uint32_t)I.npuv) {
+      slot = (uint32_t)I.np + (mmax - 1) * nmax + (k - last);
+    }
+    out[i] = slot < (uint32_t)I.nslot ? G(src)[slot] : 0.f;
+  }
+}
+
 // The levels back to their first side (after an odd number of steps), for the kernels that work
 // on one side only.
 __global__ void __launch_bounds__(BLOCK) k_step_settle(const DevInst* __restrict__ I0) {
@@ -2442,6 +2487,11 @@ struct sfx_handle {
   // step kernel: whether the handle may use it (step_rule), is meant to (not pinned to other
   // shapes) and is using it now (on_step: the state lies on Scalars::side of the level arrays)
   bool stepable = false, use_step = false, on_step = false;
+  // The step scalars as they are on the device (hs_ok: every kernel that changes them is followed
+  // by k_give_scalars into `pin`, pinned host memory), so that calls need not fetch them first.
+  Scalars hs{};
+  bool hs_ok = false, staged = false;
+  Scalars* pin = nullptr;
   template <typename T> T* upload(const T* src, size_t n);
   template <typename T> T* alloc(size_t n);
 };
@@ -2506,6 +2556,9 @@ struct sfx_batch {
   WorkList wl_s[2] = {};
   int n_step = 0, flip = 0;
   std::vector<char> built_step;  // per member: in the step lists
+  std::vector<int32_t> ids;      // dIds on the host
+  Scalars* pin = nullptr;        // pinned host memory for the members' scalars
+  size_t pin_cap = 0;
   bool dirty = true;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -2636,6 +2689,8 @@ extern "C" int sfx_model_footprint(const sfx_model* M, size_t* bytes) {
 }
 
 namespace {
+void stage_open(sfx_handle* H);
+void stage_close(sfx_handle* H);
 bool step_rule(const DevInst& I, const sfx_model* M);
 void build_step(sfx_handle* H, const sfx_model* M, const std::vector<int32_t>& bf);
 }
@@ -2922,7 +2977,12 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
     if (H->stepable) build_step(H, M, slot);
   }
   H->dI = H->upload(&I, 1);
+  if (hipHostMalloc((void**)&H->pin, sizeof(Scalars)) != hipSuccess) H->pin = nullptr;
+  stage_open(H);
+  H->hs = s; H->hs_ok = true;
+  H->allocs.push_back(H->pin);   // checked with the rest, freed apart
   for (void* p : H->allocs) if (!p) { set_error("hipMalloc failed"); return SFX_ERR_MEMORY; }
+  H->allocs.pop_back();
   HIPCHK(hipDeviceSynchronize());
   HIPCHK(hipStreamCreateWithFlags(&H->stream, hipStreamNonBlocking));
   *out = H;
@@ -3018,6 +3078,8 @@ extern "C" int sfx_destroy(sfx_handle* H) {
   if (H->solo) { sfx_batch_destroy(H->solo); H->solo = nullptr; }
   hipDeviceSynchronize();
   for (void* p : H->allocs) hipFree(p);
+  if (H->pin) hipHostFree(H->pin);
+  stage_close(H);
   if (H->stream) hipStreamDestroy(H->stream);
   delete H;
   return SFX_OK;
@@ -3026,37 +3088,170 @@ extern "C" int sfx_destroy(sfx_handle* H) {
 // -------------------------------------------------------------------------- state exchange
 namespace {
 
+// Pinned host memory through which state passes to and from the device, one set per GPU: NSTAGE
+// buffers of STAGE bytes, allocated with the first copy and given back with the GPU's last handle.
+// A copy to pageable memory takes 17 us for 24 KB, 120 us for 256 KB and 1.95 ms for 33 MB (its
+// staging is serial and waits per piece); through these buffers 9, 25 and 0.9 ms: the pieces follow
+// each other on the copy engine (55 GB/s) while up to four threads move the last one on.
+constexpr size_t STAGE = (size_t)2 << 20;
+constexpr int NSTAGE = 4, STAGE_THREADS = 4;
+constexpr size_t STAGE_PAR = (size_t)6 << 20;   // from here on helper threads pay for their start (50 us)
+struct Stage {
+  std::mutex mu;
+  int refs = 0;
+  char* buf = nullptr;
+  hipEvent_t ev[NSTAGE] = {};
+};
+Stage g_stage[64];
+
+void stage_open(sfx_handle* H) {
+  if (H->device >= 64 || H->staged) return;
+  std::lock_guard<std::mutex> lk(g_stage[H->device].mu);
+  ++g_stage[H->device].refs;
+  H->staged = true;
+}
+void stage_close(sfx_handle* H) {
+  if (!H->staged) return;
+  Stage& S = g_stage[H->device];
+  std::lock_guard<std::mutex> lk(S.mu);
+  if (--S.refs > 0 || !S.buf) return;
+  for (auto& e : S.ev) { hipEventDestroy(e); e = nullptr; }
+  hipHostFree(S.buf);
+  S.buf = nullptr;
+}
+// With S.mu held: its buffers, or null when they cannot be had (the caller copies directly).
+char* stage_buf(Stage& S) {
+  if (S.buf) return S.buf;
+  char* b = nullptr;
+  if (hipHostMalloc((void**)&b, NSTAGE * STAGE) != hipSuccess) return nullptr;
+  for (int k = 0; k < NSTAGE; ++k)
+    if (hipEventCreateWithFlags(&S.ev[k], hipEventDisableTiming) != hipSuccess) {
+      while (k-- > 0) { hipEventDestroy(S.ev[k]); S.ev[k] = nullptr; }
+      hipHostFree(b);
+      return nullptr;
+    }
+  return S.buf = b;
+}
+
+// n bytes to the host, made piece by piece: put(buf, from, bytes) enqueues the bytes [from, from +
+// bytes) into pinned memory on the handle's stream. Returns 1 when there is no pinned memory.
+template <typename Put>
+int staged_out(sfx_handle* H, void* dst, size_t n, Put put) {
+  if (!H->staged) return 1;
+  Stage& S = g_stage[H->device];
+  std::lock_guard<std::mutex> lk(S.mu);
+  char* buf = stage_buf(S);
+  if (!buf) return 1;
+  if (n <= STAGE) {
+    HIPCHK(put(buf, (size_t)0, n));
+    HIPCHK(hipStreamSynchronize(H->stream));
+    std::memcpy(dst, buf, n);
+    return SFX_OK;
+  }
+  const size_t pieces = (n + STAGE - 1) / STAGE;
+  const int T = n >= STAGE_PAR ? STAGE_THREADS : 1;
+  std::atomic<size_t> ready{0}, done{0};
+  std::atomic<bool> stop{false};
+  auto move = [&](int t, size_t k) {   // thread t's share of piece k
+    const size_t len = std::min(STAGE, n - k * STAGE), lo = len * t / T, hi = len * (t + 1) / T;
+    std::memcpy((char*)dst + k * STAGE + lo, buf + (k % NSTAGE) * STAGE + lo, hi - lo);
+    done.fetch_add(1, std::memory_order_release);
+  };
+  std::vector<std::thread> help;
+  for (int t = 1; t < T; ++t)
+    help.emplace_back([&, t] {
+      for (size_t k = 0; k < pieces; ++k) {
+        while (ready.load(std::memory_order_acquire) <= k) {
+          if (stop.load()) return;
+          std::this_thread::yield();
+        }
+        move(t, k);
+      }
+    });
+  hipError_t e = hipSuccess;
+  size_t issued = 0;
+  for (size_t k = 0; k < pieces && e == hipSuccess; ++k) {
+    for (; issued < std::min(pieces, k + NSTAGE) && e == hipSuccess; ++issued) {
+      e = put(buf + (issued % NSTAGE) * STAGE, issued * STAGE, std::min(STAGE, n - issued * STAGE));
+      if (e == hipSuccess) e = hipEventRecord(S.ev[issued % NSTAGE], H->stream);
+    }
+    if (e == hipSuccess) e = hipEventSynchronize(S.ev[k % NSTAGE]);
+    if (e != hipSuccess) break;
+    ready.store(k + 1, std::memory_order_release);
+    move(0, k);
+    while (done.load(std::memory_order_acquire) < (size_t)T * (k + 1)) std::this_thread::yield();
+  }
+  stop.store(true);
+  for (auto& t : help) t.join();
+  HIPCHK(e);
+  return SFX_OK;
+}
+
+// Device memory of a handle to the host and back; the handle's stream is idle when they return.
+int to_host(sfx_handle* H, void* dst, const void* src, size_t n) {
+  if (!n) return SFX_OK;
+  const int rc = staged_out(H, dst, n, [&](char* to, size_t from, size_t len) {
+    return hipMemcpyAsync(to, (const char*)src + from, len, hipMemcpyDeviceToHost, H->stream);
+  });
+  if (rc <= 0) return rc;
+  HIPCHK(hipStreamSynchronize(H->stream));
+  HIPCHK(hipMemcpy(dst, src, n, hipMemcpyDeviceToHost));
+  return SFX_OK;
+}
+int to_device(sfx_handle* H, void* dst, const void* src, size_t n) {
+  if (!n) return SFX_OK;
+  if (H->staged && n <= STAGE) {
+    Stage& S = g_stage[H->device];
+    std::lock_guard<std::mutex> lk(S.mu);
+    if (char* buf = stage_buf(S)) {
+      std::memcpy(buf, src, n);
+      HIPCHK(hipMemcpyAsync(dst, buf, n, hipMemcpyHostToDevice, H->stream));
+      HIPCHK(hipStreamSynchronize(H->stream));
+      return SFX_OK;
+    }
+  }
+  HIPCHK(hipStreamSynchronize(H->stream));
+  HIPCHK(hipMemcpy(dst, src, n, hipMemcpyHostToDevice));
+  return SFX_OK;
+}
+
+// The step scalars (after a flip of the step kernel's sets; with fold, after the last sweep).
+int fetch_scalars(sfx_handle* H, int flip, int fold) {
+  H->hs_ok = false;
+  hipLaunchKernelGGL(k_give_scalars, dim3(1), dim3(FBLOCK), 0, H->stream, H->dI, (const int32_t*)nullptr, flip, fold, H->pin);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(H->stream));
+  H->hs = *H->pin;
+  H->hs_ok = true;
+  return SFX_OK;
+}
 int read_scalars(sfx_handle* H, Scalars& s) {
   HIPCHK(hipStreamSynchronize(H->stream));
-  HIPCHK(hipMemcpy(&s, H->dS, sizeof(Scalars), hipMemcpyDeviceToHost));
+  if (!H->hs_ok) {
+    const int rc = fetch_scalars(H, 0, 0);
+    if (rc) return rc;
+  }
+  s = H->hs;
   return SFX_OK;
 }
-// Host write of the step scalars; it also drops a next step computed ahead on the old ones.
+// Host write of the step scalars, in order on the handle's stream; it also drops a next step
+// computed ahead on the old ones.
 int write_scalars(sfx_handle* H, const Scalars& s) {
-  HIPCHK(hipStreamSynchronize(H->stream));
-  Scalars w = s;
-  w.ahead = 0;
-  HIPCHK(hipMemcpy(H->dS, &w, sizeof(Scalars), hipMemcpyHostToDevice));
+  H->hs = s;
+  H->hs.ahead = 0;
+  hipLaunchKernelGGL(k_put_scalars, dim3(1), dim3(WAVE), 0, H->stream, H->dS, H->hs);
+  HIPCHK(hipGetLastError());
+  H->hs_ok = true;
   return SFX_OK;
 }
-// Completes a pending momentum sweep (fold of the tile minima, buffer flip) so that
+// Completes a pending momentum sweep (fold of the tile keys, buffer flip) so that
 // `cur` holds the latest q/uv and min_dt the sweep's minimum.
 int normalise(sfx_handle* H, Scalars& s) {
   int rc = read_scalars(H, s);
-  if (!rc && s.pend) {   // the step kernel's last sweep (its buffers have flipped already)
-    uint32_t key[NKEY * KEY_STRIDE], k = 0u;
-    HIPCHK(hipMemcpy(key, H->hI.sb->key[s.kset], sizeof(key), hipMemcpyDeviceToHost));
-    for (uint32_t v : key) k = std::max(k, v);
-    float den;
-    std::memcpy(&den, &k, 4);
-    s.min_dt = k ? std::fmin(H->hI.c.dtmax, 1.0f / den) : H->hI.c.dtmax;
-    s.pend = 0;
-    return SFX_OK;
-  }
-  if (rc || !s.mom_done) return rc;
-  hipLaunchKernelGGL(k_fold, dim3(1), dim3(FBLOCK), 0, H->stream, H->dI, (const int32_t*)nullptr);
-  HIPCHK(hipGetLastError());
-  return read_scalars(H, s);
+  if (rc || !(s.mom_done || s.pend)) return rc;
+  if ((rc = fetch_scalars(H, 0, 1))) return rc;
+  s = H->hs;
+  return SFX_OK;
 }
 
 // 4-byte per-slot words (f32 or i32) of the npuv uv-points, in reference order.
@@ -3073,8 +3268,18 @@ int get_uv_words(sfx_handle* H, const void* src, void* dst, size_t nbytes) {
 template <typename R>
 int get_uv_field(sfx_handle* H, void* src, void* dst, size_t nbytes, bool is_q) {
   (void)is_q;
+  static_assert(STAGE % 16 == 0, "pieces hold whole values");
   const size_t n = H->ref2slot.size();
   if (nbytes != n * sizeof(R) && nbytes != n * sizeof(float)) { set_error("size mismatch"); return SFX_ERR_ARG; }
+  if (sizeof(R) == sizeof(float) && !H->hI.dense) return to_host(H, dst, src, nbytes);   // slots are in reference order
+  if (sizeof(R) == sizeof(float)) {
+    const int rc = staged_out(H, dst, nbytes, [&](char* to, size_t from, size_t len) {
+      const uint32_t k = (uint32_t)(len / 4), nb = std::min(2048u, (k + BLOCK - 1) / BLOCK);
+      hipLaunchKernelGGL(k_give_uv, dim3(nb), dim3(BLOCK), 0, H->stream, H->dI, (const float*)src, (uint32_t)(from / 4), k, (float*)to);
+      return hipGetLastError();
+    });
+    if (rc <= 0) return rc;
+  }
   std::vector<R> buf(H->nslot + 1);
   HIPCHK(hipMemcpy(buf.data(), src, buf.size() * sizeof(R), hipMemcpyDeviceToHost));
   if (nbytes == n * sizeof(R)) {
@@ -3104,7 +3309,7 @@ int set_uv_field(sfx_handle* H, void* dst, const void* src, size_t nbytes) {
 
 template <typename R>
 int get_cell_r(sfx_handle* H, const void* src, void* dst, size_t nbytes, size_t n) {
-  if (nbytes == n * sizeof(R)) { HIPCHK(hipMemcpy(dst, src, nbytes, hipMemcpyDeviceToHost)); return SFX_OK; }
+  if (nbytes == n * sizeof(R)) return to_host(H, dst, src, nbytes);
   if (nbytes != n * sizeof(float)) { set_error("size mismatch"); return SFX_ERR_ARG; }
   std::vector<R> b(n);
   HIPCHK(hipMemcpy(b.data(), src, n * sizeof(R), hipMemcpyDeviceToHost));
@@ -3114,8 +3319,7 @@ int get_cell_r(sfx_handle* H, const void* src, void* dst, size_t nbytes, size_t 
 
 template <typename R>
 int set_cell_r(sfx_handle* H, void* dst, const void* src, size_t nbytes, size_t n) {
-  (void)H;
-  if (nbytes == n * sizeof(R)) { HIPCHK(hipMemcpy(dst, src, nbytes, hipMemcpyHostToDevice)); return SFX_OK; }
+  if (nbytes == n * sizeof(R)) return to_device(H, dst, src, nbytes);
   if (nbytes != n * sizeof(float)) { set_error("size mismatch"); return SFX_ERR_ARG; }
   std::vector<R> b(n);
   for (size_t i = 0; i < n; ++i) b[i] = (R)((const float*)src)[i];
@@ -3134,15 +3338,14 @@ extern "C" int sfx_get_state(sfx_handle* H, const char* name, void* dst, size_t 
   const std::string k = name;
   const size_t np = H->hI.np;
   DevInst& I = H->hI;
-  if (k == "zs") { if (nbytes != np * 8) { set_error("size mismatch"); return SFX_ERR_ARG; } HIPCHK(hipMemcpy(dst, I.zs_s[s.side], nbytes, hipMemcpyDeviceToHost)); return SFX_OK; }
+  if (k == "zs") { if (nbytes != np * 8) { set_error("size mismatch"); return SFX_ERR_ARG; } return to_host(H, dst, I.zs_s[s.side], nbytes); }
   if (k == "zb") {
     if (!I.zb || nbytes != np * 4) { set_error("sfx_get_state: zb needs a regular (not subgrid) mesh and np f32 values"); return SFX_ERR_ARG; }
-    HIPCHK(hipMemcpy(dst, I.zb, nbytes, hipMemcpyDeviceToHost));
-    return SFX_OK;
+    return to_host(H, dst, I.zb, nbytes);
   }
   if (k == "z_volume") {
     if (!I.vol || nbytes != np * 8) { set_error("no z_volume / size mismatch"); return SFX_ERR_ARG; }
-    HIPCHK(hipMemcpy(dst, I.vol_s[s.side], nbytes, hipMemcpyDeviceToHost)); return SFX_OK;
+    return to_host(H, dst, I.vol_s[s.side], nbytes);
   }
   if (k == "q" || k == "uv") {
     void* src = k == "q" ? I.q[s.cur] : I.uv[s.cur];
@@ -3181,14 +3384,12 @@ extern "C" int sfx_get_state(sfx_handle* H, const char* name, void* dst, size_t 
   if (k == "cumprcp" || k == "cuminf") {   // curve-number cumulative rain and infiltration, f32 per cell
     const float* src = k == "cumprcp" ? I.cumprcp : I.cuminf;
     if (!src || nbytes != (size_t)np * 4) { set_error("sfx_get_state: " + k + " needs curve-number infiltration and np f32"); return SFX_ERR_ARG; }
-    HIPCHK(hipMemcpy(dst, src, nbytes, hipMemcpyDeviceToHost));
-    return SFX_OK;
+    return to_host(H, dst, src, nbytes);
   }
   if (k == "qtsrc") {   // the step's discharges: point sources, then each drainage intake and outfall
     const size_t n = (size_t)I.nsrc + 2 * (size_t)I.ndrn;
     if (n == 0 || nbytes != n * 4) { set_error("sfx_get_state: qtsrc needs (nsrc + 2 ndrn) f32 values"); return SFX_ERR_ARG; }
-    HIPCHK(hipMemcpy(dst, I.qtsrc, nbytes, hipMemcpyDeviceToHost));
-    return SFX_OK;
+    return to_host(H, dst, I.qtsrc, nbytes);
   }
   set_error("unknown state field " + k);
   return SFX_ERR_ARG;
@@ -3223,17 +3424,17 @@ extern "C" int sfx_set_state(sfx_handle* H, const char* name, const void* src, s
   DevInst& I = H->hI;
   if (k == "zs") {
     if (nbytes != np * 8) { set_error("size mismatch"); return SFX_ERR_ARG; }
-    HIPCHK(hipMemcpy(I.zs_s[s.side], src, nbytes, hipMemcpyHostToDevice));
+    if ((rc = to_device(H, I.zs_s[s.side], src, nbytes))) return rc;
     return clear_steady(H);
   }
   if (k == "z_volume") {
     if (!I.vol || nbytes != np * 8) { set_error("no z_volume / size mismatch"); return SFX_ERR_ARG; }
-    HIPCHK(hipMemcpy(I.vol_s[s.side], src, nbytes, hipMemcpyHostToDevice));
+    if ((rc = to_device(H, I.vol_s[s.side], src, nbytes))) return rc;
     return clear_steady(H);
   }
   if (k == "zb") {   // bed level of a regular mesh, e.g. written by a coupler through the BMI
     if (!I.zb || nbytes != np * 4) { set_error("sfx_set_state: zb needs a regular (not subgrid) mesh and np f32 values"); return SFX_ERR_ARG; }
-    HIPCHK(hipMemcpy((void*)I.zb, src, nbytes, hipMemcpyHostToDevice));
+    if ((rc = to_device(H, (void*)I.zb, src, nbytes))) return rc;
     return clear_steady(H);
   }
   if (k == "q" || k == "uv") {
@@ -3268,8 +3469,7 @@ extern "C" int sfx_set_state(sfx_handle* H, const char* name, const void* src, s
   }
   if (k == "qext") {   // external sources (m/s per cell), e.g. from a coupled model through the BMI
     if (!I.qext || nbytes != np * 4) { set_error("sfx_set_state: qext needs use_qext and np f32 values"); return SFX_ERR_ARG; }
-    HIPCHK(hipMemcpy(I.qext, src, nbytes, hipMemcpyHostToDevice));
-    return SFX_OK;
+    return to_device(H, I.qext, src, nbytes);
   }
   if (k == "vmax" || k == "qmax" || k == "twet") {   // e.g. the reset after each maximum output
     void* dst = k == "vmax" ? I.vmax : (k == "qmax" ? I.qmax : I.twet);
@@ -3431,6 +3631,15 @@ int rebuild(sfx_batch* B) {
   B->n_step = (int)ids_step.size();
   ids.insert(ids.end(), ids_step.begin(), ids_step.end());   // the step kernel's scenarios follow the others
   if (ids.size()) HIPCHK(hipMemcpy(B->dIds, ids.data(), ids.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+  B->ids = ids;
+  if (B->pin_cap < nm) {
+    if (B->pin) hipHostFree(B->pin);
+    B->pin = nullptr;
+    B->pin_cap = 0;
+    const size_t cap = std::max<size_t>(nm, 8);
+    HIPCHK(hipHostMalloc((void**)&B->pin, cap * sizeof(Scalars)));
+    B->pin_cap = cap;
+  }
   auto wl = [&](size_t off, const Src& r) {
     WorkList w{};
     w.items = B->dItems + off;
@@ -3558,6 +3767,8 @@ void end_steps(sfx_batch* B) {
   B->flip = 0;
 }
 
+constexpr int GRAPH_STEPS = 32;   // steps per graph of a single scenario
+
 int ensure_graph(sfx_batch* B, int steps) {
   if (B->dirty) { int rc = rebuild(B); if (rc) return rc; }
   if (B->exec && B->graph_steps == steps) return SFX_OK;
@@ -3599,6 +3810,7 @@ int enter_step(sfx_handle* H) {
   HIPCHK(hipMemsetAsync(I.fquiet, 0, (size_t)I.fnt * (BLOCK / WAVE), H->stream));
   HIPCHK(hipMemsetAsync(I.sb->key, 0, sizeof(I.sb->key), H->stream));
   if ((rc = write_scalars(H, s)) || (rc = clear_marks(H, 1))) return rc;
+  HIPCHK(hipStreamSynchronize(H->stream));   // a batch runs on its own stream
   H->on_step = true;
   if (H->solo) H->solo->dirty = true;
   return SFX_OK;
@@ -3632,9 +3844,8 @@ extern "C" int sfx_compute_fluxes(sfx_handle* H, float dt, float* min_dt) {
   sfx_batch* B = solo(H);
   if (B->dirty && (rc = rebuild(B))) return rc;
   launch(B, 2, 0);
-  HIPCHK(hipGetLastError());
-  if ((rc = normalise(H, s))) return rc;
-  if (min_dt) *min_dt = s.min_dt;
+  if ((rc = fetch_scalars(H, 0, 1))) return rc;
+  if (min_dt) *min_dt = H->hs.min_dt;
   return SFX_OK;
 }
 
@@ -3665,20 +3876,28 @@ extern "C" int sfx_update_forcing(sfx_handle* H, double t, float dt) {
   sfx_batch* B = solo(H);
   if (B->dirty && (rc = rebuild(B))) return rc;
   launch(B, 1, 1);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(H->stream));
-  return SFX_OK;
+  return fetch_scalars(H, 0, 0);
 }
 
 namespace {
+// About how many steps are left to tend at the next step's size, and a little more (steps past
+// tend do nothing); a run's first steps are tiny, so they are taken two at a time.
+int steps_left(const sfx_handle* H, const Scalars& s) {
+  const double dt = (double)H->hI.c.alpha * (double)s.min_dt, n = (s.tend - s.t) / dt + 2.0;
+  if (s.nt < 2) return 2;
+  return n < 512.0 ? std::max(1, (int)n) : 512;
+}
+
 // The step loop of sfincs_update (sfincs_lib.f90:379-648): one step (single), or steps
-// while t < tend, in graph launches of 32 steps whose steps past tend do nothing.
+// while t < tend, launched as many at a time as are expected to remain: graphs of 32 steps of the
+// separate kernels, single launches of the step kernel (2 us of host time each against 8 us and
+// more on the GPU) and of the rest.
 int update_loop(sfx_handle* H, int mode, double arg, sfx_step_stats* st) {
   HIPCHK(hipSetDevice(H->device));
   auto t_start = std::chrono::steady_clock::now();
   Scalars s;
   int rc = enter_step(H);
-  if (rc || (rc = H->on_step ? normalise(H, s) : read_scalars(H, s))) return rc;
+  if (rc || (rc = normalise(H, s))) return rc;
   if (s.error_pending) { s.error = 1; s.error_pending = 0; s.t = (double)H->hI.c.t1 + 1.0; }
   const int64_t nt0 = s.nt;
   bool single = false;
@@ -3689,20 +3908,19 @@ int update_loop(sfx_handle* H, int mode, double arg, sfx_step_stats* st) {
   if ((rc = write_scalars(H, s))) return rc;
   sfx_batch* B = solo(H);
   if (B->dirty && (rc = rebuild(B))) return rc;
-  if (single) {
-    launch(B, 7, 0);
-    end_steps(B);
-    HIPCHK(hipGetLastError());
-  } else {
-    const int K = 32;
-    if ((rc = ensure_graph(B, K))) return rc;
-    for (;;) {
-      HIPCHK(hipGraphLaunch(B->exec, B->stream));
-      if ((rc = read_scalars(H, s))) return rc;
-      if (!s.active || s.error || s.error_pending || !(s.t < s.tend)) break;
+  for (;;) {
+    int n = single ? 1 : steps_left(H, s);
+    if (!H->on_step && n >= GRAPH_STEPS) {
+      if ((rc = ensure_graph(B, GRAPH_STEPS))) return rc;
+      for (; n >= GRAPH_STEPS; n -= GRAPH_STEPS) HIPCHK(hipGraphLaunch(B->exec, B->stream));
     }
+    for (int k = 0; k < n; ++k) launch(B, 7, 0);
+    const int flip = B->flip;
+    B->flip = 0;
+    if ((rc = fetch_scalars(H, flip, 1))) return rc;
+    s = H->hs;
+    if (single || !s.active || s.error || s.error_pending || !(s.t < s.tend)) break;
   }
-  if ((rc = normalise(H, s))) return rc;
   if (s.error_pending) { s.error = 1; s.error_pending = 0; s.t = (double)H->hI.c.t1 + 1.0; if ((rc = write_scalars(H, s))) return rc; }
   if (st) {
     st->t = s.t; st->dt = s.dt; st->min_dt = s.min_dt; st->nt = s.nt; st->error = s.error;
@@ -3912,6 +4130,7 @@ extern "C" int sfx_batch_destroy(sfx_batch* B) {
   if (B->dInsts) hipFree(B->dInsts);
   if (B->dItems) hipFree(B->dItems);
   if (B->dIds) hipFree(B->dIds);
+  if (B->pin) hipHostFree(B->pin);
   if (B->own_stream && B->stream) hipStreamDestroy(B->stream);
   delete B;
   return SFX_OK;
@@ -3927,6 +4146,7 @@ extern "C" int sfx_batch_add(sfx_batch* B, sfx_handle* H, double t_end) {
   if (rc) return rc;
   s.tend = t_end;
   if ((rc = write_scalars(H, s))) return rc;
+  HIPCHK(hipStreamSynchronize(H->stream));   // the batch runs on its own stream
   B->members.push_back(H);
   B->tend.push_back(t_end);
   B->live.push_back(1);
@@ -3963,18 +4183,33 @@ extern "C" int sfx_batch_advance(sfx_batch* B, int32_t nsteps, int32_t* n_active
   }
   if (B->dirty && (rc = rebuild(B))) return rc;
   if (B->n_live + B->n_step > 0) {
-    const int K = std::max(1, std::min(nsteps, 64));
-    if ((rc = ensure_graph(B, K))) return rc;
-    for (int r = 0; r < nsteps / K; ++r) HIPCHK(hipGraphLaunch(B->exec, B->stream));
-    for (int r = 0; r < nsteps % K; ++r) launch(B, 7, 0);
-    end_steps(B);
+    if (B->n_live == 0) {   // the step kernel alone: one or two launches a step
+      for (int r = 0; r < nsteps; ++r) launch(B, 7, 0);
+    } else {
+      const int K = std::max(1, std::min(nsteps, 64));
+      if ((rc = ensure_graph(B, K))) return rc;
+      for (int r = 0; r < nsteps / K; ++r) HIPCHK(hipGraphLaunch(B->exec, B->stream));
+      for (int r = 0; r < nsteps % K; ++r) launch(B, 7, 0);
+    }
+    // the members' scalars to the host; the step kernel's last sweep is completed with them
+    const int flip = B->flip, ng = B->n_live;
+    B->flip = 0;
+    for (int32_t id : B->ids) B->members[id]->hs_ok = false;
+    if (ng) hipLaunchKernelGGL(k_give_scalars, dim3(ng), dim3(FBLOCK), 0, B->stream, B->dInsts, B->dIds, 0, 0, B->pin);
+    if (B->n_step)
+      hipLaunchKernelGGL(k_give_scalars, dim3(B->n_step), dim3(FBLOCK), 0, B->stream, B->dInsts, B->dIds + ng, flip, 1, B->pin + ng);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(B->stream));
+    for (size_t k = 0; k < B->ids.size(); ++k) {
+      sfx_handle* H = B->members[B->ids[k]];
+      H->hs = B->pin[k];
+      H->hs_ok = true;
+    }
   }
   int act = 0;
   for (size_t i = 0; i < B->members.size(); ++i) {
     Scalars s;
-    HIPCHK(hipMemcpy(&s, B->members[i]->dS, sizeof(Scalars), hipMemcpyDeviceToHost));
+    if ((rc = read_scalars(B->members[i], s))) return rc;
     if (!s.error && !s.error_pending && s.t < s.tend) ++act;
     else if (B->live[i]) { B->live[i] = 0; B->dirty = true; }   // leaves the work lists
   }
@@ -3987,7 +4222,8 @@ extern "C" int sfx_batch_done(sfx_batch* B, sfx_handle* H, int32_t* done) {
   HIPCHK(hipSetDevice(B->device));
   HIPCHK(hipStreamSynchronize(B->stream));
   Scalars s;
-  HIPCHK(hipMemcpy(&s, H->dS, sizeof(Scalars), hipMemcpyDeviceToHost));
+  const int rc = read_scalars(H, s);
+  if (rc) return rc;
   *done = (s.error || s.error_pending || !(s.t < s.tend)) ? 1 : 0;
   return SFX_OK;
 }
@@ -4019,6 +4255,7 @@ int time_phases(sfx_handle* H, int what, int trials, hipEvent_t e0, hipEvent_t e
     HIPCHK(hipEventSynchronize(e1));
     HIPCHK(hipEventElapsedTime(&t[k], e0, e1));
   }
+  H->hs_ok = false;
   std::sort(t.begin(), t.end());
   median = t[trials / 2];
   return SFX_OK;
@@ -4225,7 +4462,7 @@ extern "C" int sfx_profile_steps(sfx_handle* H, int32_t nsteps, double ms[3]) {
   sfx_batch* B = solo(H);
   if (B->dirty && (rc = rebuild(B))) return rc;
   Scalars s;
-  if ((rc = H->on_step ? normalise(H, s) : read_scalars(H, s))) return rc;
+  if ((rc = normalise(H, s))) return rc;
   s.tend = 1.0e30;
   if ((rc = write_scalars(H, s))) return rc;
   hipEvent_t ev[4];
@@ -4247,6 +4484,7 @@ extern "C" int sfx_profile_steps(sfx_handle* H, int32_t nsteps, double ms[3]) {
     }
   }
   end_steps(B);
+  H->hs_ok = false;
   for (auto& e : ev) hipEventDestroy(e);
   for (int k = 0; k < 3; ++k) ms[k] = acc[k] / nsteps;
   return SFX_OK;

@@ -99,6 +99,30 @@ struct StepImage {
 };
 static_assert(sizeof(Scalars) % 4 == 0 && sizeof(StepImage) % 4 == 0, "copied as words");
 
+// What a boundary flux point's step reads before levels and series: its index (<< 1 | whether the
+// reader stores its mean), its cells and uv-point, its direction, its boundary cell's index, series
+// and weight, a river cell's interior cell and offset. One record each, so that a thread has all of
+// them after one read.
+struct alignas(16) BndRec {
+  int32_t ib2, nmb, nmi, ip;
+  int32_t dir, indb, i1, i2;
+  int32_t rcell;
+  float fac, rdzs, zbuv;
+};
+// A face of the volume balance: its uv slot and its factor.
+struct alignas(16) BalRec {
+  double coef;
+  int32_t slot, pad_;
+};
+
+// A tile of the step kernel: the first of its boundary points and of its balance faces, their
+// numbers, and what the tile holds (FT_*).
+struct alignas(16) StepTile {
+  int32_t b0, f0;
+  uint16_t nb, nf;
+  int32_t flag;
+};
+
 struct DevInst {
   Consts c;
   int32_t dense, subgrid, fp64;
@@ -113,12 +137,12 @@ struct DevInst {
   int32_t nmt;                   // momentum tiles of the current tile shape
   int32_t mrow_sh;               // per-point kernel: log2 of the cell rows of a tile (mtm * P)
   // step kernel (k_step): rows and number of its tiles, n-columns (nmax * row blocks), division by
-  // nmax; per tile: how often it did nothing in a row, the marks that wake it (two sets), what it
-  // holds (FT_*), its boundary flux points (index << 1 | owner) and balance faces, as CSR lists
+  // nmax; per tile: how often it did nothing in a row, the marks that wake it (two sets), and its
+  // lists (StepTile) of boundary flux points and of balance faces
   int32_t frows, fnt, fcols;
   uint32_t fmagic;
-  uint8_t* fquiet; uint8_t* fwake; const uint8_t* fflag;
-  const int32_t* fb_ptr; const int32_t* fb_ent; const int32_t* ff_ptr; const int32_t* ff_ent;
+  uint8_t* fquiet; uint8_t* fwake;
+  const StepTile* ftile; const BndRec* fb_rec; const BalRec* ff_rec;
   // its level arrays: [0] are zs, vol, zsderv, kfuv, uvmean below
   double* zs_s[2]; double* vol_s[2]; float* zsd_s[2]; int8_t* kf_s[2]; float* um_s[2];
   ScalarBlock* sb;
@@ -194,19 +218,15 @@ struct DevInst {
   const float4* uv_lev;          // nslot*nl {havg, nrep, pwet, 0}
   // boundaries
   int32_t ngbnd, nkcuv2, nbnd, ntbnd;
-  const int32_t* gb_cell; const int32_t* gb_ind1; const int32_t* gb_ind2; const float* gb_fac; const int32_t* gb_nmi;
-  const int32_t* gb_rcell; const float* gb_rdzs;   // river cells (kcs 5): interior cell and level offset
   const float* zsi_bnd;                            // infragravity levels as zs_bnd (null: none)
   float* zsb; float* zsb0;
-  const int32_t* k2_slot; const int32_t* k2_nmb; const int32_t* k2_nmi; const int32_t* k2_ib; const int8_t* k2_dir;
-  const float* k2_zbuv;
   void* uvmean;
   const float* t_bnd; const float* zs_bnd;
   int32_t bnd_overlap;           // a Neumann copy and a boundary flux point share a cell
   int32_t n6;                    // Neumann boundary cells (kcs 6) ...
   const int32_t* gb6;            // ... as pairs {cell, interior cell}
   int32_t nflux;                 // kcuv 2/6 points whose boundary cell is not a Neumann cell ...
-  const int32_t* k2_flux;        // ... as indices into the k2_* tables
+  const BndRec* k2_rec;          // ... their records
   // sources and meteo; src_cell and qtsrc hold nsrc point sources, then each drainage
   // structure's intake and outfall
   int32_t nsrc, ntsrc, ntprcp, ntwnd;
@@ -560,6 +580,13 @@ __device__ __forceinline__ float rain_at(const DevInst& I, double t, int32_t& la
   return (G(I.tprcpv)[itp - 2] * (1.0f - twfac) + G(I.tprcpv)[itp - 1] * twfac) / (float)(1000 * 3600);
 }
 
+// A value that is the same in every lane, in scalar registers.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ float uniform(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
+__device__ __forceinline__ double uniform(double v) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)), __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
 // Position of time t in the boundary series: the samples itb0, itb1 (1-based) and the weight of
 // the second (sfincs_boundaries.f90:700-727).
 __device__ __forceinline__ float boundary_at(const DevInst& I, double t, int32_t& last, int32_t& itb0, int32_t& itb1) {
@@ -769,64 +796,81 @@ struct BndStep {
 };
 
 // One boundary flux point's inputs: everything update_boundary_fluxes reads from tables and
-// levels before its arithmetic (the level of its boundary cell, the interior level, the uv
-// tables), loaded by bnd_load without a store in between.
+// levels before its arithmetic (the samples its boundary cell's level lies between, the interior
+// level, the uv tables), loaded by bnd_load without a store or a test in between.
 template <typename R>
 struct BndPt {
-  int ib, nmb, nmi, ip, dir, kb;
+  int ib2, nmb, ip, dir, kb, kcuv;
+  float za1, zb1, za2, zb2, fac;   // the two samples at the cell's one or two series points
   float zsb1, zsb0, floorz, zbuv_or_zmin, zmaxu, havg_zmax, zb_nmi;
   R zsnmi, uvm;
   double vol_nmi;
-  int kcuv;
 };
 
-// update_boundary_points / update_boundary_conditions (:728-917) for the point's boundary
-// cell, and the point's other inputs (:941-1000).
+__device__ __forceinline__ BndRec bnd_record(const BndRec* rec, uint32_t k) {
+  const auto w = G((const float4*)rec);
+  const float4 a = ldf4(w, 3u * k), b = ldf4(w, 3u * k + 1u), c = ldf4(w, 3u * k + 2u);
+  return {__float_as_int(a.x), __float_as_int(a.y), __float_as_int(a.z), __float_as_int(a.w),
+          __float_as_int(b.x), __float_as_int(b.y), __float_as_int(b.z), __float_as_int(b.w),
+          __float_as_int(c.x), c.y, c.z, c.w};
+}
+
+// The samples itb0, itb1 of the series that the point's cell interpolates between.
 template <typename R>
-__device__ __forceinline__ void bnd_load(const DevInst& I, const BndStep<R>& B, int ib, BndPt<R>& p, GA<const double> zs,
+__device__ __forceinline__ void bnd_series(const DevInst& I, int i1, int i2, int itb0, int itb1, BndPt<R>& p) {
+  if (I.nbnd <= 0) return;
+  const int o0 = (itb0 - 1) * I.nbnd, o1 = (itb1 - 1) * I.nbnd;
+  p.za1 = G(I.zs_bnd)[o0 + i1]; p.zb1 = G(I.zs_bnd)[o1 + i1];
+  p.za2 = G(I.zs_bnd)[o0 + i2]; p.zb2 = G(I.zs_bnd)[o1 + i2];
+}
+
+template <typename R>
+__device__ __forceinline__ void bnd_load(const DevInst& I, const BndRec& r, int itb0, int itb1, BndPt<R>& p, GA<const double> zs,
                                          GA<const double> vol, GA<const R> uvmean) {
-  const Consts& c = I.c;
-  p.ib = ib;
-  p.nmb = G(I.k2_nmb)[ib];
+  p.ib2 = r.ib2; p.nmb = r.nmb; p.ip = r.ip; p.dir = r.dir; p.fac = r.fac;
   p.kb = G(I.kcs)[p.nmb] & KCS_MASK;
-  const int indb = G(I.k2_ib)[ib];
-  p.nmi = G(I.k2_nmi)[ib];
-  p.ip = G(I.k2_slot)[ib];
-  p.dir = G(I.k2_dir)[ib];
-  p.zsnmi = (R)zs[p.nmi];
-  p.uvm = uvmean[ib];
+  p.zsnmi = (R)zs[r.nmi];
+  p.uvm = uvmean[r.ib2 >> 1];
   p.kcuv = G(I.kcuv)[p.ip];
   p.floorz = I.subgrid ? G(I.z_zmin)[p.nmb] : G(I.zb)[p.nmb];
   if (I.subgrid) {
     const float4 s4 = ldf4(G(I.uv_s4), p.ip);
     p.zmaxu = s4.x; p.havg_zmax = s4.y;
     p.zbuv_or_zmin = G(I.uv_zmin)[p.ip];
-    p.vol_nmi = vol[p.nmi];
+    p.vol_nmi = vol[r.nmi];
     p.zb_nmi = 0.0f;
   } else {
-    p.zbuv_or_zmin = G(I.k2_zbuv)[ib];
-    p.zb_nmi = G(I.zb)[p.nmi];
+    p.zbuv_or_zmin = r.zbuv;
+    p.zb_nmi = G(I.zb)[r.nmi];
     p.zmaxu = p.havg_zmax = 0.0f;
     p.vol_nmi = 0.0;
   }
+  bnd_series<R>(I, r.i1, r.i2, itb0, itb1, p);
+}
+
+// update_boundary_points / update_boundary_conditions (:728-917): the level of the point's boundary
+// cell. The record is read again for what few points need.
+template <typename R>
+__device__ __forceinline__ void bnd_level(const DevInst& I, const BndStep<R>& B, const BndRec* rec, uint32_t k, BndPt<R>& p,
+                                          GA<const double> zs) {
+  const Consts& c = I.c;
   if (p.kb == 2) {
-    // update_boundary_points (:728-756) at the points this cell interpolates between
-    auto series_at = [&](const float* ser, int k) -> float {
-      const float za = G(ser)[(B.itb0 - 1) * I.nbnd + k], zb = G(ser)[(B.itb1 - 1) * I.nbnd + k];
-      return za + (zb - za) * B.tbfac;
-    };
     // update_boundary_conditions, water-level boundary (:789-917); the infragravity level
     // zig (bzi, :829-848) is interpolated as the water level
     double zst;
     float zig = 0.0f;
-    if (I.nbnd > 1) {
-      const float f = G(I.gb_fac)[indb];
-      const int i1 = G(I.gb_ind1)[indb] - 1, i2 = G(I.gb_ind2)[indb] - 1;
-      zst = (double)(series_at(I.zs_bnd, i1) * f + series_at(I.zs_bnd, i2) * (1.0f - f));
-      if (I.zsi_bnd) zig = series_at(I.zsi_bnd, i1) * f + series_at(I.zsi_bnd, i2) * (1.0f - f);
-    } else {
-      zst = (double)series_at(I.zs_bnd, 0);
-      if (I.zsi_bnd) zig = series_at(I.zsi_bnd, 0);
+    const float z1 = p.za1 + (p.zb1 - p.za1) * B.tbfac;   // update_boundary_points (:728-756)
+    if (I.nbnd > 1) zst = (double)(z1 * p.fac + (p.za2 + (p.zb2 - p.za2) * B.tbfac) * (1.0f - p.fac));
+    else zst = (double)z1;
+    if (I.zsi_bnd) {
+      const int o0 = (B.itb0 - 1) * I.nbnd, o1 = (B.itb1 - 1) * I.nbnd;
+      auto series_at = [&](int k) -> float {
+        const float za = G(I.zsi_bnd)[o0 + k], zb = G(I.zsi_bnd)[o1 + k];
+        return za + (zb - za) * B.tbfac;
+      };
+      const BndRec r = bnd_record(rec, k);
+      zig = series_at(r.i1);
+      if (I.nbnd > 1) zig = zig * p.fac + series_at(r.i2) * (1.0f - p.fac);
     }
     if ((c.flags & sfx::F_PATM) && c.pavbnd > 1.0f)   // barometric correction (:820-826)
       zst = zst + (double)((c.pavbnd - meteo_patm(I, B.m, p.nmb)) / (c.rhow * 9.81f));
@@ -846,10 +890,12 @@ __device__ __forceinline__ void bnd_load(const DevInst& I, const BndStep<R>& B, 
   } else if (p.kb == 5) {
     // downstream river cell (:878-901): the interior level plus the slope offset, raised
     // to the bed, in f64 (the interior cell is an ordinary cell, which no boundary step writes)
-    const double zst = sfx::vmax<double>(zs[G(I.gb_rcell)[indb]] + (double)G(I.gb_rdzs)[indb], (double)p.floorz);
+    const BndRec r = bnd_record(rec, k);
+    const double zst = sfx::vmax<double>(zs[r.rcell] + (double)r.rdzs, (double)p.floorz);
     p.zsb0 = (float)zst;
     p.zsb1 = p.zsb0;
   } else {
+    const int indb = bnd_record(rec, k).indb;
     p.zsb1 = G(I.zsb)[indb];
     p.zsb0 = G(I.zsb0)[indb];
   }
@@ -922,7 +968,7 @@ __device__ __forceinline__ void bnd_finish(const DevInst& I, const BndStep<R>& B
   R qb, ub, um;
   bnd_flux<R>(I, B, p, qb, ub, um);
   q[p.ip] = qb; uv[p.ip] = ub;
-  uvmean[p.ib] = um;
+  uvmean[p.ib2 >> 1] = um;
   G(I.zs)[p.nmb] = (double)p.zsb1;
   mark_cell(I, p.nmb);
   if (I.c.flags & sfx::F_ZSMAX) zsmax[p.nmb] = (R)sfx::vmax<double>((double)zsmax[p.nmb], (double)p.zsb1);
@@ -973,8 +1019,8 @@ __global__ void __launch_bounds__(FBLOCK) k_forcing(const DevInst* __restrict__ 
   if (I.bnd_overlap) __syncthreads();
   // update_boundary_fluxes (:941-1117), bndtype 1 (weakly reflective), over the flux
   // points (kcuv 2 points whose boundary cell is not a Neumann cell). Each thread takes two
-  // points and issues the loads of both before it finishes either, so the dependent chain
-  // of table and level reads is paid once per two points.
+  // points and issues the loads of both before it finishes either, so the two dependent reads
+  // (record, then levels and samples) are paid once per two points.
   const int curb = __builtin_amdgcn_readfirstlane(F.s.cur);
   const auto q = G((R*)I.q[curb]);
   const auto uv = G((R*)I.uv[curb]);
@@ -984,12 +1030,17 @@ __global__ void __launch_bounds__(FBLOCK) k_forcing(const DevInst* __restrict__ 
                      meteo_now(I, &F.s)};
   for (int k0 = threadIdx.x; k0 < I.nflux; k0 += 2 * FBLOCK) {
     const int k1 = k0 + FBLOCK;
+    const BndRec ra = bnd_record(I.k2_rec, k0), rb = bnd_record(I.k2_rec, min(k1, I.nflux - 1));
     BndPt<R> a, b;
-    bnd_load<R>(I, B, G(I.k2_flux)[k0], a, G((const double*)I.zs), G((const double*)I.vol), G((const R*)I.uvmean));
+    bnd_load<R>(I, ra, F.itb0, F.itb1, a, G((const double*)I.zs), G((const double*)I.vol), G((const R*)I.uvmean));
     if (k1 < I.nflux)
-      bnd_load<R>(I, B, G(I.k2_flux)[k1], b, G((const double*)I.zs), G((const double*)I.vol), G((const R*)I.uvmean));
+      bnd_load<R>(I, rb, F.itb0, F.itb1, b, G((const double*)I.zs), G((const double*)I.vol), G((const R*)I.uvmean));
+    bnd_level<R>(I, B, I.k2_rec, k0, a, G((const double*)I.zs));
     bnd_finish<R>(I, B, a, q, uv, uvmean, zsmax);
-    if (k1 < I.nflux) bnd_finish<R>(I, B, b, q, uv, uvmean, zsmax);
+    if (k1 < I.nflux) {
+      bnd_level<R>(I, B, I.k2_rec, k1, b, G((const double*)I.zs));
+      bnd_finish<R>(I, B, b, q, uv, uvmean, zsmax);
+    }
   }
   if (I.ndrn > 0) {   // update_discharges' drainage structures, after the boundaries (sfincs_lib.f90:530-550)
     __syncthreads();
@@ -2002,6 +2053,13 @@ __global__ void __launch_bounds__(BLOCK) k_continuity(const DevInst* __restrict_
 // and after, no cell changed) twice in a row hold the same values on both sides and are skipped
 // until a neighbouring block does something, rain falls or the host writes state; blocks with
 // boundary, source or inactive cells always run.
+//
+// A small mesh's step is one chain of dependent reads and divisions per block (a block of 64 x 96
+// cells: 0.6 us to the scalars, 0.7 to the keys and levels, 0.7 for the scalars' arithmetic, 1.3 for
+// the faces, 0.8 for the cells, and 2 at a boundary), so what a tile needs first comes in few reads:
+// a tile's marks and lists in one (StepTile), a boundary point's tables in another (BndRec). With
+// them, and uniform values in scalar registers so that no subgrid wave spills, 161 x 203 subgrid
+// cells take 9.6 us a step (10.4 before), 2048 x 2048 take 83 (88), 64 x 96 regular ones 8.5 (8.7).
 constexpr int STEP_COLS = WAVE - 1;
 constexpr uint8_t FT_RUN = 1, FT_BND = 2, FT_BAL = 4;          // fflag: never skipped; has boundary points; has balance faces
 
@@ -2009,6 +2067,12 @@ constexpr uint8_t FT_RUN = 1, FT_BND = 2, FT_BAL = 4;          // fflag: never s
 // for the point in its last step, 4 when it did so in its last two (both q buffers hold zeros, so
 // nothing is stored while it stays dry). Readers of kfuv take bit 0.
 constexpr int8_t SF_ZERO1 = 2, SF_ZERO2 = 4;
+
+__device__ __forceinline__ void bal_record(GA<const float4> rec, uint32_t k, double& coef, uint32_t& slot) {
+  const float4 r = ldf4(rec, k);
+  coef = __hiloint2double(__float_as_int(r.y), __float_as_int(r.x));
+  slot = (uint32_t)__float_as_int(r.z);
+}
 
 // What decides a face's branch, read ahead of its turn: kcuv, kfuv, the levels of its two cells and
 // its wet/dry threshold. n, m: its cell; ok: the face exists and is wanted.
@@ -2163,7 +2227,10 @@ __global__ void __launch_bounds__(BLOCK, SG ? 7 : 8) k_step(const DevInst* __res
   const int lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   constexpr int W = BLOCK / WAVE;
 
-  // the step's scalars, in every wave
+  // the step's scalars, in every wave, and what the tile holds
+  const float4 T4 = ldf4(G((const float4*)I.ftile), (uint32_t)tile);
+  const uint32_t quiet4 = G((const uint32_t*)I.fquiet)[tile];   // one byte per wave
+  const uint8_t wake0 = G(I.fwake)[(uint32_t)tile], wake1 = G(I.fwake)[(uint32_t)(I.fnt + tile)];
   Scalars n;
   {
     const auto src = G((const uint32_t*)&SB->s[flip]);
@@ -2173,8 +2240,10 @@ __global__ void __launch_bounds__(BLOCK, SG ? 7 : 8) k_step(const DevInst* __res
     __builtin_memcpy(&n, words, sizeof(Scalars));
   }
   const int kset = n.kset, side = n.side, cur = n.cur;
-  const uint8_t flag = G(I.fflag)[tile], woken = G(I.fwake)[(uint32_t)(side * I.fnt + tile)];
-  const uint32_t quiet = G((const uint32_t*)I.fquiet)[tile];   // one byte per wave
+  const int tb0 = uniform(__float_as_int(T4.x)), tf0 = uniform(__float_as_int(T4.y));   // as StepTile
+  const int tnn = uniform(__float_as_int(T4.z)), flag = uniform(__float_as_int(T4.w));
+  const uint32_t quiet = (uint32_t)uniform((int)quiet4);
+  const int woken = uniform(side ? wake1 : wake0);
   const bool asleep = !woken && !(flag & FT_RUN) && quiet == 0x02020202u && !(I.c.flags & sfx::F_QEXT);
   if (asleep && !(I.c.flags & sfx::F_PRECIP)) return;
 
@@ -2197,11 +2266,11 @@ __global__ void __launch_bounds__(BLOCK, SG ? 7 : 8) k_step(const DevInst* __res
   FaceIn f = step_load<SG>(I, w, cn, m0, jok, lane, zs0, kf0);   // in flight while the scalars are worked out
 
   if (n.pend) {
-    uint32_t k = wave_max_last(G(SB->key[kset])[lane * KEY_STRIDE]);
+    const uint32_t k = wave_max_last(G(SB->key[kset])[lane * KEY_STRIDE]);
     n.min_dt = key_step((uint32_t)__builtin_amdgcn_readlane((int)k, WAVE - 1), 0, I.c.dtmax);
     n.pend = 0;
   }
-  const int go = advance(I.c, n);
+  const int go = uniform(advance(I.c, n));
   const int k1 = kset == 2 ? 0 : kset + 1, k2 = k1 == 2 ? 0 : k1 + 1;
   int itb0 = 1, itb1 = 1;
   float tbfac = 0.f;
@@ -2221,7 +2290,7 @@ __global__ void __launch_bounds__(BLOCK, SG ? 7 : 8) k_step(const DevInst* __res
       if (w == 0) G(SB->key[k2])[lane * KEY_STRIDE] = 0u;
       if (n.ahead)
         for (int k = threadIdx.x; k < I.nsrc; k += BLOCK) G(I.qtsrc)[k] = source_at(I, n.t, n.itsrclast + 1, k);
-      if (threadIdx.x == 0 && (I.c.flags & sfx::F_PRECIP)) I.bal[2] = I.bal[2] + (double)(n.netprcp * n.dt) * I.rain_area;
+      if (threadIdx.x == 0 && (I.c.flags & sfx::F_PRECIP)) atomicAdd(I.bal + 2, (double)(n.netprcp * n.dt) * I.rain_area);
     }
     Scalars o = n;
     o.ahead = 0; o.mom_done = 0;
@@ -2230,22 +2299,27 @@ __global__ void __launch_bounds__(BLOCK, SG ? 7 : 8) k_step(const DevInst* __res
   }
   const bool dry_sky = !(I.c.flags & sfx::F_PRECIP) || n.netprcp == 0.f;
   if (!go || (asleep && dry_sky)) return;
+  if (SG) {   // fewer vector registers, or a wave would spill; regular waves have room, and dt there is quicker to use
+    n.t = uniform(n.t); n.dt = uniform(n.dt); n.netprcp = uniform(n.netprcp);
+    n.ahead = uniform(n.ahead); n.itsrclast = uniform(n.itsrclast);
+  }
 
   if (flag & FT_BND) {   // the boundary points this block reads, at the step's time (see above)
     const BndStep<float> B{itb0, itb1, tbfac, n.t, n.factime, n.facrel, n.one_minus_factime, MeteoNow{}};
     const auto um0 = G((const float*)I.um_s[side]);
     const auto um1 = G(I.um_s[side ^ 1]);
-    const int e1 = G(I.fb_ptr)[tile + 1];
-    for (int e = G(I.fb_ptr)[tile] + (int)threadIdx.x; e < e1; e += BLOCK) {
-      const int ent = G(I.fb_ent)[e];
+    const int bn = tnn & 0xffff;
+    for (int e = (int)threadIdx.x; e < bn; e += BLOCK) {
+      const uint32_t k = (uint32_t)(tb0 + e);
       BndPt<float> p;
-      bnd_load<float>(I, B, ent >> 1, p, zs0, vol0, um0);
+      bnd_load<float>(I, bnd_record(I.fb_rec, k), itb0, itb1, p, zs0, vol0, um0);
+      bnd_level<float>(I, B, I.fb_rec, k, p, zs0);
       float qb, ub, um;
       bnd_flux<float>(I, B, p, qb, ub, um);
       G((float*)I.q[cur])[p.ip] = qb;
       G((float*)I.uv[cur])[p.ip] = ub;
       G(I.zs_s[side])[p.nmb] = (double)p.zsb1;
-      if (ent & 1) um1[p.ib] = um;
+      if (p.ib2 & 1) um1[p.ib2 >> 1] = um;
     }
     __syncthreads();
   }
@@ -2265,7 +2339,14 @@ __global__ void __launch_bounds__(BLOCK, SG ? 7 : 8) k_step(const DevInst* __res
   }
   const uint32_t key = wave_max_last(step_key<float>(mden, I.c.dtmax));
   if (lane == WAVE - 1) lkey[w] = key;
+  const int fn = w == 0 ? (int)((uint32_t)tnn >> 16) : 0;   // balance faces, in the first wave
+  uint32_t bslot = 0u;
+  double bcoef = 0.0;
+  const auto fw = G((const float4*)I.ff_rec);
+  if (lane < fn) bal_record(fw, (uint32_t)(tf0 + lane), bcoef, bslot);
   __syncthreads();
+  float bq = 0.f;
+  if (lane < fn) bq = q1[bslot];
   if (threadIdx.x == 0) {
     uint32_t k = lkey[0];
     for (int i = 1; i < W; ++i) k = lkey[i] > k ? lkey[i] : k;
@@ -2280,12 +2361,11 @@ __global__ void __launch_bounds__(BLOCK, SG ? 7 : 8) k_step(const DevInst* __res
                         lv[r * WAVE + lane - 1], lv[r * WAVE + lane], dry_sky, zs0, zs1, vol0, vol1, zsd0, zsd1))
         act = true;
   }
-  if ((flag & FT_BAL) && w == 0) {   // volume into the interior cells through this block's balance faces
-    double acc = 0.0;
-    const int e1 = G(I.ff_ptr)[tile + 1];
-    for (int e = G(I.ff_ptr)[tile] + lane; e < e1; e += WAVE) {
-      const int f = G(I.ff_ent)[e];
-      acc += G(I.bf_coef)[f] * (double)q1[G(I.bf_slot)[f]];
+  if (fn) {   // volume into the interior cells through this block's balance faces
+    double acc = bcoef * (double)bq;
+    for (int e = lane + WAVE; e < fn; e += WAVE) {
+      bal_record(fw, (uint32_t)(tf0 + e), bcoef, bslot);
+      acc += bcoef * (double)q1[bslot];
     }
     for (int o = WAVE / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, WAVE);
     if (lane == 0 && acc != 0.0) atomicAdd(I.bal, acc * (double)n.dt);
@@ -2487,6 +2567,7 @@ struct sfx_handle {
   // step kernel: whether the handle may use it (step_rule), is meant to (not pinned to other
   // shapes) and is using it now (on_step: the state lies on Scalars::side of the level arrays)
   bool stepable = false, use_step = false, on_step = false;
+  std::vector<BndRec> bnd_recs;   // while the handle is made
   // The step scalars as they are on the device (hs_ok: every kernel that changes them is followed
   // by k_give_scalars into `pin`, pinned host memory), so that calls need not fetch them first.
   Scalars hs{};
@@ -2692,7 +2773,7 @@ namespace {
 void stage_open(sfx_handle* H);
 void stage_close(sfx_handle* H);
 bool step_rule(const DevInst& I, const sfx_model* M);
-void build_step(sfx_handle* H, const sfx_model* M, const std::vector<int32_t>& bf);
+void build_step(sfx_handle* H, const sfx_model* M, const std::vector<int32_t>& bf, const std::vector<double>& coef);
 }
 
 extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, sfx_handle** out);
@@ -2833,9 +2914,6 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
   {
     std::vector<int32_t> cell(M->ngbnd), nmi(M->ngbnd);
     for (int i = 0; i < M->ngbnd; ++i) { cell[i] = M->nmindbnd[i] - 1; nmi[i] = M->nmi_gbp[i] - 1; }
-    I.gb_cell = H->upload(cell.data(), cell.size()); I.gb_nmi = H->upload(nmi.data(), nmi.size());
-    I.gb_ind1 = H->upload(M->ind1_bnd_gbp.data(), M->ngbnd); I.gb_ind2 = H->upload(M->ind2_bnd_gbp.data(), M->ngbnd);
-    I.gb_fac = H->upload(M->fac_bnd_gbp.data(), M->ngbnd);
     std::vector<int32_t> rcell(M->ngbnd, -1);
     std::vector<float> rdzs(M->ngbnd, 0.f);
     for (int i = 0; i < M->ngbnd; ++i)
@@ -2843,7 +2921,6 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
         rcell[i] = M->index_zsi_bdr[M->index_bdr_gbp[i] - 1] - 1;
         rdzs[i] = M->dzs_bdr[M->index_bdr_gbp[i] - 1];
       }
-    I.gb_rcell = H->upload(rcell.data(), rcell.size()); I.gb_rdzs = H->upload(rdzs.data(), rdzs.size());
     I.zsb = H->upload(M->zsb.data(), M->ngbnd); I.zsb0 = H->upload(M->zsb0.data(), M->ngbnd);
     std::vector<int32_t> slot(M->nkcuv2), nmb(M->nkcuv2), nmi2(M->nkcuv2), ib(M->nkcuv2);
     std::vector<float> zbuv(M->nkcuv2, 0.f);
@@ -2852,9 +2929,6 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
       ib[i] = M->ibkcuv2[i] - 1;
       if (!M->subgrid) zbuv[i] = M->zbuv[M->index_kcuv2[i] - 1];
     }
-    I.k2_slot = H->upload(slot.data(), slot.size()); I.k2_nmb = H->upload(nmb.data(), nmb.size());
-    I.k2_nmi = H->upload(nmi2.data(), nmi2.size()); I.k2_ib = H->upload(ib.data(), ib.size());
-    I.k2_dir = H->upload(M->ibuvdir.data(), M->ibuvdir.size()); I.k2_zbuv = H->upload(zbuv.data(), zbuv.size());
     I.t_bnd = H->upload(M->t_bnd.data(), M->t_bnd.size()); I.zs_bnd = H->upload(M->zs_bnd.data(), M->zs_bnd.size());
     I.zsi_bnd = M->zsi_bnd.empty() ? nullptr : H->upload(M->zsi_bnd.data(), M->zsi_bnd.size());
     // Neumann copies (kcs 6) run before the flux points only when they share a cell
@@ -2872,11 +2946,24 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
       if (M->kcs[cell[i]] == 6) { g6.push_back(cell[i]); g6.push_back(nmi[i]); }
     I.n6 = (int32_t)(g6.size() / 2);
     I.gb6 = g6.empty() ? nullptr : H->upload(g6.data(), g6.size());
-    std::vector<int32_t> fl;
+    H->bnd_recs.clear();   // also for the step kernel's tiles
     for (int i = 0; i < M->nkcuv2; ++i)
-      if (M->kcs[nmb[i]] != 6) fl.push_back(i);
-    I.nflux = (int32_t)fl.size();
-    I.k2_flux = fl.empty() ? nullptr : H->upload(fl.data(), fl.size());
+      if (M->kcs[nmb[i]] != 6) {
+        BndRec r{};
+        const int g = ib[i];
+        auto point = [&](int k) { return std::min(std::max(k - 1, 0), std::max(0, M->nbnd - 1)); };
+        r.ib2 = 2 * i + 1; r.nmb = nmb[i]; r.nmi = nmi2[i]; r.ip = slot[i];
+        r.dir = M->ibuvdir[i]; r.indb = g; r.zbuv = zbuv[i];
+        r.rcell = r.nmi;   // a place to read where there is no river cell
+        if (g >= 0) {
+          r.i1 = point(M->ind1_bnd_gbp[g]); r.i2 = point(M->ind2_bnd_gbp[g]); r.fac = M->fac_bnd_gbp[g];
+          if (rcell[g] >= 0) { r.rcell = rcell[g]; r.rdzs = rdzs[g]; }
+        }
+        if (M->nbnd <= 1) r.i1 = r.i2 = 0;   // one series serves every cell
+        H->bnd_recs.push_back(r);
+      }
+    I.nflux = (int32_t)H->bnd_recs.size();
+    I.k2_rec = H->bnd_recs.empty() ? nullptr : H->upload(H->bnd_recs.data(), H->bnd_recs.size());
   }
   I.nsrc = M->nsrc; I.ntsrc = M->ntsrc; I.ntprcp = M->ntprcp; I.ntwnd = M->ntwnd;
   I.ndrn = M->ndrn; I.structure_relax = M->p.structure_relax;
@@ -2974,7 +3061,8 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
     }
     H->stepable = step_rule(I, M);
     H->use_step = H->stepable;
-    if (H->stepable) build_step(H, M, slot);
+    if (H->stepable) build_step(H, M, slot, coef);
+    H->bnd_recs = {};
   }
   H->dI = H->upload(&I, 1);
   if (hipHostMalloc((void**)&H->pin, sizeof(Scalars)) != hipSuccess) H->pin = nullptr;
@@ -3014,8 +3102,8 @@ int step_rows(size_t np) {
   return np <= 150000 ? 1 : (np <= 750000 ? 3 : (np <= 2000000 ? 5 : 7));
 }
 
-// The step kernel's second side and per-tile tables. bf: the balance faces' slots.
-void build_step(sfx_handle* H, const sfx_model* M, const std::vector<int32_t>& bf) {
+// The step kernel's second side and per-tile tables. bf, coef: the balance faces' slots and factors.
+void build_step(sfx_handle* H, const sfx_model* M, const std::vector<int32_t>& bf, const std::vector<double>& coef) {
   DevInst& I = H->hI;
   const int nmax = I.nmax, mmax = I.mmax, np = I.np, fr = step_rows((size_t)np);
   I.frows = fr;
@@ -3033,34 +3121,36 @@ void build_step(sfx_handle* H, const sfx_model* M, const std::vector<int32_t>& b
   }
   // a tile reads the values of points up to two rows and columns from its cells (its own faces and
   // the repeated ones, and their stencils), and sets the levels of its boundary cells
-  std::vector<std::vector<int32_t>> pts(I.fnt), faces(I.fnt);
-  for (int i = 0; i < M->nkcuv2; ++i) {
-    if (M->kcs[M->nmbkcuv2[i] - 1] == 6) continue;
-    const int s = H->ref2slot[M->index_kcuv2[i] - 1], c = s % np, n = c % nmax, m = c / nmax, own = tile_of(n, m);
+  std::vector<std::vector<BndRec>> pts(I.fnt);
+  std::vector<std::vector<BalRec>> faces(I.fnt);
+  for (const BndRec& r : H->bnd_recs) {
+    const int c = r.ip % np, n = c % nmax, m = c / nmax, own = tile_of(n, m);
     for (int dm = -2; dm <= 2; ++dm)
       for (int dn = -2; dn <= 2; ++dn) {
         if (n + dn < 0 || n + dn >= nmax || m + dm < 0 || m + dm >= mmax) continue;
-        const int t = tile_of(n + dn, m + dm), ent = 2 * i + (t == own ? 1 : 0);
-        if (std::find(pts[t].rbegin(), pts[t].rend(), ent) == pts[t].rend()) pts[t].push_back(ent);
+        const int t = tile_of(n + dn, m + dm);
+        if (!pts[t].empty() && pts[t].back().ib2 >> 1 == r.ib2 >> 1) continue;   // one point's turns follow each other
+        pts[t].push_back(r);
+        if (t != own) pts[t].back().ib2 &= ~1;
       }
   }
   for (size_t f = 0; f < bf.size(); ++f) {
     const int c = bf[f] % np;
-    faces[tile_of(c % nmax, c / nmax)].push_back((int32_t)f);
+    faces[tile_of(c % nmax, c / nmax)].push_back(BalRec{coef[f], bf[f], 0});
   }
-  auto csr = [&](const std::vector<std::vector<int32_t>>& v, uint8_t bit, const int32_t*& ptr, const int32_t*& ent) {
-    std::vector<int32_t> p(1, 0), e;
-    for (int t = 0; t < I.fnt; ++t) {
-      e.insert(e.end(), v[t].begin(), v[t].end());
-      p.push_back((int32_t)e.size());
-      if (!v[t].empty()) flag[t] |= bit | FT_RUN;
-    }
-    ptr = H->upload(p.data(), p.size());
-    ent = H->upload(e.data(), e.size());
-  };
-  csr(pts, FT_BND, I.fb_ptr, I.fb_ent);
-  csr(faces, FT_BAL, I.ff_ptr, I.ff_ent);
-  I.fflag = H->upload(flag.data(), flag.size());
+  std::vector<StepTile> tiles(I.fnt);
+  std::vector<BndRec> recs;
+  std::vector<BalRec> bals;
+  for (int t = 0; t < I.fnt; ++t) {
+    if (!pts[t].empty()) flag[t] |= FT_BND | FT_RUN;
+    if (!faces[t].empty()) flag[t] |= FT_BAL | FT_RUN;
+    tiles[t] = StepTile{(int32_t)recs.size(), (int32_t)bals.size(), (uint16_t)pts[t].size(), (uint16_t)faces[t].size(), flag[t]};
+    recs.insert(recs.end(), pts[t].begin(), pts[t].end());
+    bals.insert(bals.end(), faces[t].begin(), faces[t].end());
+  }
+  I.ftile = H->upload(tiles.data(), tiles.size());
+  I.fb_rec = H->upload(recs.data(), recs.size());
+  I.ff_rec = H->upload(bals.data(), bals.size());
   I.fquiet = H->alloc<uint8_t>((size_t)I.fnt * (BLOCK / WAVE));
   I.fwake = H->alloc<uint8_t>((size_t)I.fnt * 2);
   I.zs_s[1] = H->alloc<double>(np);

@@ -123,6 +123,12 @@ struct alignas(16) StepTile {
   int32_t flag;
 };
 
+// Quadtrees of up to this many cells make their combined points in the continuity launch of a whole
+// step: that saves a launch of 3 to 5 us, but the few cells that do it hold up their waves. Measured,
+// us per step with the launch / without it: 22 thousand cells 19.0 / 17.4, 88 thousand 20.2 / 18.5,
+// 298 thousand 26.9 / 25.2, 559 thousand 33.7 / 31.9, 2.4 million 90 / 95.
+constexpr int CUV_FACES_CELLS = 1 << 20;
+
 struct DevInst {
   Consts c;
   int32_t dense, subgrid, fp64;
@@ -212,6 +218,7 @@ struct DevInst {
   const uint8_t* uvf;            // indexed: iref | (type+1)<<4 | dir<<6
   const int32_t* nb;             // indexed: 10 tables of npuv (nm,nmu,u_nmd,u_nmu,u_ndm,u_num,v_ndm,v_nm,v_ndmu,v_nmu)
   const int32_t* cuv;            // indexed: 3 tables of ncuv (cuv, uv1, uv2)
+  int32_t cuv_faces;             // cells make the combined points: each j is slot npuv + j and a face of one cell
   const float* uv_zmin;
   const float4* uv_s4;           // {zmax, havg_zmax, nrep_zmax, navg_w}
   const float* uv_fnfit;
@@ -1708,7 +1715,28 @@ __global__ void __launch_bounds__(BLOCK) k_mom_idx(const DevInst* __restrict__ i
   mom_epilogue<R>(I, tile, mden);
 }
 
-// Combined uv-points at refinement transitions (sfincs_momentum.f90:757-779).
+// Combined uv-points at refinement transitions (sfincs_momentum.f90:757-779): the mean of their two
+// points, q and uv of the sweep. The reference averages inside compute_fluxes, before
+// compute_fluxes_over_structures sets this step's weir discharges, so a weir point (kcuv 3) enters
+// with the last step's value: the other ping-pong buffer. Its uv is 0 in both.
+template <typename R>
+__device__ __forceinline__ R combined_q(const DevInst& I, GA<const R> q, GA<const R> q_last, uint32_t j) {
+  const int a = G(I.cuv)[I.ncuv + j], b = G(I.cuv)[2 * I.ncuv + j];
+  R qa = q[a], qb = q[b];
+  if (I.struc_of) {
+    if (G(I.kcuv)[a] == 3) qa = q_last[a];
+    if (G(I.kcuv)[b] == 3) qb = q_last[b];
+  }
+  return (qa + qb) / R(2);
+}
+template <typename R>
+__device__ __forceinline__ R combined_uv(const DevInst& I, GA<const R> uv, uint32_t j) {
+  return (uv[G(I.cuv)[I.ncuv + j]] + uv[G(I.cuv)[2 * I.ncuv + j]]) / R(2);
+}
+
+// All of them, after a momentum sweep of its own (compute_fluxes). In a whole step the continuity
+// launch, whose cells are the first to read them, makes them (make_combined) on meshes of up to
+// CUV_FACES_CELLS cells.
 template <typename R>
 __global__ void __launch_bounds__(BLOCK) k_cuv(const DevInst* __restrict__ insts, WorkList L) {
   int tile, inst;
@@ -1721,15 +1749,9 @@ __global__ void __launch_bounds__(BLOCK) k_cuv(const DevInst* __restrict__ insts
   const int cur = G(Sp)->cur, cur1 = cur ^ 1;
   const auto q = G((R*)I.q[cur1]);
   const auto uv = G((R*)I.uv[cur1]);
-  const int c = G(I.cuv)[j], a = G(I.cuv)[I.ncuv + j], b = G(I.cuv)[2 * I.ncuv + j];
-  // The reference averages inside compute_fluxes, before compute_fluxes_over_structures
-  // sets this step's weir discharges, so a weir point (kcuv 3) enters with the last
-  // step's value: the other ping-pong buffer. Its uv is 0 in both.
-  const auto q_last = G((const R*)I.q[cur]);
-  const R qa = G(I.kcuv)[a] == 3 ? q_last[a] : q[a];
-  const R qb = G(I.kcuv)[b] == 3 ? q_last[b] : q[b];
-  q[c] = (qa + qb) / R(2);
-  uv[c] = (uv[a] + uv[b]) / R(2);
+  const int c = G(I.cuv)[j];
+  q[c] = combined_q<R>(I, G((const R*)I.q[cur1]), G((const R*)I.q[cur]), (uint32_t)j);
+  uv[c] = combined_uv<R>(I, G((const R*)I.uv[cur1]), (uint32_t)j);
 }
 
 // ----------------------------------------------------------------------------- continuity
@@ -1923,18 +1945,35 @@ __device__ __forceinline__ void count_stores(const DevInst& I, int tile, unsigne
   }
 }
 
+// Makes the combined point at `slot`, a face of this thread's cell and of no other, and stores it.
+template <typename R>
+__device__ __forceinline__ R make_combined(const DevInst& I, int qb, uint32_t slot) {
+  const uint32_t j = slot - (uint32_t)I.npuv;
+  const R v = combined_q<R>(I, G((const R*)I.q[qb]), G((const R*)I.q[qb ^ 1]), j);
+  G((R*)I.q[qb])[slot] = v;
+  G((R*)I.uv[qb])[slot] = combined_uv<R>(I, G((const R*)I.uv[qb]), j);
+  return v;
+}
+
 // One block of a continuity launch per scenario: the volume this step's update moves
 // through the faces between interior cells and cells that are not interior, from the same
 // q buffer and dt as the cells, and the step's rain volume, added in FP64 to bal[0], bal[2].
 template <typename R>
-__device__ void balance_block(const DevInst& I) {
+__device__ void balance_block(const DevInst& I, bool make) {
   const auto S = G(I.sc);
   if (!S->active) return;
   const int qb = __builtin_amdgcn_readfirstlane(S->mom_done ? (S->cur ^ 1) : S->cur);
   const auto q = G((const R*)I.q[qb]);
   const R dt = (R)S->dt;
   double acc = 0.0;
-  for (int f = threadIdx.x; f < I.nbf; f += BLOCK) acc += G(I.bf_coef)[f] * (double)q[G(I.bf_slot)[f]];
+  make = make && I.cuv_faces;
+  for (int f = threadIdx.x; f < I.nbf; f += BLOCK) {
+    const uint32_t slot = (uint32_t)G(I.bf_slot)[f];
+    R v = q[slot];
+    if (make && slot >= (uint32_t)I.npuv && slot < (uint32_t)(I.npuv + I.ncuv))   // a cell makes it meanwhile
+      v = combined_q<R>(I, q, G((const R*)I.q[qb ^ 1]), slot - (uint32_t)I.npuv);
+    acc += G(I.bf_coef)[f] * (double)v;
+  }
   for (int o = WAVE / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, WAVE);
   __shared__ double red[BLOCK / WAVE];
   if (threadIdx.x % WAVE == 0) red[threadIdx.x / WAVE] = acc;
@@ -1951,17 +1990,17 @@ __device__ void balance_block(const DevInst& I) {
 // The first `nahead` blocks compute the next step of scenario ahead_ids[b] of ahead_insts
 // (forcing_ahead_block), the next `nbal` blocks the volume balance of scenario
 // ahead_ids[b - nahead] (balance_block); the leading blocks are padded to a multiple of 8,
-// so the cells keep their XCDs. RX: some scenario of the launch has infiltration or
+// so the cells keep their XCDs. step: a whole step (the cells make the combined points). RX: some scenario of the launch has infiltration or
 // gridded rain (per-cell rain and its balance slots); the instantiation without it
 // carries none of that code.
 template <typename R, bool RX>
 __global__ void __launch_bounds__(BLOCK) k_continuity(const DevInst* __restrict__ insts, WorkList L, int indexed,
-                                                      int nahead, int nbal, const DevInst* __restrict__ ahead_insts,
+                                                      int step, int nahead, int nbal, const DevInst* __restrict__ ahead_insts,
                                                       const int32_t* __restrict__ ahead_ids) {
   const uint32_t lead = (uint32_t)(nahead + nbal + 7) / 8 * 8;
   if (blockIdx.x < lead) {
     if ((int)blockIdx.x < nahead) forcing_ahead_block(ahead_insts[ahead_ids[blockIdx.x]]);
-    else if ((int)blockIdx.x < nahead + nbal) balance_block<R>(ahead_insts[ahead_ids[blockIdx.x - nahead]]);
+    else if ((int)blockIdx.x < nahead + nbal) balance_block<R>(ahead_insts[ahead_ids[blockIdx.x - nahead]], step != 0);
     return;
   }
   int tile, inst;
@@ -2008,7 +2047,21 @@ __global__ void __launch_bounds__(BLOCK) k_continuity(const DevInst* __restrict_
   } else {
     const int c = tile * BLOCK + threadIdx.x;
     if (c < I.np) {
-    const R q_md = q[G(I.zmd)[c]], q_mu = q[G(I.zmu)[c]], q_nd = q[G(I.znd)[c]], q_nu = q[G(I.znu)[c]];
+    const uint32_t md = G(I.zmd)[c], mu = G(I.zmu)[c], nd = G(I.znd)[c], nu = G(I.znu)[c];
+    R q_md = q[md], q_mu = q[mu], q_nd = q[nd], q_nu = q[nu];
+    if (step && I.cuv_faces) {   // a turn per combined face: rarely more than one in a wave
+      const uint32_t lo = (uint32_t)I.npuv, n = (uint32_t)I.ncuv;
+      unsigned todo = (md - lo < n ? 1u : 0u) | (mu - lo < n ? 2u : 0u) | (nd - lo < n ? 4u : 0u) | (nu - lo < n ? 8u : 0u);
+      while (todo) {
+        const unsigned k = todo & (0u - todo);
+        todo ^= k;
+        const R v = make_combined<R>(I, qb, k == 1u ? md : (k == 2u ? mu : (k == 4u ? nd : nu)));
+        if (k == 1u) q_md = v;
+        else if (k == 2u) q_mu = v;
+        else if (k == 4u) q_nd = v;
+        else q_nu = v;
+      }
+    }
     const int iref = G(I.z_iref)[c];
     const unsigned w = I.subgrid ? cont_update<R, true, RX>(I, c, q_md, q_mu, q_nd, q_nu, iref, dt, netprcp, dry_sky, mt, inf)
                                  : cont_update<R, false, RX>(I, c, q_md, q_mu, q_nd, q_nu, iref, dt, netprcp, dry_sky, mt, inf);
@@ -2017,7 +2070,7 @@ __global__ void __launch_bounds__(BLOCK) k_continuity(const DevInst* __restrict_
       R u_md = R(0), u_mu = R(0), u_nd = R(0), u_nu = R(0);
       if (I.c.flags & sfx::F_VELMAX) {
         const auto uv = G((const R*)I.uv[qb]);
-        u_md = uv[G(I.zmd)[c]]; u_mu = uv[G(I.zmu)[c]]; u_nd = uv[G(I.znd)[c]]; u_nu = uv[G(I.znu)[c]];
+        u_md = uv[md]; u_mu = uv[mu]; u_nd = uv[nd]; u_nu = uv[nu];
       }
       store_vars<R>(I, c, q_md, q_mu, q_nd, q_nu, u_md, u_mu, u_nd, u_nu, dt);
     }
@@ -2647,6 +2700,7 @@ struct sfx_batch {
   // [cell sg, cell reg, strip sg, strip reg, idx sg, idx reg, point sg, point reg]
   size_t off_m[NLIST_M] = {}, n_m[NLIST_M] = {};
   WorkList wl_m[NLIST_M] = {}, wl_cuv = {}, wl_cd = {}, wl_ci = {};   // launch arguments of the lists
+  bool cuv_apart = false;        // a member's combined points need k_cuv in whole steps too
   size_t off_cuv = 0, n_cuv = 0, off_cd = 0, n_cd = 0, off_ci = 0, n_ci = 0;
   // step kernel lists (subgrid, regular), the scenarios in them (dIds + n_live onwards), and which
   // scalar set the next launch reads
@@ -2887,6 +2941,13 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
       cv[j] = M->cuv_index_uv[j] - 1; cv[ncuv + j] = M->cuv_index_uv1[j] - 1; cv[2 * ncuv + j] = M->cuv_index_uv2[j] - 1;
     }
     I.cuv = H->upload(cv.data(), cv.size());
+    std::vector<int> used(ncuv, 0);
+    for (const auto* z : {&a, &b, &c2, &d})
+      for (int k : *z)
+        if (k >= npuv && k < npuv + ncuv) ++used[k - npuv];
+    I.cuv_faces = ncuv > 0 && np <= CUV_FACES_CELLS;
+    for (int j = 0; j < ncuv; ++j)
+      if (used[j] != 1 || cv[j] != npuv + j) I.cuv_faces = 0;
   }
   // uv slots
   {
@@ -3661,6 +3722,7 @@ int rebuild(sfx_batch* B) {
   std::vector<Item> mom[NLIST_M], cu, cd, ci, st[2];
   std::vector<int32_t> ids, ids_step;
   int fp64 = -1;
+  B->cuv_apart = false;
   B->built_step.assign(nm, 0);
   if (B->live.size() != nm) B->live.assign(nm, 1);
   for (size_t i = 0; i < nm; ++i) {
@@ -3684,6 +3746,7 @@ int rebuild(sfx_batch* B) {
     if (!I.dense) {
       const int tq = (I.ncuv + BLOCK - 1) / BLOCK;
       for (int t = 0; t < tq; ++t) cu.push_back(Item{(int)i, t});
+      B->cuv_apart = B->cuv_apart || (tq > 0 && !I.cuv_faces);
     }
   }
   B->fp64 = fp64 < 0 ? 0 : fp64;
@@ -3829,7 +3892,7 @@ void launch_phases(sfx_batch* B, int what, int forcing_mode) {
     SFX_MOM_POINT(8, true, 2) SFX_MOM_POINT(9, false, 2)
     SFX_MOM_POINT(10, true, 4) SFX_MOM_POINT(11, false, 4)
 #undef SFX_MOM_POINT
-    if (B->n_cuv) hipLaunchKernelGGL(k_cuv<R>, dim3(B->n_cuv), dim3(BLOCK), 0, st, base_of(B, B->wl_cuv), B->wl_cuv);
+    if (B->n_cuv && (what != 7 || B->cuv_apart)) hipLaunchKernelGGL(k_cuv<R>, dim3(B->n_cuv), dim3(BLOCK), 0, st, base_of(B, B->wl_cuv), B->wl_cuv);
     int tsa_slots = 0;   // timestep analysis of the members that have it on (not while tuning)
     for (sfx_handle* H : B->members)   // (the step kernel's rule leaves members with it to these kernels)
       if (H->hI.tsa_req && !H->tsa_paused) tsa_slots = std::max(tsa_slots, (int)H->hI.nslot);
@@ -3850,11 +3913,11 @@ void launch_phases(sfx_batch* B, int what, int forcing_mode) {
     for (sfx_handle* H : B->members) rx = rx || (H->hI.c.flags & (sfx::F_INFIL | sfx::F_MPRCP | sfx::F_CNA)) != 0;
     auto kc = rx ? k_continuity<R, true> : k_continuity<R, false>;
     if (B->n_cd)
-      hipLaunchKernelGGL(kc, dim3(B->n_cd + lead), dim3(BLOCK), 0, st, base_of(B, B->wl_cd), B->wl_cd, 0,
+      hipLaunchKernelGGL(kc, dim3(B->n_cd + lead), dim3(BLOCK), 0, st, base_of(B, B->wl_cd), B->wl_cd, 0, what == 7,
                          nahead, nbal, B->dInsts, B->dIds);
     if (B->n_ci) {
       const int la = B->n_cd ? 0 : nahead, lb = B->n_cd ? 0 : nbal, ll = B->n_cd ? 0 : lead;
-      hipLaunchKernelGGL(kc, dim3(B->n_ci + ll), dim3(BLOCK), 0, st, base_of(B, B->wl_ci), B->wl_ci, 1,
+      hipLaunchKernelGGL(kc, dim3(B->n_ci + ll), dim3(BLOCK), 0, st, base_of(B, B->wl_ci), B->wl_ci, 1, what == 7,
                          la, lb, B->dInsts, B->dIds);
     }
   }

@@ -2434,8 +2434,15 @@ __device__ __forceinline__ void step_tile(const DevInst* __restrict__ insts, con
   }
 }
 
-template <bool SG>
-__global__ void __launch_bounds__(BLOCK, SG ? 7 : 8) k_step(const DevInst* __restrict__ insts, WorkList L, int flip) {
+// W: the waves a SIMD holds at once. Regular tiles run 8 (64 vector registers). Subgrid ones take
+// fewer instructions with 69 registers, 7 waves, which is quicker while all of a launch's blocks are
+// on the chip at once (STEP_RESIDENT); beyond that the eighth wave is worth more. Measured, ms for
+// the same run with 7 / 8: 161 x 203 cells (519 blocks) 2.79 / 2.86, 512 x 700 (1896) 5.17 / 4.78,
+// 2048 x 2048 (9728) 13.1 / 12.9.
+constexpr int STEP_RESIDENT = 256 * 7;   // blocks: 256 CUs, a wave of each block on each of the 4 SIMDs
+
+template <bool SG, int W>
+__global__ void __launch_bounds__(BLOCK, W) k_step(const DevInst* __restrict__ insts, WorkList L, int flip) {
   int tile, inst;
   if (!work_item(L, blockIdx.x, gridDim.x, tile, inst)) return;
   step_tile<SG>(insts, L, tile, inst, flip);
@@ -2443,8 +2450,8 @@ __global__ void __launch_bounds__(BLOCK, SG ? 7 : 8) k_step(const DevInst* __res
 
 // The same for a batch with both kinds of meshes. Its scenarios wait for nothing of each other, and
 // as two launches the short list left the chip idle around the long one: 8 scenarios of 2 to 160
-// thousand cells took 35 us a step, 27 so. A batch of one kind keeps its own instance (8 regular
-// waves a SIMD against 7 here).
+// thousand cells took 35 us a step, 27 so. 7 waves a SIMD: with 8 it would spill (a 32-step advance
+// of those scenarios 0.89 ms / 1.01).
 __global__ void __launch_bounds__(BLOCK, 7) k_step_mixed(const DevInst* __restrict__ insts, WorkList L, int flip) {
   int tile, inst;
   if (!work_item(L, blockIdx.x, gridDim.x, tile, inst)) return;
@@ -3873,7 +3880,8 @@ void launch_phases(sfx_batch* B, int what, int forcing_mode) {
     size_t lds = 0;
     for (sfx_handle* H : B->members)
       if (H->on_step) lds = std::max(lds, (size_t)(2 * H->hI.frows + 1) * WAVE * sizeof(float));
-    auto ks = B->step_kinds == 3 ? k_step_mixed : (B->step_kinds == 1 ? k_step<true> : k_step<false>);
+    auto ks = B->step_kinds == 3 ? k_step_mixed
+            : B->step_kinds == 2 ? k_step<false, 8> : (B->n_s > (size_t)STEP_RESIDENT ? k_step<true, 8> : k_step<true, 7>);
     hipLaunchKernelGGL(ks, dim3(B->n_s), dim3(BLOCK), lds, st, base_of(B, B->wl_s), B->wl_s, B->flip);
     B->flip ^= 1;
   }

@@ -4126,8 +4126,9 @@ extern "C" int sfx_set_counting(sfx_handle* H, int32_t on) {
   H->hI.count = on ? 1 : 0;
   HIPCHK(hipStreamSynchronize(H->stream));
   HIPCHK(hipMemcpy(H->dI, &H->hI, sizeof(DevInst), hipMemcpyHostToDevice));
-  HIPCHK(hipMemset(H->hI.blkcnt, 0, NCNT * H->nmt_cap * sizeof(uint32_t)));
-  HIPCHK(hipMemset(H->hI.cntstore, 0, NSTORE * std::max<size_t>(1, H->nct_cap) * sizeof(uint32_t)));
+  HIPCHK(hipMemsetAsync(H->hI.blkcnt, 0, NCNT * H->nmt_cap * sizeof(uint32_t), H->stream));
+  HIPCHK(hipMemsetAsync(H->hI.cntstore, 0, NSTORE * std::max<size_t>(1, H->nct_cap) * sizeof(uint32_t), H->stream));
+  HIPCHK(hipStreamSynchronize(H->stream));
   if (H->solo) H->solo->dirty = true;
   return SFX_OK;
 }
@@ -4436,17 +4437,20 @@ int time_phases(sfx_handle* H, int what, int trials, hipEvent_t e0, hipEvent_t e
   return SFX_OK;
 }
 
-// No per-point tile is quiescent (after host writes of state and tile-shape changes).
+// No per-point tile is quiescent (after host writes of state and tile-shape changes). On the handle's
+// stream and finished on return, as all such clears are: no stream of a handle or batch waits for the
+// null stream, and a step that still found a tile quiet would drop what the host wrote.
 int reset_tile_flags(sfx_handle* H) {
-  HIPCHK(hipMemset(H->hI.mq, 0, H->nmt_cap * sizeof(uint32_t)));
-  if (H->stepable) HIPCHK(hipMemset(H->hI.fquiet, 0, (size_t)H->hI.fnt * (BLOCK / WAVE)));
+  HIPCHK(hipMemsetAsync(H->hI.mq, 0, H->nmt_cap * sizeof(uint32_t), H->stream));
+  if (H->stepable) HIPCHK(hipMemsetAsync(H->hI.fquiet, 0, (size_t)H->hI.fnt * (BLOCK / WAVE), H->stream));
+  HIPCHK(hipStreamSynchronize(H->stream));
   return SFX_OK;
 }
 
 // Tile keys back to 0 (after sweeps that were not folded, e.g. timing runs), and no tile
 // quiescent.
 int reset_keys(sfx_handle* H) {
-  HIPCHK(hipMemset(H->hI.blkkey, 0, H->nmt_cap * sizeof(uint32_t)));
+  HIPCHK(hipMemsetAsync(H->hI.blkkey, 0, H->nmt_cap * sizeof(uint32_t), H->stream));
   return reset_tile_flags(H);
 }
 

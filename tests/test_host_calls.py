@@ -1,0 +1,67 @@
+"""Host code of the library without a GPU: libsfx.so on the runtime of fake_hip.cpp, which runs no
+kernel but keeps what was issued on which stream, what the host waited for, and what is allocated.
+Each case runs in a process of its own, where the fake runtime comes before the real one."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C, os, sys
+F = C.CDLL(sys.argv[1], mode=os.RTLD_GLOBAL | os.RTLD_NOW)
+import numpy as np
+from sfincs_amd import _lib
+from sfincs_amd import workloads as W
+F.fake_live.restype = F.fake_launches.restype = F.fake_stale.restype = C.c_long
+F.fake_fail.argtypes = [C.c_long]
+
+def busy():
+    b = C.create_string_buffer(4000)
+    F.fake_busy(b, 4000)
+    F.fake_settle()
+    return b.value.decode()
+
+def regular(n=30, m=41, **kw):
+    return W.regular_case(n, m, seed=1, t_end=4.0e3, **kw).build_model()
+
+def subgrid(n=30, m=41):
+    return W.subgrid_case(n, m, seed=1, t_end=4.0e3, nsrc=2).build_model()
+"""
+
+
+@pytest.fixture(scope="session")
+def fake(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                           "-o", out, os.path.join(HERE, "fake_hip.cpp")])
+    return out
+
+
+def run(fake, body):
+    p = subprocess.run([sys.executable, "-c", PRELUDE + body, fake], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, (p.returncode, p.stdout[-1500:], p.stderr[-1500:])
+    return p.stdout
+
+
+CALLS = ["x.set('zs', x.get('zs'))", "x.set('z_volume', x.get('z_volume'))", "x.set('zsderv', x.get('zsderv'))",
+         "x.set('q', x.get('q'))", "x.set('kfuv', x.get('kfuv'))", "x.set_counting(True)", "x.set_counting(False)",
+         "x.compute_fluxes(1.0)", "x.autotune(1)", "x.set_tuning(-1, (32, 8), (64, 4))"]
+
+
+def test_nothing_is_in_flight_on_return(fake):
+    """A handle may be in a batch, which runs on another stream: what a call issued is finished when
+    it returns, on the handle's stream and on the null stream, for which no stream waits."""
+    left = run(fake, f"""
+x = _lib.Instance(subgrid())
+for call in {CALLS!r}:
+    x.update(0.0)
+    assert busy() == ''
+    exec(call)
+    left = busy()
+    if left: print(call, '|', left)
+""")
+    assert left == "", left

@@ -4096,7 +4096,11 @@ int update_loop(sfx_handle* H, int mode, double arg, sfx_step_stats* st) {
     s = H->hs;
     if (single || !s.active || s.error || s.error_pending || !(s.t < s.tend)) break;
   }
-  if (s.error_pending) { s.error = 1; s.error_pending = 0; s.t = (double)H->hI.c.t1 + 1.0; if ((rc = write_scalars(H, s))) return rc; }
+  if (s.error_pending) {
+    s.error = 1; s.error_pending = 0; s.t = (double)H->hI.c.t1 + 1.0;
+    if ((rc = write_scalars(H, s))) return rc;
+    HIPCHK(hipStreamSynchronize(H->stream));
+  }
   if (st) {
     st->t = s.t; st->dt = s.dt; st->min_dt = s.min_dt; st->nt = s.nt; st->error = s.error;
     st->cell_updates = (double)(s.nt - nt0) * (double)H->hI.np;
@@ -4663,6 +4667,8 @@ extern "C" int sfx_profile_steps(sfx_handle* H, int32_t nsteps, double ms[3]) {
     }
   }
   end_steps(B);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(H->stream));   // a batch of this handle's runs on its own stream
   H->hs_ok = false;
   for (auto& e : ev) hipEventDestroy(e);
   for (int k = 0; k < 3; ++k) ms[k] = acc[k] / nsteps;

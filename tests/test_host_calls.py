@@ -47,21 +47,24 @@ def run(fake, body):
     return p.stdout
 
 
-CALLS = ["x.set('zs', x.get('zs'))", "x.set('z_volume', x.get('z_volume'))", "x.set('zsderv', x.get('zsderv'))",
+CALLS = ["x.profile(1)", "x.profile(2)", "x.set('zs', x.get('zs'))", "x.set('z_volume', x.get('z_volume'))",
+         "x.set('zsderv', x.get('zsderv'))",
          "x.set('q', x.get('q'))", "x.set('kfuv', x.get('kfuv'))", "x.set_counting(True)", "x.set_counting(False)",
-         "x.compute_fluxes(1.0)", "x.autotune(1)", "x.set_tuning(-1, (32, 8), (64, 4))"]
+         "x.compute_fluxes(1.0)", "x.autotune(1)", "b.add(x, 50.0)", "b.advance(3)", "b.done(x)",
+         "b.remove(x)", "F.fake_ones(1); x.update(50.0); F.fake_ones(0)", "x.set_tuning(-1, (32, 8), (64, 4))"]
 
 
 def test_nothing_is_in_flight_on_return(fake):
     """A handle may be in a batch, which runs on another stream: what a call issued is finished when
     it returns, on the handle's stream and on the null stream, for which no stream waits."""
     left = run(fake, f"""
-x = _lib.Instance(subgrid())
+x, b = _lib.Instance(subgrid()), _lib.Batch()
 for call in {CALLS!r}:
-    x.update(0.0)
+    if not x._nbatch: x.update(0.0)
     assert busy() == ''
     exec(call)
     left = busy()
     if left: print(call, '|', left)
+assert F.fake_launches(b'k_step_scalars') > 0      # an odd number of steps was profiled
 """)
     assert left == "", left

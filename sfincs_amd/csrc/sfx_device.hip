@@ -4605,32 +4605,35 @@ extern "C" int sfx_autotune(sfx_handle* H, int32_t trials) {
     if (!rc && ms < best) { best = ms; bxc = chunks[k]; }
   }
   H->hI.xchunk_c = bxc;
-  // the step kernel against the separate kernels, forcing included
+  H->tile_tn = H->hI.tn; H->tile_tm = H->hI.tm; H->strip_rows = H->hI.sk;
+  H->mtile_tn = H->hI.mtn; H->mtile_tm = H->hI.mtm; H->xchunk = H->hI.xchunk; H->xchunk_c = H->hI.xchunk_c;
+  // the scenario as it was, with these scalars; the handle's own descriptor, with which finished sweeps
+  // are completed and marks cleared, has the chosen shapes
+  auto restore = [&](const Scalars& at) -> int {
+    HIPCHK(hipMemcpy(H->dI, &H->hI, sizeof(DevInst), hipMemcpyHostToDevice));
+    int r;
+    if ((r = write_scalars(H, at)) || (r = reset_keys(H))) return r;
+    for (auto& f : fields)
+      if ((r = sfx_set_state(H, f.c_str(), snap[f].data(), snap[f].size()))) return r;
+    HIPCHK(hipMemcpy(H->hI.bal, bal_keep, sizeof(bal_keep), hipMemcpyHostToDevice));
+    if (!um.empty()) HIPCHK(hipMemcpy(H->hI.uvmean, um.data(), um.size(), hipMemcpyHostToDevice));
+    if (H->solo) H->solo->dirty = true;
+    return SFX_OK;
+  };
+  // the step kernel against the separate kernels, forcing included, each from the scenario's own state
   if (H->stepable && !rc) {
     float apart = 0.f, step = 0.f;
     H->use_step = false;
-    rc = time_phases(H, 7, trials, e0, e1, apart);
+    if (!(rc = restore(s))) rc = time_phases(H, 7, trials, e0, e1, apart);
     H->use_step = true;
-    if (!rc) rc = enter_step(H);
-    if (!rc) rc = time_phases(H, 7, trials, e0, e1, step);
+    if (!rc && !(rc = restore(s)) && !(rc = enter_step(H))) rc = time_phases(H, 7, trials, e0, e1, step);
     end_steps(solo(H));
     if (!rc) rc = enter_general(H);
     H->use_step = !rc && step <= apart;
   }
   hipEventDestroy(e0);
   hipEventDestroy(e1);
-  if (rc) return rc;
-  HIPCHK(hipMemcpy(H->dI, &H->hI, sizeof(DevInst), hipMemcpyHostToDevice));
-  H->tile_tn = H->hI.tn; H->tile_tm = H->hI.tm; H->strip_rows = H->hI.sk;
-  H->mtile_tn = H->hI.mtn; H->mtile_tm = H->hI.mtm; H->xchunk = H->hI.xchunk; H->xchunk_c = H->hI.xchunk_c;
-  if ((rc = write_scalars(H, s0))) return rc;
-  if ((rc = reset_keys(H))) return rc;
-  for (auto& f : fields)
-    if ((rc = sfx_set_state(H, f.c_str(), snap[f].data(), snap[f].size()))) return rc;
-  HIPCHK(hipMemcpy(H->hI.bal, bal_keep, sizeof(bal_keep), hipMemcpyHostToDevice));
-  if (!um.empty()) HIPCHK(hipMemcpy(H->hI.uvmean, um.data(), um.size(), hipMemcpyHostToDevice));
-  if (H->solo) H->solo->dirty = true;
-  return SFX_OK;
+  return rc ? rc : restore(s0);
 }
 
 // -------------------------------------------------------------------------- profiling

@@ -68,3 +68,16 @@ for call in {CALLS!r}:
 assert F.fake_launches(b'k_step_scalars') > 0      # an odd number of steps was profiled
 """)
     assert left == "", left
+
+
+def test_autotune_moves_between_kernels_on_the_chosen_shapes(fake):
+    """Sweeps that autotune completes are completed with the tiles they ran on: the handle's own
+    descriptor is the one its trials were launched with."""
+    run(fake, """
+x = _lib.Instance(subgrid(130, 70))
+x.update(0.0)
+n = F.fake_launches(b'k_give_scalars')
+x.autotune(1)
+assert F.fake_launches(b'k_step') > 0 and F.fake_launches(b'k_give_scalars') > n
+assert F.fake_stale() == 0, F.fake_stale()
+""")

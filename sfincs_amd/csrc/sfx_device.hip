@@ -4552,6 +4552,8 @@ extern "C" int sfx_autotune(sfx_handle* H, int32_t trials) {
   if ((rc = write_scalars(H, s))) return rc;
   std::vector<char> um((size_t)H->sz.nkcuv2 * (H->fp64 ? 8 : 4));   // whole steps are timed too
   if (!um.empty()) HIPCHK(hipMemcpy(um.data(), H->hI.uvmean, um.size(), hipMemcpyDeviceToHost));
+  std::vector<float> qs((size_t)H->hI.nsrc);   // and work out discharges, which stay as they are past the series' end
+  if (!qs.empty()) HIPCHK(hipMemcpy(qs.data(), H->hI.qtsrc, qs.size() * sizeof(float), hipMemcpyDeviceToHost));
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
@@ -4617,6 +4619,7 @@ extern "C" int sfx_autotune(sfx_handle* H, int32_t trials) {
       if ((r = sfx_set_state(H, f.c_str(), snap[f].data(), snap[f].size()))) return r;
     HIPCHK(hipMemcpy(H->hI.bal, bal_keep, sizeof(bal_keep), hipMemcpyHostToDevice));
     if (!um.empty()) HIPCHK(hipMemcpy(H->hI.uvmean, um.data(), um.size(), hipMemcpyHostToDevice));
+    if (!qs.empty()) HIPCHK(hipMemcpy(H->hI.qtsrc, qs.data(), qs.size() * sizeof(float), hipMemcpyHostToDevice));
     if (H->solo) H->solo->dirty = true;
     return SFX_OK;
   };

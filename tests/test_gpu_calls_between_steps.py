@@ -45,3 +45,28 @@ def test_profiled_steps_of_a_batch_member(steps):
             y.update(0.0)
     b.close()
     _same(x, y, m, steps)
+
+
+@pytest.mark.parametrize("at", [150.0, 400.0])
+def test_autotune_leaves_the_scenario_as_it_was(at):
+    """Every field and the sums of the volume balance are the bits from before, the discharges too, inside
+    their series and past its end, where the next steps keep them; the steps after are those of a
+    scenario that was not tuned. (The balance's volume is no state: each call adds it up anew, in an
+    order that is not fixed.)"""
+    sc = W.subgrid_case(66, 70, seed=5, t_end=4.0e3, nsrc=2)
+    sc.params["t1"] = 1.0e7
+    px, py, _, q = sc.src
+    sc.src = (px, py, np.array([0.0, 290.0], np.float32), np.stack([q[0] + 1.0, q[0] + 40.0]).astype(np.float32))
+    m = sc.build_model()
+    x, y = _lib.Instance(m), _lib.Instance(m)
+    for i in (x, y):
+        i.update_to(at)
+    before = {f: x.get(f).tobytes() for f in _fields(m)}
+    sums = ("boundary", "sources", "rain", "qext")
+    balance = [x.balance()[k] for k in sums]
+    x.autotune(2)
+    assert [f for f in before if x.get(f).tobytes() != before[f]] == []
+    assert [x.balance()[k] for k in sums] == balance
+    for i in (x, y):
+        i.update_to(at + 60.0)
+    _same(x, y, m, at)

@@ -4624,7 +4624,8 @@ extern "C" int sfx_autotune(sfx_handle* H, int32_t trials) {
     return SFX_OK;
   };
   // the step kernel against the separate kernels, forcing included, each from the scenario's own state
-  if (H->stepable && !rc) {
+  // (while counting is on every step takes the separate kernels and there is nothing to choose by)
+  if (H->stepable && !H->hI.count && !rc) {
     float apart = 0.f, step = 0.f;
     H->use_step = false;
     if (!(rc = restore(s))) rc = time_phases(H, 7, trials, e0, e1, apart);

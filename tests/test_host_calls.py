@@ -81,3 +81,17 @@ x.autotune(1)
 assert F.fake_launches(b'k_step') > 0 and F.fake_launches(b'k_give_scalars') > n
 assert F.fake_stale() == 0, F.fake_stale()
 """)
+
+
+def test_autotune_while_counting_keeps_the_choice_of_kernel(fake):
+    """With counting on, steps run on the separate kernels only, so no trial of theirs decides against
+    the step kernel (the fake clock calls every later trial slower)."""
+    run(fake, """
+for pin in (-8, -1):
+    x = _lib.Instance(subgrid())
+    x.set_tuning(pin, (32, 8), (64, 4))
+    x.set_counting(True)
+    assert x.autotune(1)['momentum_kernel'] == -8 if pin == -8 else x.autotune(1)['momentum_kernel'] != -8
+x = _lib.Instance(subgrid())
+assert x.autotune(1)['momentum_kernel'] != -8
+""")

@@ -698,6 +698,8 @@ __device__ void step_series(const DevInst& I, StepImage& F, float* qout, int mod
     itsel = __shfl(itsel, 0, WAVE);
     if (itsel)
       for (int src = lane; src < I.nsrc; src += WAVE) G(qout)[src] = source_at(I, t, itsel, src);
+    else if (qout != I.qtsrc)   // they stay; the staged ones may be older (the step kernel, a forcing call)
+      for (int src = lane; src < I.nsrc; src += WAVE) G(qout)[src] = G(I.qtsrc)[src];
   }
   __syncthreads();
 }

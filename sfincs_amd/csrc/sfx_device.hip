@@ -20,6 +20,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
 #include <string>
@@ -3327,7 +3328,7 @@ int staged_out(sfx_handle* H, void* dst, size_t n, Put put) {
     return SFX_OK;
   }
   const size_t pieces = (n + STAGE - 1) / STAGE;
-  const int T = n >= STAGE_PAR ? STAGE_THREADS : 1;
+  int T = 1;   // threads that move the pieces; the helpers read it after the first one is ready
   std::atomic<size_t> ready{0}, done{0};
   std::atomic<bool> stop{false};
   auto move = [&](int t, size_t k) {   // thread t's share of piece k
@@ -3335,17 +3336,22 @@ int staged_out(sfx_handle* H, void* dst, size_t n, Put put) {
     std::memcpy((char*)dst + k * STAGE + lo, buf + (k % NSTAGE) * STAGE + lo, hi - lo);
     done.fetch_add(1, std::memory_order_release);
   };
-  std::vector<std::thread> help;
-  for (int t = 1; t < T; ++t)
-    help.emplace_back([&, t] {
-      for (size_t k = 0; k < pieces; ++k) {
-        while (ready.load(std::memory_order_acquire) <= k) {
-          if (stop.load()) return;
-          std::this_thread::yield();
-        }
-        move(t, k);
+  auto follow = [&](int t) {
+    for (size_t k = 0; k < pieces; ++k) {
+      while (ready.load(std::memory_order_acquire) <= k) {
+        if (stop.load()) return;
+        std::this_thread::yield();
       }
-    });
+      move(t, k);
+    }
+  };
+  std::thread help[STAGE_THREADS];
+  if (n >= STAGE_PAR) {
+    try {
+      for (; T < STAGE_THREADS; ++T) help[T] = std::thread(follow, T);
+    } catch (const std::exception&) {   // no more threads (or memory) to be had: those that started do it
+    }
+  }
   hipError_t e = hipSuccess;
   size_t issued = 0;
   for (size_t k = 0; k < pieces && e == hipSuccess; ++k) {
@@ -3360,7 +3366,7 @@ int staged_out(sfx_handle* H, void* dst, size_t n, Put put) {
     while (done.load(std::memory_order_acquire) < (size_t)T * (k + 1)) std::this_thread::yield();
   }
   stop.store(true);
-  for (auto& t : help) t.join();
+  for (int t = 1; t < T; ++t) help[t].join();
   HIPCHK(e);
   return SFX_OK;
 }

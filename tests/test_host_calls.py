@@ -95,3 +95,22 @@ for pin in (-8, -1):
 x = _lib.Instance(subgrid())
 assert x.autotune(1)['momentum_kernel'] != -8
 """)
+
+
+def test_reads_go_on_without_helper_threads(fake):
+    """A read of 8 MB takes helper threads; where none can be started (here: no address space for
+    their stacks) the calling thread moves the pieces alone."""
+    run(fake, """
+import resource
+x = _lib.Instance(regular(1000, 1050))
+zs = np.arange(1050000, dtype=np.float64)
+x.set('zs', zs)
+out = [np.zeros_like(zs), np.zeros_like(zs)]
+def read(a):
+    return _lib.lib().sfx_get_state(x.h, b'zs', a.ctypes.data_as(C.c_void_p), C.c_size_t(a.nbytes))
+size = int(open('/proc/self/statm').read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (size + (4 << 20), -1))     # a stack takes 8 MB
+assert read(out[0]) == 0 and np.array_equal(out[0], zs)
+resource.setrlimit(resource.RLIMIT_AS, (-1, -1))
+assert read(out[1]) == 0 and np.array_equal(out[1], zs)
+""")

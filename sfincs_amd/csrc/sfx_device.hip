@@ -2632,6 +2632,7 @@ struct sfx_handle {
   DevInst* dI = nullptr;
   Scalars* dS = nullptr;
   std::vector<void*> allocs;
+  bool alloc_failed = false;
   std::vector<int32_t> ref2slot;   // reference uv index (0-based, incl. cuv and dummy) -> slot
   int32_t nslot = 0;
   hipStream_t stream = nullptr;
@@ -2660,7 +2661,7 @@ struct sfx_handle {
 template <typename T> T* sfx_handle::alloc(size_t n) {
   void* p = nullptr;
   if (n == 0) n = 1;
-  if (hipMalloc(&p, n * sizeof(T)) != hipSuccess) return nullptr;
+  if (hipMalloc(&p, n * sizeof(T)) != hipSuccess) { alloc_failed = true; return nullptr; }
   (void)hipMemset(p, 0, n * sizeof(T));
   allocs.push_back(p);
   return (T*)p;
@@ -3075,7 +3076,7 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
     I.wnddir = H->upload(M->wnddir.data(), M->wnddir.size()); I.cdval = H->upload(M->cdval.data(), M->cdval.size());
     I.x73 = H->upload(M->x73.data(), M->x73.size());
     std::string perr;
-    if (!sfx::pow_tables_device(device, I.pw, perr)) { set_error(perr); delete H; return SFX_ERR_STATE; }
+    if (!sfx::pow_tables_device(device, I.pw, perr)) { set_error(perr); sfx_destroy(H); return SFX_ERR_STATE; }
   }
   rc = H->fp64 ? upload_state<double>(H, M) : upload_state<float>(H, M);
   // scalars
@@ -3157,11 +3158,19 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
   if (hipHostMalloc((void**)&H->pin, sizeof(Scalars)) != hipSuccess) H->pin = nullptr;
   stage_open(H);
   H->hs = s; H->hs_ok = true;
-  H->allocs.push_back(H->pin);   // checked with the rest, freed apart
-  for (void* p : H->allocs) if (!p) { set_error("hipMalloc failed"); return SFX_ERR_MEMORY; }
-  H->allocs.pop_back();
-  HIPCHK(hipDeviceSynchronize());
-  HIPCHK(hipStreamCreateWithFlags(&H->stream, hipStreamNonBlocking));
+  if (H->alloc_failed || !H->pin) {
+    (void)hipGetLastError();   // the allocation's, reported here
+    set_error("hipMalloc failed");
+    sfx_destroy(H);   // with what it has so far
+    return SFX_ERR_MEMORY;
+  }
+  const hipError_t e = hipDeviceSynchronize();
+  if (e != hipSuccess || hipStreamCreateWithFlags(&H->stream, hipStreamNonBlocking) != hipSuccess) {
+    set_error(std::string("sfx_create: ") + hipGetErrorString(e != hipSuccess ? e : hipGetLastError()));
+    H->stream = nullptr;
+    sfx_destroy(H);
+    return SFX_ERR_HIP;
+  }
   *out = H;
   return rc;
 }

@@ -114,3 +114,32 @@ assert read(out[0]) == 0 and np.array_equal(out[0], zs)
 resource.setrlimit(resource.RLIMIT_AS, (-1, -1))
 assert read(out[1]) == 0 and np.array_equal(out[1], zs)
 """)
+
+
+def test_a_failed_create_keeps_nothing(fake):
+    """Whichever allocation fails, device or pinned, the call says so and gives back what it had; the
+    buffers that handles share are given back with the last of them, failed ones not counted."""
+    run(fake, """
+m = subgrid()
+_lib.Instance(m).close()                 # the tables that stay
+live = lambda: (F.fake_live(0), F.fake_live(1))
+base = live()
+x = _lib.Instance(m)
+n = sum(live()) - sum(base)
+x.close()
+assert live() == base and n > 40
+for k in range(1, n + 1):
+    F.fake_fail(k)
+    try:
+        _lib.Instance(m)
+        raise SystemExit('allocation %d: no error' % k)
+    except _lib.SfxError as e:
+        assert 'hipMalloc failed' in str(e), (k, e)
+    assert live() == base, (k, live(), base)
+F.fake_fail(0)
+x = _lib.Instance(m)
+x.get('zs')
+assert F.fake_live(1) > base[1] + 1      # the shared buffers are there
+x.close()
+assert live() == base, (live(), base)
+""")

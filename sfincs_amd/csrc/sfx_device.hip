@@ -3307,15 +3307,20 @@ void stage_close(sfx_handle* H) {
   hipHostFree(S.buf);
   S.buf = nullptr;
 }
-// With S.mu held: its buffers, or null when they cannot be had (the caller copies directly).
+// With S.mu held: its buffers, or null when they cannot be had (the caller copies directly, and the
+// runtime's record of the failed call is taken back, or the next check of a launch would find it).
 char* stage_buf(Stage& S) {
   if (S.buf) return S.buf;
   char* b = nullptr;
-  if (hipHostMalloc((void**)&b, NSTAGE * STAGE) != hipSuccess) return nullptr;
+  if (hipHostMalloc((void**)&b, NSTAGE * STAGE) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
   for (int k = 0; k < NSTAGE; ++k)
     if (hipEventCreateWithFlags(&S.ev[k], hipEventDisableTiming) != hipSuccess) {
       while (k-- > 0) { hipEventDestroy(S.ev[k]); S.ev[k] = nullptr; }
       hipHostFree(b);
+      (void)hipGetLastError();
       return nullptr;
     }
   return S.buf = b;

@@ -22,6 +22,7 @@ std::map<void*, size_t> device, pinned;
 std::map<std::string, long> launches;
 long fail_in = 0, stale = 0, clock_ms = 0;
 bool ones = false, capturing = false;
+thread_local hipError_t last = hipSuccess;   // until it is asked for, as the real one
 std::map<size_t, std::pair<void*, std::vector<char>>> copied;   // by size: the last copy to the device
 
 struct Call { dim3 grid, block; size_t lds; hipStream_t stream; };
@@ -34,7 +35,7 @@ void issue(hipStream_t s, const std::string& what) {
 }
 hipError_t take(void** p, size_t n, std::map<void*, size_t>& in) {
   std::lock_guard<std::mutex> lk(mu);
-  if (fail_in > 0 && --fail_in == 0) return hipErrorOutOfMemory;
+  if (fail_in > 0 && --fail_in == 0) return last = hipErrorOutOfMemory;
   if (!(*p = std::calloc(n, 1))) return hipErrorOutOfMemory;
   in[*p] = n;
   return hipSuccess;
@@ -86,7 +87,7 @@ hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "fake error"; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() { const hipError_t e = last; last = hipSuccess; return e; }
 hipError_t hipGetSymbolAddress(void** p, const void*) { static char room[1 << 16]; *p = room; return hipSuccess; }
 
 hipError_t hipMalloc(void** p, size_t n) { return take(p, n, device); }

@@ -143,3 +143,21 @@ assert F.fake_live(1) > base[1] + 1      # the shared buffers are there
 x.close()
 assert live() == base, (live(), base)
 """)
+
+
+def test_reads_and_writes_without_pinned_memory(fake):
+    """Where the shared pinned buffers cannot be had, state is copied directly, and the failed
+    allocation is no error of this call or of the next."""
+    run(fake, """
+x = _lib.Instance(regular())
+zs = np.linspace(0.0, 1.0, x.sizes['np'])
+F.fake_fail(1)
+x.set('zs', zs)
+x.update_forcing(1.0, 1.0)
+F.fake_fail(1)
+assert np.array_equal(x.get('zs'), zs)
+x.update_forcing(2.0, 1.0)
+pins = F.fake_live(1)
+x.get('zs')
+assert F.fake_live(1) == pins + 1        # tried again
+""")

@@ -430,8 +430,9 @@ int  sfx_autotune(sfx_handle* h, int32_t trials);
  *        per XCD)} */
 int  sfx_get_tuning(sfx_handle* h, int32_t out[8]);
 /* Pins the dense shapes without timing: in = {momentum kernel as above, momentum tile n,
- * momentum tile m, continuity tile n, continuity tile m}; tiles hold 256 cells. No effect
- * on indexed meshes. Call it before the handle joins a batch. */
+ * momentum tile m, continuity tile n, continuity tile m}; tiles hold 256 cells. -8 on a
+ * scenario that may not use the step kernel keeps its momentum kernel and sets the tiles. No
+ * effect on indexed meshes. Call it before the handle joins a batch. */
 int  sfx_set_tuning(sfx_handle* h, const int32_t in[5]);
 /* Pins the work-list order without timing: the runs of tiles dealt to the XCDs in turn,
  * for the momentum and the continuity sweep (out[6], out[7] of sfx_get_tuning; 0: one

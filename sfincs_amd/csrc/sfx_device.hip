@@ -4494,12 +4494,14 @@ void set_shapes(sfx_handle* H, int sk, int mtn, int mtm, int tn, int tm) {
 
 extern "C" int sfx_set_tuning(sfx_handle* H, const int32_t in[5]) {
   if (!H || !in) { set_error("null"); return SFX_ERR_ARG; }
+  // the step kernel where the scenario may use it; elsewhere (a tuning taken from a run with the default
+  // physics) its number leaves the separate kernel as it is
   const bool step = in[0] == STEP_KERNEL && H->stepable;
-  const int sk = step ? H->hI.sk : in[0], mtn = in[1], mtm = in[2], tn = in[3], tm = in[4];
+  const int sk = in[0] == STEP_KERNEL ? H->hI.sk : in[0], mtn = in[1], mtm = in[2], tn = in[3], tm = in[4];
   const bool sk_ok = sk == -1 || sk == -2 || sk == -4 || (sk >= 0 && sk <= 256);
   if (!sk_ok || mtn <= 0 || mtm <= 0 || mtn * mtm != BLOCK || tn <= 0 || tm <= 0 || tn * tm != BLOCK) {
-    set_error("sfx_set_tuning: the momentum kernel must be -1, -2, -4 (per-point), 0 (per-cell) or 1..256 strip rows, "
-              "and tiles must hold 256 cells");
+    set_error("sfx_set_tuning: the momentum kernel must be -8 (the step kernel), -1, -2, -4 (per-point), 0 (per-cell) "
+              "or 1..256 strip rows, and tiles must hold 256 cells");
     return SFX_ERR_ARG;
   }
   if (H->in_batches) { set_error("sfx_set_tuning: set shapes before adding the scenario to a batch"); return SFX_ERR_STATE; }

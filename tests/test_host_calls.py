@@ -161,3 +161,31 @@ pins = F.fake_live(1)
 x.get('zs')
 assert F.fake_live(1) == pins + 1        # tried again
 """)
+
+
+def test_a_tuning_can_be_pinned_on_any_run_of_the_mesh(fake):
+    """What tuning() reports for a default run (the step kernel) is accepted by the same mesh with
+    wind, by its FP64 twin and by an indexed mesh, which keep a kernel of their own; other unknown
+    numbers are refused as ever."""
+    run(fake, """
+d = _lib.Instance(regular()).tuning()
+assert d['momentum_kernel'] == -8
+two = np.array([0.0, 1.0e5], np.float32)
+wind = regular(wind=(two, np.full(2, 12.0, np.float32), np.full(2, 200.0, np.float32)))
+for x in (_lib.Instance(wind), _lib.Instance(regular(), fp64=True), _lib.Instance(W.quadtree_case(5, 5, nlev=2).build_model())):
+    own = x.tuning()['momentum_kernel']
+    assert own != -8
+    x.pin_tuning(d)
+    assert x.tuning()['momentum_kernel'] == own
+    for bad in (-3, -7, -9, 257):
+        try:
+            x.set_tuning(bad, (32, 8), (64, 4))
+            raise SystemExit('accepted %d' % bad)
+        except _lib.SfxError as e:
+            assert '-8' in str(e)
+x = _lib.Instance(regular())
+x.set_tuning(-1, (32, 8), (64, 4))
+assert x.tuning()['momentum_kernel'] == -1
+x.pin_tuning(d)
+assert x.tuning()['momentum_kernel'] == -8
+""")

@@ -113,34 +113,33 @@ SFX_HD inline double pow_estimate(float x, int which) {
 // z0 = x^(-1/3) to about 2^-19.7 (the log2 of x, at most 128 in magnitude, is rounded to f32), and
 // one third-order step z = z0 (1 + r/3 + 2 r^2/9), r = 1 - x z0^3, leaves 14 r^3/81 < 2^-56: z0^2
 // is exact in f64, so the cube root takes six f64 operations and no range reduction. The float
-// exponents' offsets from 1/3, 5/3 and 7/3 (at most 8e-8) multiply by 1 + t + t^2/2, t = d ln x,
-// from the same log2: in f32 for 1/3 (t < 2.8e-7 over the table range, so 2^-45 of the result), in
-// f64 for the others. The rounding decisions need it within 2^-40 of the exact power: a device
-// test checks it against pow_estimate (itself verified within 2^-44 of pow for every table input)
-// for every float of [2^-40, 2^14) and each exponent. The power is the largest single piece of a
-// wet point's arithmetic (67 of about 450 vector instructions with the polynomial and two Newton
-// steps of pow_estimate, 33 here).
+// exponents' offsets from 1/3, 5/3 and 7/3 (at most 8e-8) add t + t^2/2, t = d ln x, in f64: the
+// exponent exactly, the mantissa's log2 from the hardware on [1, 2). Largest relative error
+// against the 64-bit power over every float of [2^-40, 2^14): 1.42e-15 for 1/3, 4.47e-15 for 5/3
+// and 7.67e-15 for 7/3 (1.47e-15, 4.47e-15 and 7.74e-15 with the polynomial and two Newton steps
+// of pow_estimate); with t in f32 from the rounded log2, 3.8e-14 for 1/3. The rounding decisions
+// need it within 2^-40 of the exact power: a device test checks it against pow_estimate (itself
+// verified within 2^-44 of pow for every table input) for every float of [2^-40, 2^14) and each
+// exponent. The power is the largest single piece of the about 450 vector instructions of a
+// wet point: 28, against 62 of the polynomial and two Newton steps.
 __device__ inline double pow_estimate_dev(float x, int which) {
   if (which == 3) return (double)x * sqrt((double)x);
   if (f2u(x) < 0x00800000u) return pow_estimate(x, which);
   const float xf = x < 3.4028234663852886e38f ? x : 3.4028234663852886e38f;
-  const float L = (float)__builtin_amdgcn_frexp_expf(xf) + __builtin_amdgcn_logf(__builtin_amdgcn_frexp_mantf(xf));
+  const uint32_t b = f2u(xf);
+  const int e = (int)(b >> 23) - 127;
+  const float lm = __builtin_amdgcn_logf(u2f((b & 0x7fffffu) | 0x3f800000u)), L = (float)e + lm;
   const double xd = (double)xf, z0 = (double)__builtin_amdgcn_exp2f(L * (-1.0f / 3.0f));
   const double r = fma(-(xd * (z0 * z0)), z0, 1.0);
   const double z = fma(z0 * r, fma(r, 2.0 / 9.0, 1.0 / 3.0), z0);
   const double y = xd * z * z;
-  if (which == 0) {
-    const float t = L * (float)(((double)(1.0f / 3.0f) - 1.0 / 3.0) * 0.69314718055994530942);
-    return fma(y, (double)__builtin_fmaf(0.5f * t, t, t), y);
-  }
-  const double lnx = ((double)__builtin_amdgcn_frexp_expf(xf) + (double)__builtin_amdgcn_logf(__builtin_amdgcn_frexp_mantf(xf))) *
-                     0.69314718055994530942;
-  const double d53 = (double)(5.0f / 3.0f) - 5.0 / 3.0;
-  const double d73 = (double)(7.0f / 3.0f) - 7.0 / 3.0;
-  const double t = (which == 1 ? d53 : d73) * lnx;
-  const double corr = fma(t, fma(0.5, t, 1.0), 1.0);
-  if (which == 1) return xd * y * y * corr;
-  return xd * xd * y * corr;
+  const double ln2 = 0.69314718055994530942;   // d ln 2 of each exponent is one constant
+  const double d13 = ((double)(1.0f / 3.0f) - 1.0 / 3.0) * ln2;
+  const double d53 = ((double)(5.0f / 3.0f) - 5.0 / 3.0) * ln2;
+  const double d73 = ((double)(7.0f / 3.0f) - 7.0 / 3.0) * ln2;
+  const double t = ((double)e + (double)lm) * (which == 0 ? d13 : (which == 1 ? d53 : d73));
+  const double p = which == 0 ? y : (which == 1 ? xd * y * y : xd * xd * y);
+  return fma(p, fma(0.5 * t, t, t), p);
 }
 
 // True when the double value r lies within 2^-32 (relative) of a midpoint between two

@@ -117,3 +117,19 @@ def test_device_estimate_is_within_its_bound_for_every_table_input(which):
     worst = out[1:2].view(np.float64)[0]
     print("estimate", which, "beyond 2^-44:", int(out[0]), "largest relative difference", worst, flush=True)
     assert out[0] == 0 and worst < 2.0 ** -44
+
+
+@pytest.mark.gpu
+def test_device_cube_root_estimate_is_as_close_as_its_double_steps_allow():
+    """The estimate for x^(1/3) takes the float exponent's offset from 1/3 (1e-8) in double: an error of
+    2^-23 in the hardware's log2 of the mantissa makes 2^-49.6 of the power, and the last few double
+    operations stay below 2^-51, so it lies within 2^-49 of the power and within 2^-46 + 2^-49 of
+    pow_estimate, which is within 2^-46. With the offset in float it was 2^-44.6 off."""
+    L = _lib.lib()
+    f = L.sfx_libm_estimate_check
+    f.argtypes = [C.c_int32, C.c_void_p]
+    f.restype = C.c_int
+    out = np.zeros(2, np.uint64)
+    _lib.check(f(0, out.ctypes.data), "libm_estimate_check")
+    worst = out[1:2].view(np.float64)[0]
+    assert worst < 2.0 ** -46 + 2.0 ** -49, worst

@@ -2840,13 +2840,19 @@ int upload_state(sfx_handle* H, const sfx_model* M) {
 }  // namespace
 
 // -------------------------------------------------------------------------- create / destroy
+namespace {
+bool step_rule(const sfx::Consts& c, const sfx_model* M);
+}
+
 extern "C" int sfx_model_footprint(const sfx_model* M, size_t* bytes) {
   if (!M || !bytes) { set_error("sfx_model_footprint: null"); return SFX_ERR_ARG; }
   const size_t np = M->np, nslot = M->dense ? 2 * (size_t)M->np : (size_t)(M->npuv + M->ncuv);
   size_t b = np * (8 + 4 * 3 + 1) + nslot * (4 * 4 + 3);
   if (M->subgrid) b += np * (8 + 12 + 4 * (size_t)M->nl) + nslot * (4 + 16 + 4 + 16 * (size_t)M->nl);
   else b += np * 4 + nslot * 8;
-  if (M->dense) b += np * (8 + (M->subgrid ? 12 : 0)) + nslot;   // the step kernel's second side
+  sfx::Consts c{};
+  if (M->initialized && fill_consts(M, c) == SFX_OK && step_rule(c, M))   // the step kernel's second side
+    b += np * (8 + (M->subgrid ? 12 : 0)) + nslot;
   if (!M->dense) b += (size_t)M->npuv * (40 + 1) + np * 17 + (size_t)M->ncuv * 12;
   *bytes = b + (1 << 20);
   return SFX_OK;
@@ -2855,7 +2861,6 @@ extern "C" int sfx_model_footprint(const sfx_model* M, size_t* bytes) {
 namespace {
 void stage_open(sfx_handle* H);
 void stage_close(sfx_handle* H);
-bool step_rule(const DevInst& I, const sfx_model* M);
 void build_step(sfx_handle* H, const sfx_model* M, const std::vector<int32_t>& bf, const std::vector<double>& coef);
 }
 
@@ -3149,7 +3154,7 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
     for (int k = 0; k < 2; ++k) {
       I.zs_s[k] = I.zs; I.vol_s[k] = I.vol; I.zsd_s[k] = (float*)I.zsderv; I.kf_s[k] = I.kfuv; I.um_s[k] = (float*)I.uvmean;
     }
-    H->stepable = step_rule(I, M);
+    H->stepable = !H->fp64 && step_rule(I.c, M);
     H->use_step = H->stepable;
     if (H->stepable) build_step(H, M, slot, coef);
     H->bnd_recs = {};
@@ -3176,13 +3181,13 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
 }
 
 namespace {
-// Whether a scenario may take its steps in one launch each (k_step): a full rectangle in FP32
-// with the default physics, whose boundary is made of flux points only (no Neumann copies, no
-// weirs, no drainage structures), driven by uniform rain, discharges and external sources at
-// most. Everything else takes the separate kernels.
-bool step_rule(const DevInst& I, const sfx_model* M) {
-  return I.dense && !I.fp64 && sfx::std_physics(I.c) && I.n6 == 0 && I.ndrn == 0 && M->structure_uv_index.empty() &&
-         (size_t)M->mmax * (size_t)M->nmax < ((size_t)1 << 30);
+// Whether an FP32 scenario may take its steps in one launch each (k_step): a full rectangle with the
+// default physics, whose boundary is made of flux points only (no Neumann copies, no weirs, no
+// drainage structures), driven by uniform rain, discharges and external sources at most. Everything
+// else takes the separate kernels.
+bool step_rule(const sfx::Consts& c, const sfx_model* M) {
+  return M->dense && sfx::std_physics(c) && std::count(M->kcs.begin(), M->kcs.end(), 6) == 0 && M->ndrn == 0 &&
+         M->structure_uv_index.empty();
 }
 
 // Rows of a step kernel tile. Its 4 waves compute 2 frows + 1 wave-rows of faces, one of them for

@@ -70,6 +70,12 @@ int fake_busy(char* what, int n) {
 }
 void fake_settle() { std::lock_guard<std::mutex> lk(mu); for (auto& s : streams) s.second.waited = s.second.issued; }
 long fake_live(int pins) { std::lock_guard<std::mutex> lk(mu); return (long)(pins ? pinned : device).size(); }
+long fake_bytes() {
+  std::lock_guard<std::mutex> lk(mu);
+  long n = 0;
+  for (auto& d : device) n += (long)d.second;
+  return n;
+}
 void fake_fail(long in) { std::lock_guard<std::mutex> lk(mu); fail_in = in; }
 // The scalars handed over from now on: every word 1 (an unstable step), or what was there.
 void fake_ones(int on) { std::lock_guard<std::mutex> lk(mu); ones = on != 0; }

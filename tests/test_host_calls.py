@@ -16,7 +16,7 @@ F = C.CDLL(sys.argv[1], mode=os.RTLD_GLOBAL | os.RTLD_NOW)
 import numpy as np
 from sfincs_amd import _lib
 from sfincs_amd import workloads as W
-F.fake_live.restype = F.fake_launches.restype = F.fake_stale.restype = C.c_long
+F.fake_live.restype = F.fake_launches.restype = F.fake_stale.restype = F.fake_bytes.restype = C.c_long
 F.fake_fail.argtypes = [C.c_long]
 
 def busy():
@@ -188,4 +188,22 @@ x.set_tuning(-1, (32, 8), (64, 4))
 assert x.tuning()['momentum_kernel'] == -1
 x.pin_tuning(d)
 assert x.tuning()['momentum_kernel'] == -8
+""")
+
+
+def test_footprint_counts_the_second_side_where_there_is_one(fake):
+    """Admission by footprint: scenarios outside the step kernel's rule hold one side of the levels, and
+    those inside it allocate no more than the footprint says."""
+    run(fake, """
+two = np.array([0.0, 1.0e5], np.float32)
+wind = regular(300, 301, wind=(two, np.full(2, 12.0, np.float32), np.full(2, 200.0, np.float32)))
+step = regular(300, 301)
+np_ = 300 * 301
+assert step.footprint() - wind.footprint() == np_ * 8 + 2 * np_          # levels, kfuv of 2 np slots
+_lib.Instance(regular()).close()                                        # the tables that stay
+base = F.fake_bytes()
+for m in (step, wind, subgrid(), W.quadtree_case(5, 5, nlev=2).build_model()):
+    x = _lib.Instance(m)
+    assert F.fake_bytes() - base <= m.footprint(), (F.fake_bytes(), m.footprint())
+    x.close()
 """)

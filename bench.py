@@ -5,9 +5,14 @@ subgrid tables from a seeded 5 m fBm DEM, 8 point discharges, 1.5 m tidal bounda
 A step is one model time step (forcing + momentum with CFL reduction + continuity) of
 the whole grid with all state resident in HBM; value = cell-updates/s.
 
-Prints one JSON line. `roofline.achieved` is the momentum kernel's algorithmic bytes per
-launch (per-branch byte counts below times the branch counters of the device) divided by
-its mean launch time, measured with HIP events on the launch stream.
+Prints one JSON line. `roofline.achieved` is the bytes that the work of a launch needs (per-branch
+byte counts below times the branch counters of the device) divided by its mean launch time,
+measured with HIP events on the launch stream. The launch is the step kernel's, a whole step, or
+the momentum kernel's where tuning picks the separate kernels. The counters are the separate
+kernels' (counting runs on them): points of their quiet tiles need nothing, a field that stays the
+same is not stored. So they are what a step needs, not what the step kernel moves: it skips tiles of
+63 columns by 1 to 7 rows and stores levels, volumes, wiggle detector and kfuv of every cell of a
+tile it runs. `roofline.traffic` is what it moves, from the counters of a profiled run.
 """
 import argparse
 import json
@@ -73,8 +78,8 @@ def byte_model(sizes, counts_per_step, stores_per_step, point_kernel, step_kerne
     mom = (np_ - c5 / 2) * MOM_CELL[sg] + copied * MOM_UV["copied"] + c1 * dry + c2 * MOM_UV["wet"][sg] + \
         c3 * MOM_UV["partial"] + c4 * MOM_UV["held"] + c5 * MOM_UV["tile_skipped"]
     cont = cont_bytes(CONT_READ[sg], np_, stores_per_step)
-    if step_kernel:   # one launch: the levels and faces that continuity needs are already there
-        cont -= (np_ - c5 / 2) * MOM_CELL[sg] + 8 * np_
+    if step_kernel:   # one launch: the faces that continuity needs are there, and the levels of cells both read
+        cont -= min(np_ - c5 / 2, np_ - stores_per_step[5]) * MOM_CELL[sg] + 8 * np_
     return mom, cont, dict(copied=copied, dry=c1, dry_zeros_held=c4, quiescent_tile=c5, wet=c2, partial=c3)
 
 
@@ -508,9 +513,11 @@ def main():
     cont_gbs = None if one else cont_b / (ms[2] * 1e-3) / 1e9
     step_gbs = (mom_b + cont_b) / (secs / args.steps) / 1e9
     mk = tuning["momentum_kernel"]
-    kernel = ("k_step<true>" if one else f"k_mom_point<float, true, {-mk}>" if mk < 0 else
+    # the step kernel's register budget goes by its blocks: eight waves a SIMD beyond 1792 of them, which
+    # every mesh of more than 750000 cells has
+    kernel = ("k_step<true, 8>" if one and sizes["np"] > 750000 else "k_step<true>" if one else f"k_mom_point<float, true, {-mk}>" if mk < 0 else
               "k_mom_cell<float, true>" if mk == 0 else "k_mom_strip<float, true>")
-    traffic = traffic_of(kernel)
+    traffic = traffic_of(kernel) if args.size == 2048 else None   # the size that was profiled
     out = {
         "metric": "cell-updates/s (mom+cont) & % HBM peak; ensemble p50/p99 time-to-result",
         "value": value,

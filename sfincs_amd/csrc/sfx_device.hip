@@ -65,7 +65,7 @@ struct Scalars {
   double t, tend;
   float dt, min_dt, dtchk;
   int32_t nt, active, error, error_pending, cur;
-  int32_t mom_done;              // a momentum sweep wrote buffer cur^1 and its per-tile minima
+  int32_t mom_done;              // a momentum sweep wrote buffer cur^1 and its per-tile keys
   int32_t itbndlast, itsrclast, itwndlast, itprcplast;
   float tauwu, tauwv, netprcp;   // uniform meteo forcing of this step
   float factime, facrel, one_minus_factime;
@@ -398,7 +398,7 @@ inline uint32_t div_magic(int d, size_t tiles) {
 // Completes a momentum sweep (run by one whole block): min_dt = min(dtmax, the points'
 // steps) as in sfincs_momentum.f90:121,542-545, and the q/uv double buffer flips.
 // Blocks of the per-scenario kernels (forcing, fold): one block covers a scenario's
-// boundary points and tile minima.
+// boundary points and tile keys.
 constexpr int FBLOCK = 1024;
 
 __device__ void fold_sweep(const DevInst& I) {
@@ -2115,9 +2115,10 @@ __global__ void __launch_bounds__(BLOCK) k_continuity(const DevInst* __restrict_
 // the faces, 0.8 for the cells, and 2 at a boundary), so what a tile needs first comes in few reads:
 // a tile's marks and lists in one (StepTile), a boundary point's tables in another (BndRec). With
 // them, and uniform values in scalar registers so that no subgrid wave spills, 161 x 203 subgrid
-// cells take 9.6 us a step (10.4 before), 2048 x 2048 take 83 (88), 64 x 96 regular ones 8.5 (8.7).
+// cells of a coast two thirds under water take 9.5 us a step (10.4 without), 2048 x 2048 of them 84
+// (88), 64 x 96 regular ones 8.1 (8.7).
 constexpr int STEP_COLS = WAVE - 1;
-constexpr uint8_t FT_RUN = 1, FT_BND = 2, FT_BAL = 4;          // fflag: never skipped; has boundary points; has balance faces
+constexpr uint8_t FT_RUN = 1, FT_BND = 2;   // StepTile::flag: never skipped; has boundary points
 
 // kfuv on the step kernel's sides: 1 wet; 0, 2, 4 dry -- 2 when the kernel has stored q = uv = 0
 // for the point in its last step, 4 when it did so in its last two (both q buffers hold zeros, so
@@ -2439,9 +2440,9 @@ __device__ __forceinline__ void step_tile(const DevInst* __restrict__ insts, con
 
 // W: the waves a SIMD holds at once. Regular tiles run 8 (64 vector registers). Subgrid ones take
 // fewer instructions with 69 registers, 7 waves, which is quicker while all of a launch's blocks are
-// on the chip at once (STEP_RESIDENT); beyond that the eighth wave is worth more. Measured, ms for
-// the same run with 7 / 8: 161 x 203 cells (519 blocks) 2.79 / 2.86, 512 x 700 (1896) 5.17 / 4.78,
-// 2048 x 2048 (9728) 13.1 / 12.9.
+// on the chip at once (STEP_RESIDENT); beyond that the eighth wave is worth more. Measured, us a step
+// with 7 / 8: 161 x 203 cells (519 blocks) 9.5 / 9.7, 420 x 420 (934) 12.5 / 12.8, 512 x 700 (1902)
+// 15.7 / 14.7, 700 x 1000 (3712) 23.7 / 22.7, 2048 x 2048 (9525) 84.8 / 83.6.
 constexpr int STEP_RESIDENT = 256 * 7;   // blocks: 256 CUs, a wave of each block on each of the 4 SIMDs
 
 template <bool SG, int W>
@@ -2713,7 +2714,7 @@ struct sfx_batch {
   WorkList wl_m[NLIST_M] = {}, wl_cuv = {}, wl_cd = {}, wl_ci = {};   // launch arguments of the lists
   bool cuv_apart = false;        // a member's combined points need k_cuv in whole steps too
   size_t off_cuv = 0, n_cuv = 0, off_cd = 0, n_cd = 0, off_ci = 0, n_ci = 0;
-  // step kernel lists (subgrid, regular), the scenarios in them (dIds + n_live onwards), and which
+  // the step kernel's list (subgrid tiles, then regular ones), the scenarios in it (dIds + n_live onwards), and which
   // scalar set the next launch reads
   size_t off_s = 0, n_s = 0;
   int step_kinds = 0;            // 1: subgrid tiles, 2: regular ones
@@ -3192,15 +3193,20 @@ bool step_rule(const sfx::Consts& c, const sfx_model* M) {
 
 // Rows of a step kernel tile. Its 4 waves compute 2 frows + 1 wave-rows of faces, one of them for
 // the neighbour's benefit, so few rows repeat more work; but the rows of a wave follow each other,
-// and a small mesh has waves to spare. The lines lie where the waves (4 np / (63 frows)) pass the
-// 8192 that the chip holds at once. Measured, us per step, regular / subgrid meshes (as separate
-// kernels about 16 / 17 at 64K cells, 19 / 22 at 256K, 62 / 60 at 1M, 93 / 98 at 3.1M / 4.2M):
-//    cells        frows 1        3            5            7
-//    64K         8.8 / 10.2  10.5 / 12.3  12.3 / 15.7  14.4 / 19.9
-//    130K / 176K 10.6 / 14.2 11.1 / 13.6  13.0 / 19.2  15.5 / 19.7
-//    256K / 358K 17.4 / 20.5 13.3 / 16.4  14.5 / 20.3  16.0 / 25.2
-//    1M          39.6 / 49   25.7 / 32.4  25.3 / 32.5  23.8 / 35.2
-//    3.1M / 4.2M  150 / 165  79.5 / 99.9  67.6 / 92.6  62.4 / 89.4
+// and a small mesh has waves to spare. The lines are taken from this table, one set for both kinds of
+// meshes: microseconds a step of regular / subgrid coasts, two thirds under water, advanced by 160
+// steps (as separate kernels about 16 / 17 at 64K cells, 19 / 22 at 256K, 62 / 60 at 1M, 93 / 98 at
+// 3.1M / 4.2M).
+//    cells          frows 1        3            5            7
+//    6K / 33K      8.3 / 9.5    9.8 / 11.4  11.6 / 14.4  13.2 / 16.7
+//    66K           8.8 / 10.0  10.4 / 11.9  12.0 / 14.4  14.0 / 16.7
+//    130K / 176K  10.5 / 13.3  11.1 / 12.5  12.5 / 15.9  14.7 / 17.6
+//    262K / 358K  17.0 / 18.4  12.8 / 14.8  14.0 / 18.5  15.8 / 20.8
+//    490K / 700K  28.2 / 31.1  19.1 / 22.6  19.0 / 25.5  20.5 / 26.1
+//    1.05M        53.3 / 46.1  31.9 / 31.7  29.1 / 31.3  27.9 / 33.0
+//    1.96M        94.0 / 80.4  52.5 / 51.5  45.5 / 48.6  42.5 / 49.5
+//    3.1M / 4.2M   149 / 151   78.6 / 91.9  66.8 / 85.6  62.2 / 83.9
+// (Regular meshes of 0.75M to 2M cells would take 7 rows by it, for 4 to 7%.)
 int step_rows(size_t np) {
   return np <= 150000 ? 1 : (np <= 750000 ? 3 : (np <= 2000000 ? 5 : 7));
 }
@@ -3246,7 +3252,7 @@ void build_step(sfx_handle* H, const sfx_model* M, const std::vector<int32_t>& b
   std::vector<BalRec> bals;
   for (int t = 0; t < I.fnt; ++t) {
     if (!pts[t].empty()) flag[t] |= FT_BND | FT_RUN;
-    if (!faces[t].empty()) flag[t] |= FT_BAL | FT_RUN;
+    if (!faces[t].empty()) flag[t] |= FT_RUN;
     tiles[t] = StepTile{(int32_t)recs.size(), (int32_t)bals.size(), (uint16_t)pts[t].size(), (uint16_t)faces[t].size(), flag[t]};
     recs.insert(recs.end(), pts[t].begin(), pts[t].end());
     bals.insert(bals.end(), faces[t].begin(), faces[t].end());
@@ -3870,7 +3876,7 @@ inline const DevInst* base_of(const sfx_batch* B, const WorkList& w) {
 // Launch phases of one step. what: bit 0 forcing, bit 1 momentum (+cuv), bit 2 continuity.
 // timestep_analysis_update (sfincs_timestep_analysis.f90:26-74, called after compute_fluxes
 // at sfincs_lib.f90:588) in two launches after a momentum sweep. First, per scenario, the
-// sweep's minimum time step from its tile minima (read only: the next fold still uses
+// sweep's minimum time step from its tile keys (read only: the next fold still uses
 // them); then, per uv slot, the running sum of the wet points' required steps, the sweeps
 // they were wet and those in which they limited the step (required <= min_dt + 1e-6).
 __global__ void __launch_bounds__(FBLOCK) k_tsa_min(const DevInst* __restrict__ insts,
@@ -4390,7 +4396,7 @@ extern "C" int sfx_batch_advance(sfx_batch* B, int32_t nsteps, int32_t* n_active
   }
   if (B->dirty && (rc = rebuild(B))) return rc;
   if (B->n_live + B->n_step > 0) {
-    if (B->n_live == 0) {   // the step kernel alone: one or two launches a step
+    if (B->n_live == 0) {   // the step kernel alone: one launch a step
       for (int r = 0; r < nsteps; ++r) launch(B, 7, 0);
     } else {
       const int K = std::max(1, std::min(nsteps, 64));

@@ -2518,22 +2518,45 @@ __global__ void __launch_bounds__(BLOCK) k_give_uv(const DevInst* __restrict__ I
   }
 }
 
-// The levels back to their first side (after an odd number of steps), for the kernels that work
-// on one side only.
-__global__ void __launch_bounds__(BLOCK) k_step_settle(const DevInst* __restrict__ I0) {
+// A scenario moves to the step kernel: both sides hold what no step writes (kfuv of closed points,
+// boundary means), no tile is quiet or woken, no key is raised, and the separate kernels' marks, which
+// mean other things, are gone. s: the step scalars.
+__global__ void __launch_bounds__(BLOCK) k_enter_step(const DevInst* __restrict__ I0, Scalars s) {
   const DevInst& I = *I0;
-  for (uint32_t c = blockIdx.x * BLOCK + threadIdx.x; c < (uint32_t)I.nslot; c += gridDim.x * BLOCK) {
-    I.kf_s[0][c] = I.kf_s[1][c];
-    if (c < (uint32_t)I.np) {
-      I.zs_s[0][c] = I.zs_s[1][c];
-      if (I.subgrid) { I.vol_s[0][c] = I.vol_s[1][c]; I.zsd_s[0][c] = I.zsd_s[1][c]; }
-    }
-    if (c < (uint32_t)I.nkcuv2) I.um_s[0][c] = I.um_s[1][c];
+  const uint32_t t = blockIdx.x * BLOCK + threadIdx.x, step = gridDim.x * BLOCK;
+  for (uint32_t c = t; c <= (uint32_t)I.nslot; c += step) {   // the dummy point too
+    const int8_t k = I.kf_s[0][c] & 1;
+    I.kf_s[0][c] = k;
+    I.kf_s[1][c] = k;
+    if (c < (uint32_t)I.np) I.kcs[c] &= (uint8_t)~KCS_STEADY;
+    if (c < (uint32_t)I.nkcuv2) I.um_s[1][c] = I.um_s[0][c];
   }
+  for (uint32_t k = t; k < 2u * (uint32_t)I.fnt; k += step) I.fwake[k] = 0;
+  for (uint32_t k = t; k < (uint32_t)(BLOCK / WAVE) * (uint32_t)I.fnt; k += step) I.fquiet[k] = 0;
+  for (uint32_t k = t; k < 3u * NKEY * KEY_STRIDE; k += step) (&I.sb->key[0][0])[k] = 0u;
+  if (blockIdx.x == 0) copy_words(&I.sb->s[0], &s);
 }
 
-// No cell keeps its steady bit, and with uv set no uv-point its zero flags (host writes, and changes
-// between the step kernel and the separate ones, whose flags mean different things).
+// And back: the state on its first side (`side` holds it), no tile quiescent (nmq words of mq).
+__global__ void __launch_bounds__(BLOCK) k_enter_general(const DevInst* __restrict__ I0, Scalars s, int side, uint32_t nmq) {
+  const DevInst& I = *I0;
+  const uint32_t t = blockIdx.x * BLOCK + threadIdx.x, step = gridDim.x * BLOCK;
+  for (uint32_t c = t; c <= (uint32_t)I.nslot; c += step) {
+    I.kf_s[0][c] = I.kf_s[side][c] & 1;
+    if (c < (uint32_t)I.np) {
+      I.kcs[c] &= (uint8_t)~KCS_STEADY;
+      if (side) {
+        I.zs_s[0][c] = I.zs_s[1][c];
+        if (I.subgrid) { I.vol_s[0][c] = I.vol_s[1][c]; I.zsd_s[0][c] = I.zsd_s[1][c]; }
+      }
+    }
+    if (side && c < (uint32_t)I.nkcuv2) I.um_s[0][c] = I.um_s[1][c];
+  }
+  for (uint32_t k = t; k < nmq; k += step) I.mq[k] = 0u;
+  if (blockIdx.x == 0) copy_words(&I.sb->s[0], &s);
+}
+
+// No cell keeps its steady bit, and with uv set no uv-point its zero flags (host writes).
 __global__ void __launch_bounds__(BLOCK) k_clear_marks(const DevInst* __restrict__ I0, int uv) {
   const DevInst& I = *I0;
   for (uint32_t c = blockIdx.x * BLOCK + threadIdx.x; c < (uint32_t)I.nslot; c += gridDim.x * BLOCK) {
@@ -2637,7 +2660,8 @@ struct sfx_handle {
   std::vector<int32_t> ref2slot;   // reference uv index (0-based, incl. cuv and dummy) -> slot
   int32_t nslot = 0;
   hipStream_t stream = nullptr;
-  struct sfx_batch* solo = nullptr;
+  struct sfx_batch* solo[2] = {};   // the scenario as a batch of its own, on the separate kernels and on the step kernel
+  void changed();                // its descriptor changed: those lists are built anew
   // tuned shapes: continuity tile, momentum per-cell tile, momentum strip rows (0: per-cell)
   int tile_tn = CELL_SHAPES[0][0], tile_tm = CELL_SHAPES[0][1];
   int mtile_tn = 32, mtile_tm = 8, strip_rows = -1;   // per-point kernel on 32 x 8 tiles
@@ -2730,6 +2754,11 @@ struct sfx_batch {
   int graph_steps = 0;
   int fp64 = 0;
 };
+
+void sfx_handle::changed() {
+  for (sfx_batch* b : solo)
+    if (b) b->dirty = true;
+}
 
 namespace {
 
@@ -3274,7 +3303,8 @@ extern "C" int sfx_batch_destroy(sfx_batch* b);
 extern "C" int sfx_destroy(sfx_handle* H) {
   if (!H) return SFX_OK;
   hipSetDevice(H->device);
-  if (H->solo) { sfx_batch_destroy(H->solo); H->solo = nullptr; }
+  for (auto& b : H->solo)
+    if (b) { sfx_batch_destroy(b); b = nullptr; }
   hipDeviceSynchronize();
   for (void* p : H->allocs) hipFree(p);
   if (H->pin) hipHostFree(H->pin);
@@ -3991,36 +4021,36 @@ int ensure_graph(sfx_batch* B, int steps) {
   return SFX_OK;
 }
 
+// One for each path, so that a move between them builds no lists and keeps the captured graph.
 sfx_batch* solo(sfx_handle* H) {
-  if (!H->solo) {
-    H->solo = new sfx_batch();
-    H->solo->device = H->device;
-    H->solo->stream = H->stream;
-    H->solo->own_stream = false;
-    H->solo->members.push_back(H);
-    H->solo->tend.push_back(0.0);
-    H->solo->dirty = true;
+  sfx_batch*& b = H->solo[H->on_step ? 1 : 0];
+  if (!b) {
+    b = new sfx_batch();
+    b->device = H->device;
+    b->stream = H->stream;
+    b->own_stream = false;
+    b->members.push_back(H);
+    b->tend.push_back(0.0);
+    b->dirty = true;
   }
-  return H->solo;
+  return b;
 }
 
-// Moves a handle to the step kernel, or back to the separate ones. Both sides then hold what no
-// step writes, no tile is taken for quiet, and the separate kernels' marks are cleared.
+// Moves a handle to the step kernel, or back to the separate ones: one launch, in order on the
+// handle's stream (a batch, which runs on its own, waits for it). A host that alternates whole steps
+// and standalone calls moves twice a round.
 int enter_step(sfx_handle* H) {
   if (!H->use_step || H->hI.count || H->on_step) return SFX_OK;
   Scalars s;
   int rc = normalise(H, s);
   if (rc) return rc;
-  const DevInst& I = H->hI;
-  HIPCHK(hipMemcpyAsync(I.kf_s[1], I.kf_s[0], (size_t)H->nslot + 1, hipMemcpyDeviceToDevice, H->stream));
-  if (I.nkcuv2) HIPCHK(hipMemcpyAsync(I.um_s[1], I.um_s[0], (size_t)I.nkcuv2 * 4, hipMemcpyDeviceToDevice, H->stream));
-  HIPCHK(hipMemsetAsync(I.fwake, 0, (size_t)I.fnt * 2, H->stream));
-  HIPCHK(hipMemsetAsync(I.fquiet, 0, (size_t)I.fnt * (BLOCK / WAVE), H->stream));
-  HIPCHK(hipMemsetAsync(I.sb->key, 0, sizeof(I.sb->key), H->stream));
-  if ((rc = write_scalars(H, s)) || (rc = clear_marks(H, 1))) return rc;
-  HIPCHK(hipStreamSynchronize(H->stream));   // a batch runs on its own stream
+  s.ahead = 0;
+  const int nb = std::min(4096, (H->hI.nslot + BLOCK) / BLOCK);
+  hipLaunchKernelGGL(k_enter_step, dim3(nb), dim3(BLOCK), 0, H->stream, H->dI, s);
+  HIPCHK(hipGetLastError());
+  H->hs = s;
+  H->hs_ok = true;
   H->on_step = true;
-  if (H->solo) H->solo->dirty = true;
   return SFX_OK;
 }
 
@@ -4029,14 +4059,15 @@ int enter_general(sfx_handle* H) {
   Scalars s;
   int rc = normalise(H, s);
   if (rc) return rc;
-  const int nb = std::min(4096, (H->hI.nslot + BLOCK - 1) / BLOCK);
-  if (s.side) hipLaunchKernelGGL(k_step_settle, dim3(nb), dim3(BLOCK), 0, H->stream, H->dI);
-  HIPCHK(hipGetLastError());
+  const int nb = std::min(4096, (H->hI.nslot + BLOCK) / BLOCK), side = s.side;
   s.side = 0;
-  if ((rc = write_scalars(H, s)) || (rc = clear_marks(H, 1))) return rc;
+  s.ahead = 0;
+  hipLaunchKernelGGL(k_enter_general, dim3(nb), dim3(BLOCK), 0, H->stream, H->dI, s, side, (uint32_t)H->nmt_cap);
+  HIPCHK(hipGetLastError());
+  H->hs = s;
+  H->hs_ok = true;
   H->on_step = false;
-  if (H->solo) H->solo->dirty = true;
-  return reset_tile_flags(H);
+  return SFX_OK;
 }
 
 }  // namespace
@@ -4166,7 +4197,7 @@ extern "C" int sfx_set_counting(sfx_handle* H, int32_t on) {
   HIPCHK(hipMemsetAsync(H->hI.blkcnt, 0, NCNT * H->nmt_cap * sizeof(uint32_t), H->stream));
   HIPCHK(hipMemsetAsync(H->hI.cntstore, 0, NSTORE * std::max<size_t>(1, H->nct_cap) * sizeof(uint32_t), H->stream));
   HIPCHK(hipStreamSynchronize(H->stream));
-  if (H->solo) H->solo->dirty = true;
+  H->changed();
   return SFX_OK;
 }
 
@@ -4391,7 +4422,10 @@ extern "C" int sfx_batch_advance(sfx_batch* B, int32_t nsteps, int32_t* n_active
   int rc;
   if (B->members.empty()) { if (n_active) *n_active = 0; return SFX_OK; }
   for (size_t i = 0; i < B->members.size(); ++i) {
-    if ((rc = enter_step(B->members[i]))) return rc;
+    sfx_handle* H = B->members[i];
+    const bool moves = !H->on_step;
+    if ((rc = enter_step(H))) return rc;
+    if (moves && H->on_step) HIPCHK(hipStreamSynchronize(H->stream));
     if (i >= B->built_step.size() || i >= B->live.size() || (B->live[i] && B->built_step[i] != (char)B->members[i]->on_step)) B->dirty = true;
   }
   if (B->dirty && (rc = rebuild(B))) return rc;
@@ -4532,7 +4566,7 @@ extern "C" int sfx_set_tuning(sfx_handle* H, const int32_t in[5]) {
   H->tile_tn = tn; H->tile_tm = tm; H->strip_rows = sk; H->mtile_tn = mtn; H->mtile_tm = mtm;
   H->use_step = step;
   if ((rc = reset_keys(H))) return rc;
-  if (H->solo) H->solo->dirty = true;
+  H->changed();
   return SFX_OK;
 }
 
@@ -4547,7 +4581,7 @@ extern "C" int sfx_set_work_order(sfx_handle* H, int32_t mom_run, int32_t cont_r
   H->hI.xchunk = mom_run; H->hI.xchunk_c = cont_run;
   H->xchunk = mom_run; H->xchunk_c = cont_run;
   HIPCHK(hipMemcpy(H->dI, &H->hI, sizeof(DevInst), hipMemcpyHostToDevice));
-  if (H->solo) H->solo->dirty = true;
+  H->changed();
   return SFX_OK;
 }
 
@@ -4655,7 +4689,7 @@ extern "C" int sfx_autotune(sfx_handle* H, int32_t trials) {
     HIPCHK(hipMemcpy(H->hI.bal, bal_keep, sizeof(bal_keep), hipMemcpyHostToDevice));
     if (!um.empty()) HIPCHK(hipMemcpy(H->hI.uvmean, um.data(), um.size(), hipMemcpyHostToDevice));
     if (!qs.empty()) HIPCHK(hipMemcpy(H->hI.qtsrc, qs.data(), qs.size() * sizeof(float), hipMemcpyHostToDevice));
-    if (H->solo) H->solo->dirty = true;
+    H->changed();
     return SFX_OK;
   };
   // the step kernel against the separate kernels, forcing included, each from the scenario's own state

@@ -20,7 +20,7 @@ std::map<hipStream_t, Stream> streams;
 std::map<const void*, std::string> kernels;
 std::map<void*, size_t> device, pinned;
 std::map<std::string, long> launches;
-long fail_in = 0, stale = 0, clock_ms = 0;
+long fail_in = 0, stale = 0, clock_ms = 0, operations = 0;
 bool ones = false, capturing = false;
 thread_local hipError_t last = hipSuccess;   // until it is asked for, as the real one
 std::map<size_t, std::pair<void*, std::vector<char>>> copied;   // by size: the last copy to the device
@@ -30,6 +30,7 @@ thread_local std::vector<Call> calls;
 
 void issue(hipStream_t s, const std::string& what) {
   if (capturing) return;
+  ++operations;
   ++streams[s].issued;
   streams[s].last = what;
 }
@@ -81,6 +82,8 @@ void fake_fail(long in) { std::lock_guard<std::mutex> lk(mu); fail_in = in; }
 void fake_ones(int on) { std::lock_guard<std::mutex> lk(mu); ones = on != 0; }
 // Launches of k_give_scalars that found another descriptor than the last one given to a batch.
 long fake_stale() { std::lock_guard<std::mutex> lk(mu); return stale; }
+// Launches, copies and fills so far.
+long fake_operations() { std::lock_guard<std::mutex> lk(mu); return operations; }
 long fake_launches(const char* part) {
   std::lock_guard<std::mutex> lk(mu);
   long n = 0;
@@ -102,6 +105,7 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return take(p, n, pinne
 hipError_t hipHostFree(void* p) { return give(p, pinned); }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind k) {
   std::lock_guard<std::mutex> lk(mu);
+  ++operations;
   copy(d, s, n, k);
   streams[nullptr].waited = streams[nullptr].issued;
   return hipSuccess;

@@ -16,7 +16,7 @@ F = C.CDLL(sys.argv[1], mode=os.RTLD_GLOBAL | os.RTLD_NOW)
 import numpy as np
 from sfincs_amd import _lib
 from sfincs_amd import workloads as W
-F.fake_live.restype = F.fake_launches.restype = F.fake_stale.restype = F.fake_bytes.restype = C.c_long
+F.fake_live.restype = F.fake_launches.restype = F.fake_stale.restype = F.fake_bytes.restype = F.fake_operations.restype = C.c_long
 F.fake_fail.argtypes = [C.c_long]
 
 def busy():
@@ -206,4 +206,20 @@ for m in (step, wind, subgrid(), W.quadtree_case(5, 5, nlev=2).build_model()):
     x = _lib.Instance(m)
     assert F.fake_bytes() - base <= m.footprint(), (F.fake_bytes(), m.footprint())
     x.close()
+""")
+
+
+def test_a_move_between_the_kernels_is_one_launch(fake):
+    """A host that alternates whole steps and a standalone call on a scenario of the step kernel: beside
+    the two moves, a round takes the launches of the step and of the call (scalars written, the work,
+    scalars handed over) and builds no lists anew."""
+    run(fake, """
+x = _lib.Instance(regular())
+for k in range(3):
+    n = F.fake_operations()
+    x.update(0.0)
+    x.compute_fluxes(0.5)
+    n = F.fake_operations() - n
+assert n <= 2 + 3 + 3, n
+assert F.fake_launches(b'k_enter_step') == 3 and F.fake_launches(b'k_enter_general') == 3
 """)

@@ -4702,14 +4702,15 @@ extern "C" int sfx_autotune(sfx_handle* H, int32_t trials) {
     H->changed();
     return SFX_OK;
   };
-  // the step kernel against the separate kernels, forcing included, each from the scenario's own state
-  // (while counting is on every step takes the separate kernels and there is nothing to choose by)
+  // the separate kernels from the scenario's own state, forcing included, then the step kernel on from
+  // where they ended (while counting is on every step takes the separate kernels and there is nothing
+  // to choose by)
   if (H->stepable && !H->hI.count && !rc) {
     float apart = 0.f, step = 0.f;
     H->use_step = false;
     if (!(rc = restore(s))) rc = time_phases(H, 7, trials, e0, e1, apart);
     H->use_step = true;
-    if (!rc && !(rc = restore(s)) && !(rc = enter_step(H))) rc = time_phases(H, 7, trials, e0, e1, step);
+    if (!rc && !(rc = enter_step(H))) rc = time_phases(H, 7, trials, e0, e1, step);
     end_steps(solo(H));
     if (!rc) rc = enter_general(H);
     H->use_step = !rc && step <= apart;

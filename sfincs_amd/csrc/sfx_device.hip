@@ -3698,10 +3698,11 @@ extern "C" int sfx_set_state(sfx_handle* H, const char* name, const void* src, s
     const size_t n = H->sz.npuv;
     if (nbytes != n) { set_error("size mismatch"); return SFX_ERR_ARG; }
     std::vector<int8_t> b(H->nslot + 1, 0);
-    HIPCHK(hipMemcpy(b.data(), I.kf_s[s.side], b.size(), hipMemcpyDeviceToHost));
+    if ((rc = to_host(H, b.data(), I.kf_s[s.side], b.size()))) return rc;
     for (size_t i = 0; i < n; ++i) b[H->ref2slot[i]] = ((const int8_t*)src)[i];
-    for (int sd = 0; sd < (H->on_step ? 2 : 1); ++sd)   // points that no step writes keep it on both sides
-      HIPCHK(hipMemcpy(I.kf_s[sd], b.data(), b.size(), hipMemcpyHostToDevice));
+    if ((rc = to_device(H, I.kf_s[s.side], b.data(), b.size()))) return rc;
+    if (H->on_step)   // points that no step writes keep it on both sides
+      HIPCHK(hipMemcpyAsync(I.kf_s[s.side ^ 1], I.kf_s[s.side], b.size(), hipMemcpyDeviceToDevice, H->stream));
     return reset_tile_flags(H);
   }
   if (k == "zs0" || k == "zsderv" || k == "zsmax") {

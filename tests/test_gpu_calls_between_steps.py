@@ -102,3 +102,20 @@ def test_discharges_past_their_series_stay_through_a_move_between_kernels():
     assert np.all(want > q + 39.0)
     apart.update_to(350.0)
     assert np.array_equal(apart.get("qtsrc"), want)
+
+
+@pytest.mark.parametrize("steps", [3, 4])
+def test_a_write_of_kfuv_holds_on_either_side(steps):
+    """kfuv written after an odd and an even number of steps, closed points included."""
+    m, x, y = _pair()
+    for i in (x, y):
+        for _ in range(steps):
+            i.update(0.0)
+        k = i.get("kfuv")
+        k[::5] = 0
+        k[3::7] = 1
+        i.set("kfuv", k)
+        assert np.array_equal(i.get("kfuv"), k)
+        for _ in range(3):
+            i.update(0.0)
+    _same(x, y, m, steps)

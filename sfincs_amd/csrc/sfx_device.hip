@@ -2882,6 +2882,7 @@ int upload_state(sfx_handle* H, const sfx_model* M) {
 // -------------------------------------------------------------------------- create / destroy
 namespace {
 bool step_rule(const sfx::Consts& c, const sfx_model* M);
+bool step_default(const sfx::Consts& c, const sfx_model* M);
 }
 
 extern "C" int sfx_model_footprint(const sfx_model* M, size_t* bytes) {
@@ -3195,7 +3196,7 @@ extern "C" int sfx_create_ex(const sfx_model* M, int32_t device, int32_t fp64, s
       I.zs_s[k] = I.zs; I.vol_s[k] = I.vol; I.zsd_s[k] = (float*)I.zsderv; I.kf_s[k] = I.kfuv; I.um_s[k] = (float*)I.uvmean;
     }
     H->stepable = !H->fp64 && step_rule(I.c, M);
-    H->use_step = H->stepable;
+    H->use_step = H->stepable && step_default(I.c, M);
     if (H->stepable) build_step(H, M, slot, coef);
     H->bnd_recs = {};
   }
@@ -3228,6 +3229,19 @@ namespace {
 bool step_rule(const sfx::Consts& c, const sfx_model* M) {
   return M->dense && sfx::std_physics(c) && std::count(M->kcs.begin(), M->kcs.end(), 6) == 0 && M->ndrn == 0 &&
          M->structure_uv_index.empty();
+}
+
+// Whether it does unless told otherwise (sfx_autotune, sfx_set_tuning). Rain or sources in every cell
+// of a subgrid mesh leave nearly all its points partly wet: a step is then bound by the two level rows
+// that each point reads, and the faces that tiles repeat cost more than one launch saves once the chip
+// is full. Measured, us a step of subgrid terrain under 40 mm/h and an hour after, step kernel /
+// separate kernels: 262K cells 23.6 / 29.5, 490K 38 to 43 / 40 to 45, 640K 49 to 53 / 52 to 54, 750K 59
+// to 69 / 60 to 69, 810K 74 to 80 / 71 to 73, 900K 84 to 91 / 75 to 80, 1.05M 98 / 91, 1.96M 179 / 165,
+// 4.19M 395 / 376, with 1, 3, 5, 7, 9 or 12 rows a tile alike; on the dry terrain before the rain 31 / 38
+// at 750K, 35 / 41 at 1.05M and 73 / 83 at 4.19M, of which such a run sees less.
+constexpr int32_t STEP_RAIN_CELLS = 750000;
+bool step_default(const sfx::Consts& c, const sfx_model* M) {
+  return !(M->subgrid && (c.flags & (sfx::F_PRECIP | sfx::F_QEXT)) && M->np > STEP_RAIN_CELLS);
 }
 
 // Rows of a step kernel tile. Its 4 waves compute 2 frows + 1 wave-rows of faces, one of them for

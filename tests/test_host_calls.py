@@ -223,3 +223,23 @@ for k in range(3):
 assert n <= 2 + 3 + 3, n
 assert F.fake_launches(b'k_enter_step') == 3 and F.fake_launches(b'k_enter_general') == 3
 """)
+
+
+def test_large_subgrid_meshes_under_rain_start_on_the_separate_kernels(fake):
+    """The default by size, mesh and forcing: the step kernel up to 750000 cells, on regular meshes and
+    without rain or sources in every cell beyond; it can be pinned where it is not the default."""
+    run(fake, """
+import torch
+torch.cuda.is_available = lambda: False          # terrain is made on the host
+def kernel(make, n, m, pin=False, **kw):
+    x = _lib.Instance(make(n, m, seed=1, t_end=4.0e3, **kw).build_model())
+    if pin: x.set_tuning(-8, (32, 8), (64, 4))
+    return x.tuning()['momentum_kernel']
+sub, reg = W.subgrid_case, W.regular_case
+assert kernel(sub, 750, 1000, rain_mmh=20.0, nsrc=0) == -8
+assert kernel(sub, 751, 1000, rain_mmh=20.0, nsrc=0) == -1
+assert kernel(sub, 751, 1000, rain_mmh=0.0, nsrc=0, use_qext=1) == -1
+assert kernel(sub, 751, 1000, rain_mmh=0.0, nsrc=0) == -8
+assert kernel(sub, 751, 1000, rain_mmh=20.0, nsrc=0, pin=True) == -8
+assert kernel(reg, 1000, 1000, rain_mmh=20.0) == -8
+""")

@@ -231,15 +231,17 @@ def test_large_subgrid_meshes_under_rain_start_on_the_separate_kernels(fake):
     run(fake, """
 import torch
 torch.cuda.is_available = lambda: False          # terrain is made on the host
+torch.set_num_threads(1)
 def kernel(make, n, m, pin=False, **kw):
+    if make is sub: kw.update(refi=2, nl=2, nsrc=0)
     x = _lib.Instance(make(n, m, seed=1, t_end=4.0e3, **kw).build_model())
     if pin: x.set_tuning(-8, (32, 8), (64, 4))
     return x.tuning()['momentum_kernel']
 sub, reg = W.subgrid_case, W.regular_case
-assert kernel(sub, 750, 1000, rain_mmh=20.0, nsrc=0) == -8
-assert kernel(sub, 751, 1000, rain_mmh=20.0, nsrc=0) == -1
-assert kernel(sub, 751, 1000, rain_mmh=0.0, nsrc=0, use_qext=1) == -1
-assert kernel(sub, 751, 1000, rain_mmh=0.0, nsrc=0) == -8
-assert kernel(sub, 751, 1000, rain_mmh=20.0, nsrc=0, pin=True) == -8
+assert kernel(sub, 750, 1000, rain_mmh=20.0) == -8
+assert kernel(sub, 751, 1000, rain_mmh=20.0) == -1
+assert kernel(sub, 751, 1000, rain_mmh=0.0, use_qext=1) == -1
+assert kernel(sub, 751, 1000, rain_mmh=0.0) == -8
+assert kernel(sub, 751, 1000, rain_mmh=20.0, pin=True) == -8
 assert kernel(reg, 1000, 1000, rain_mmh=20.0) == -8
 """)
